@@ -13,6 +13,9 @@
 #include "common.hpp"
 #include "internal.hpp"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace bchip {
 
 // ggml type numbers (quant.rs:35-49).
@@ -354,44 +357,48 @@ __global__ __launch_bounds__(64 * MM_WAVES) void k_matmul(const MatmulParams p) 
 // Batched product on the matrix cores (n >= MM_MIN input rows; the reference switches its
 // batches to a matrix-unit product the same way, gpu/mod.rs:33-41, metal.rs:153-197).
 // In the affine form, group g of weight row r is w = a q + b, q a small integer; so
-// sum_k w x = a sum q x + b sum x. The MFMAs compute sum q x with x split into f16 parts,
-// x = hi + lo 2^-12 (lo stored scaled by 2^12 so it keeps its 11 bits): about 22 bits,
-// each product exact in f32, f32-level sums.
+// sum_k w x = a sum q x + b sum x. The MFMAs compute sum q x with x split into two f16 parts:
+// a unit of 256 columns of an input row is scaled by a power of two s that puts its largest
+// |x| in [2^14, 2^15), hi = f16(x s), lo = f16(x s - hi): 22 bits of every x within 2^-17 of
+// the unit's largest and an absolute error below 2^-39 of it for the rest, each product
+// exact in f32, f32-level sums. A unit's hi and lo sums meet at its end.
 //
 // k_matmul_mm: a workgroup is W waves of 16 weight rows, eight input rows and a K range of
-// at most MM_K units of 256 columns. The range's x is staged once in LDS as 16 A rows: rows
-// 0..7 the eight inputs' hi, rows 8..15 their lo, so one v_mfma_f32_16x16x32_f16 over group
-// g gives D[i][l] = sum hi_i q (i < 8) and sum lo_{i-8} q (i >= 8) for the wave's 16 rows at
-// once. Lane 16 c + l holds 8 weights of group g of row r0 + l (8c .. 8c + 7) as its B
-// operand, unpacked from the ggml bytes in registers, in the order 0, 2, 1, 3, 4, 6, 5, 7
-// (pairs of bytes 0, 2 and 1, 3 of a dword make the f16 pairs directly; staged x is
-// permuted alike, and the MFMA's sum over k is the group's either way): each field is put
-// under the f16 exponent of 1024 (one v_and_or_b32 for a pair of nibbles, v_perm_b32 for a
-// pair of bytes) and one packed f16 subtraction takes 1024 and the format's fixed offset
-// away (Q4_0 8, Q5_0 16, Q6K 32, Q8_0 -128 after a sign flip). D[4c + i][l] in lane
-// 16 c + l: c < 2 the hi sums of input 4c + i, c >= 2 the lo sums of input 4(c - 2) + i;
-// per group each lane adds a_eff D[i] (a_eff: a with the lo scale folded in) to four
-// accumulators. The b sum x terms (Q4_1, Q5_1: m; Q4K, Q5K: -dmin m_j) are a product over
-// groups of their own: a v_mfma_f32_16x16x4_f32 a half unit, A = the groups' sums of x
-// (rows 8..15 zero), B = the groups' b, accumulated across the range. Q6K (a scale a 16 weights) takes two
-// v_mfma_f32_16x16x16_f16 a group, one a half; F16 has no scale and chains its MFMAs
-// through the accumulators. The units' bytes are loaded MM_PF units ahead. K splits: their
-// number depends on rows and cols only; a split's partial is (hi + lo) + b terms of its
-// units, and the row's result the splits' partials added in split order, whether one
-// workgroup runs the splits one after another or ks workgroups run them at once and the
-// last to finish (a device counter per tile) adds them: an input row's bits depend on that
-// row alone, never on n or its place in the batch.
-constexpr float MM_LO = 4096.0f;   // lo = (x - hi) * MM_LO
+// at most MM_K units. The range's x is staged once in LDS as 16 A rows: rows 0 .. 7 the eight
+// inputs' hi, rows 8 .. 15 their lo, so one v_mfma_f32_16x16x32_f16 over group g gives D[i][l]
+// = sum hi_i q (i < 8) and sum lo_{i-8} q (i >= 8), each in a chain of its own, for the
+// wave's 16 rows at once. Lane 16 c + l holds 8 weights of group g of row r0 + l (8c .. 8c +
+// 7) as its B operand, unpacked from the ggml bytes in registers, in the order 0, 2,
+// 1, 3, 4, 6, 5, 7 (pairs of bytes 0, 2 and 1, 3 of a dword make the f16 pairs directly;
+// staged x is permuted alike, and the MFMA's sum over k is the group's either way): each
+// field is put under the f16 exponent of 1024 (one v_and_or_b32 for a pair of nibbles,
+// v_perm_b32 for a pair of bytes) and one packed f16 subtraction takes 1024 and the format's
+// fixed offset away (Q4_0 8, Q5_0 16, Q6K 32, Q8_0 -128 after a sign flip). Q6K has a scale
+// a 16 weights: its two MFMAs a group take one half each, lane c holding weights 4c .. 4c + 3
+// of the half twice, over x's hi and over its lo (A rows 8 .. 15 are inputs 0 .. 7 again). D[4c + i][l] is in lane 16 c + l.
+// Accumulation, per output element, in this order whatever kernel computes it:
+//   T_hi, T_lo = the MFMAs of a group over hi and over lo (Q4K, Q5K, F16: chained over the
+//   unit's groups; Q6K: one T of a half, hi and lo in one MFMA)
+//   t_hi += a T_hi, t_lo += a T_lo per group, zeroed each unit (Q4K, Q5K, F16: t = T)
+//   t = t_hi + t_lo (Q6K: t += a T per half)
+//   t = d t (Q4K, Q5K), then t += the unit's b sum x terms; p += t / s per unit
+//   out = the K splits' p added in split order.
+// The b sum x terms (Q4_1, Q5_1: m; Q4K, Q5K: -dmin m_j) are one more MFMA a unit: A = the
+// eight groups' sums of x s / 32 in three f16 parts (33 bits), B = the m's three times over.
+// The units' bytes are loaded MM_PF units ahead. K splits: their number depends on rows and
+// cols only; one workgroup runs the splits one after another or ks workgroups run them at
+// once and the last to finish (a device counter per tile) adds them: an input row's bits
+// depend on that row alone, never on n or its place in the batch.
 constexpr uint32_t MM_MIN = 2;     // batches of at least this many rows take the matrix cores (MM_FROM)
 // Units (256 columns) a K split at most: the staged x takes 16 rows x (256 MM_K + 8) halves of
-// LDS (the 8: 16-byte reads of 16 rows on distinct banks); the K-quants also pass each unit's
+// LDS (rows 8 banks apart measured 0.6 us a call better than 4); the K-quants also pass each unit's
 // bytes through LDS, so their splits are shorter.
 template <uint32_t TY>
 constexpr bool MM_LDSP = TY != G_F16;  // units pass through LDS (all block formats)
 template <uint32_t TY>
 constexpr uint32_t MM_K = MM_LDSP<TY> ? 4 : 8;
 template <uint32_t TY>
-constexpr uint32_t MM_XS = MM_K<TY> * 256 + 8;
+constexpr uint32_t MM_XS = MM_K<TY> * 256 + 16;
 constexpr uint32_t MM_PAR = MATMUL_COUNTERS;  // tiles (W x 16 rows x 8 inputs) up to which K splits run in parallel
 
 template <uint32_t TY>
@@ -399,7 +406,7 @@ constexpr bool mm_type() {
     return TY == G_F16 || TY == G_Q8_0 || TY == G_Q4_0 || TY == G_Q4_1 || TY == G_Q5_0 || TY == G_Q5_1 ||
            TY == G_Q4K || TY == G_Q5K || TY == G_Q6K;
 }
-// Formats whose b sum x terms take the f32 MFMA.
+// Formats with b sum x terms.
 template <uint32_t TY>
 constexpr bool mm_sum() {
     return TY == G_Q4_1 || TY == G_Q5_1 || TY == G_Q4K || TY == G_Q5K;
@@ -549,11 +556,12 @@ __device__ __forceinline__ void mm_fix(const uint32_t (&s)[MW<TY>], uint32_t (&d
         for (int l = 0; l < MW<TY> / 4; l++)
             if (4 * l + pq < NP)
                 *(u32x4*)(wt + q * MM_WT<TY> + 16 * (4 * l + pq)) = u32x4{s[4 * l], s[4 * l + 1], s[4 * l + 2], s[4 * l + 3]};
-        if constexpr (TY == G_Q4_1 || TY == G_Q5_1) {  // m of groups c and 4 + c (the b terms)
+        if constexpr (TY == G_Q4_1 || TY == G_Q5_1) {  // the unit's eight m's (the b terms)
             constexpr uint32_t BS = TY == G_Q4_1 ? 20 : 24;
             const uint8_t* rw = wt + rl * MM_WT<TY>;
-            d[0] = *(const uint16_t*)(rw + BS * c + 2);
-            d[1] = *(const uint16_t*)(rw + BS * (4 + c) + 2);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                d[k] = *(const uint16_t*)(rw + 2 * BS * k + 2) | ((uint32_t)*(const uint16_t*)(rw + 2 * BS * k + BS + 2) << 16);
         }
     }
     if constexpr (TY == G_Q6K) {
@@ -603,38 +611,96 @@ __device__ __forceinline__ void mm_fix(const uint32_t (&s)[MW<TY>], uint32_t (&d
     }
 }
 
-// What a unit's groups share: the scale factors and packed scale bytes (K-quants), and the
-// lane's two b values (groups c and 4 + c: B of the f32 MFMAs).
+// Max over the wave of unsigned values, in every lane (DPP rotations within 16 lanes, then
+// swaps of 16 and 32: no LDS).
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, false));  // row_ror:8
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xf, 0xf, false));  // row_ror:4
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x122, 0xf, 0xf, false));  // row_ror:2
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xf, 0xf, false));  // row_ror:1
+    const auto r16 = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = max(r16[0], r16[1]);
+    const auto r32 = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return max(r32[0], r32[1]);
+}
+// The power of two that puts the largest |x| of a unit (four columns a lane) in [2^14, 2^15),
+// and its inverse; 1 where that is no finite number (an infinity or NaN in x stays one).
+// Units below 2^-112 take 2^126 (a zero stays zero). Bits of |x| compare as |x| does.
+__device__ __forceinline__ void unit_scale(const float (&x)[4], float& s, float& inv) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) m = max(m, __float_as_uint(x[e]) & 0x7fffffffu);
+    const uint32_t e = max(__builtin_amdgcn_readfirstlane(wave_max_u32(m)) >> 23, 15u);
+    s = e == 255u ? 1.0f : __uint_as_float((268u - e) << 23);
+    inv = e == 255u ? 1.0f : __uint_as_float((e - 14u) << 23);
+}
+// The sum of a group of 32 columns over its 8 lanes.
+__device__ __forceinline__ float group_sum(const float (&x)[4]) {
+    float sg = ((x[0] + x[1]) + x[2]) + x[3];
+    sg += __shfl_xor(sg, 1, 64);
+    sg += __shfl_xor(sg, 2, 64);
+    sg += __shfl_xor(sg, 4, 64);
+    return sg;
+}
+// Four columns' hi and lo parts, scaled, in the order of e (x s is exact, so lo's FMA gives
+// x s - hi).
+__device__ __forceinline__ void hi_lo(const float (&x)[4], float s, half4& h, half4& l) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+        const half2 hv = __builtin_convertvector((f32x2{x[e] * s, x[e + 1] * s}), half2);
+        const half2 lv = __builtin_convertvector((f32x2{__builtin_fmaf(x[e], s, -(float)hv[0]), __builtin_fmaf(x[e + 1], s, -(float)hv[1])}), half2);
+        h[e] = hv[0]; h[e + 1] = hv[1];
+        l[e] = lv[0]; l[e + 1] = lv[1];
+    }
+}
+// A group's sum of x s / 32 in three parts.
+__device__ __forceinline__ void sum_parts(float sg, float s, f16 (&p)[3]) {
+    float r = sg * (s * 0.03125f);
+#pragma unroll
+    for (int e = 0; e < 3; e++) {
+        p[e] = (f16)r;
+        r -= (float)p[e];
+    }
+}
+// What a unit's groups share: the scale factors and packed scale bytes (K-quants), the b
+// factor over x's scale and the eight groups' m's as f16.
 struct MMUnit {
-    float dl = 0.0f, b0 = 0.0f, b1 = 0.0f;
-    uint32_t scA = 0, scB = 0;
+    float dl = 0.0f, bl = 0.0f;
+    uint32_t scA = 0, scB = 0, mnA = 0, mnB = 0;
 };
+// The m bytes of a unit (K-quants) as f16 values, in group order.
+__device__ __forceinline__ half8 mins_f16(uint32_t a, uint32_t b) {
+    const half2 o = half2{(f16)1024.0f, (f16)1024.0f};
+    auto two = [&](uint32_t v, uint32_t sel) {
+        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2, __builtin_amdgcn_perm(0x64646464u, v, sel)) - o);
+    };
+    return __builtin_bit_cast(half8, u32x4{two(a, 0x04010400u), two(a, 0x04030402u), two(b, 0x04010400u), two(b, 0x04030402u)});
+}
 
 template <uint32_t TY>
-__device__ __forceinline__ MMUnit mm_unit(const uint32_t (&d)[MWD<TY>], uint32_t c, float fl) {
+__device__ __forceinline__ MMUnit mm_unit(const uint32_t (&d)[MWD<TY>]) {
     MMUnit m;
     if constexpr (TY == G_Q4K || TY == G_Q5K) {
         // scale and min bytes of sub-blocks 0..3 and 4..7 (6 bits each, quant.rs:136-146)
         const uint32_t s0 = d[1], s1 = d[2], s2 = d[3];
         m.scA = s0 & 0x3f3f3f3fu;
         m.scB = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
-        const uint32_t mnA = s1 & 0x3f3f3f3fu, mnB = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
-        const float dd = h2f(d[0] & 0xffffu) * fl, ndm = -h2f(d[0] >> 16);
-        m.dl = dd;
-        m.b0 = ndm * (float)((mnA >> (8 * c)) & 255u);
-        m.b1 = ndm * (float)((mnB >> (8 * c)) & 255u);
+        m.mnA = s1 & 0x3f3f3f3fu;
+        m.mnB = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
+        m.dl = h2f(d[0] & 0xffffu);
+        m.bl = -32.0f * h2f(d[0] >> 16);
     } else if constexpr (TY == G_Q4_1 || TY == G_Q5_1) {
-        m.b0 = h2f(d[0]);
-        m.b1 = h2f(d[1]);
+        m.bl = 32.0f;
     }
     return m;
 }
 
-// Group j of a loaded unit for lane c: B operand(s) and a (fl and the field scale folded in).
-// Q6K gives two half operands q4[0], q4[1] (16x16x16 MFMAs) and a0, a1.
+// Group j of a loaded unit for lane c: B operand(s) and a. Q6K gives its
+// two halves' four weights q4[0], q4[1] and a0, a1.
 template <uint32_t TY>
 __device__ __forceinline__ void mm_group(const uint32_t (&d)[MWD<TY>], const MMUnit& m, const uint8_t* unit_base,
-                                         const uint8_t* rw, int j, uint32_t c, float fl, half8& q, half4 (&q4)[2],
+                                         const uint8_t* rw, int j, uint32_t c, half8& q, half4 (&q4)[2],
                                          float& a0, float& a1) {
     if constexpr (TY == G_F16) {  // weights 8c .. 8c + 7 in order (x staged unpermuted)
         q = __builtin_bit_cast(half8, u32x4{d[4 * j], d[4 * j + 1], d[4 * j + 2], d[4 * j + 3]});
@@ -644,7 +710,7 @@ __device__ __forceinline__ void mm_group(const uint32_t (&d)[MWD<TY>], const MMU
                                *(const uint32_t*)(rw + a + 4 + 2 * sh)};
         const uint32_t w0 = __builtin_amdgcn_alignbyte(w[1], w[0], sh), w1 = __builtin_amdgcn_alignbyte(w[2], w[1], sh);
         q = bytes8_f16(w0 ^ 0x80808080u, w1 ^ 0x80808080u, half2{(f16)1152.0f, (f16)1152.0f});
-        a0 = h2f(*(const uint16_t*)(rw + 34 * j)) * fl;
+        a0 = h2f(*(const uint16_t*)(rw + 34 * j));
     } else if constexpr (TY == G_Q4_0 || TY == G_Q5_0) {
         // from the lane's LDS row rw; lanes 0, 1: low nibbles, lanes 2, 3: high nibbles
         // (weights 16 ..), as q - 8 (Q4_0) or, with qh byte c as bit 4, q - 16 (Q5_0)
@@ -662,7 +728,7 @@ __device__ __forceinline__ void mm_group(const uint32_t (&d)[MWD<TY>], const MMU
             w1 = ((w1 >> ns) & 0x0f0f0f0fu) | bit4_spread(qh >> 4);
             q = bytes8_f16(w0, w1, half2{(f16)1040.0f, (f16)1040.0f});
         }
-        a0 = h2f(*(const uint16_t*)(rw + BS * j)) * fl;
+        a0 = h2f(*(const uint16_t*)(rw + BS * j));
     } else if constexpr (TY == G_Q4_1 || TY == G_Q5_1) {  // from the lane's LDS row rw
         constexpr uint32_t BS = TY == G_Q4_1 ? 20 : 24, QS = TY == G_Q4_1 ? 4 : 8;
         const uint8_t* g = rw + BS * j;
@@ -676,7 +742,7 @@ __device__ __forceinline__ void mm_group(const uint32_t (&d)[MWD<TY>], const MMU
             const uint32_t w1 = ((x1 >> ns) & 0x0f0f0f0fu) | bit4_spread(qh >> 4);
             q = bytes8_f16(w0, w1, half2{(f16)1024.0f, (f16)1024.0f});
         }
-        a0 = h2f(*(const uint16_t*)g) * fl;
+        a0 = h2f(*(const uint16_t*)g);
     } else if constexpr (TY == G_Q4K || TY == G_Q5K) {
         const int k = j / 2, hi = j % 2;
         const uint32_t v0 = d[4 + 2 * k], v1 = d[5 + 2 * k];
@@ -721,7 +787,7 @@ __device__ __forceinline__ void mm_group(const uint32_t (&d)[MWD<TY>], const MMU
         const uint32_t sw = __builtin_amdgcn_alignbyte(d[25 + hh * 2 + (qr >> 1)], d[24 + hh * 2 + (qr >> 1)], sh);
         const uint32_t sp = sw >> (16 * (qr & 1));  // bytes 2 qr, 2 qr + 1 of the 4-byte window
         const uint32_t dw = __builtin_amdgcn_alignbyte(d[28], d[28], sh) & 0xffffu;  // d: bytes 208, 209
-        const float dd = h2f(dw) * fl;
+        const float dd = h2f(dw);
         a0 = dd * (float)(int8_t)(uint8_t)(sp & 255u);
         a1 = dd * (float)(int8_t)(uint8_t)((sp >> 8) & 255u);
     }
@@ -736,27 +802,35 @@ struct MMParams {
     uint32_t rows, cols, n, npad, row_bytes, units, ks, par;
 };
 
-template <uint32_t TY>
-__global__ __launch_bounds__(64 * MM_W<TY>, MM_W<TY> / 2) void k_matmul_mm(const MMParams p) {  // two workgroups a CU
-    constexpr bool SUM = mm_sum<TY>(), KP = TY != G_F16;
+// NI: input rows a workgroup, 8 (two workgroups a CU) or 16 (one, for batches of 9 to 16:
+// each weight unpacked once for all of them).
+template <uint32_t TY, int NI>
+__global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_matmul_mm(const MMParams p) {
+    constexpr bool SUM = mm_sum<TY>(), KP = TY != G_F16, UT = TY == G_Q4K || TY == G_Q5K || TY == G_F16;
     constexpr int PF = MM_PF<TY>, W = MM_W<TY>, NT = 64 * W;
     constexpr uint32_t XS = MM_XS<TY>;
-    __shared__ __attribute__((aligned(16))) f16 xs[16 * XS];
-    __shared__ __attribute__((aligned(16))) float ss[SUM ? MM_K<TY> * 8 * 16 : 4];
+    // hi of the NI inputs, then lo (Q6K: an input's row holds each four columns' hi and lo
+    // together, 16 bytes; rows XR apart).
+    constexpr uint32_t XR = TY == G_Q6K ? 2 * MM_K<TY> * 256 + 16 : XS;
+    __shared__ __attribute__((aligned(16))) f16 xs[2 * NI * XS];
+    __shared__ __attribute__((aligned(16))) float isc[MM_K<TY> * NI];
+    __shared__ __attribute__((aligned(16))) f16 ss[SUM ? MM_K<TY> * NI * 32 : 4];
     constexpr bool KQ = MM_LDSP<TY>;  // units pass through LDS (mm_fix)
     __shared__ __attribute__((aligned(16))) uint8_t wtb[KQ ? W * 16 * MM_WT<TY> : 16];
     __shared__ uint32_t last;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    static_assert(XR <= 2 * XS, "Q6K's rows fit");
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t c = lane >> 4, rl = lane & 15;
-    const uint32_t r0 = blockIdx.x * (16 * W) + 16 * w, r = r0 + rl, i0 = blockIdx.y * 8;
+    const uint32_t r0 = blockIdx.x * (16 * W) + 16 * w, r = r0 + rl, i0 = blockIdx.y * NI;
     const bool live = r0 < p.rows;  // the wave has rows
     // the rows a lane loads: its matrix-core row (mrowp), or (KQ) its lane quad's
     const uint8_t* mrowp = p.w + (size_t)min(r, p.rows - 1) * p.row_bytes;
     const uint8_t* rowp = KQ ? p.w + (size_t)min(r0 + (lane >> 2), p.rows - 1) * p.row_bytes : mrowp;
     uint8_t* wt = wtb + (KQ ? w * 16 * MM_WT<TY> : 0);
-    const float fl = c >= 2 ? 1.0f / MM_LO : 1.0f;
     const uint32_t kz0 = p.par ? blockIdx.z : 0, kz1 = p.par ? blockIdx.z + 1 : p.ks;
     float tot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (SUM)  // the last quarter of the b terms' A rows stays 0
+        for (uint32_t q = tid; q < MM_K<TY> * NI; q += NT) *(half8*)&ss[32 * q + 24] = half8{};
     for (uint32_t kz = kz0; kz < kz1; kz++) {
         const uint32_t ua = kz * p.units / p.ks, nu = (kz + 1) * p.units / p.ks - ua;
         // Every step loads one unit (past the range's end its last unit again), so the loads
@@ -767,50 +841,52 @@ __global__ __launch_bounds__(64 * MM_W<TY>, MM_W<TY> / 2) void k_matmul_mm(const
             for (int f = 0; f < PF; f++) mm_load<TY>(rowp, ua + min((uint32_t)f, nu - 1), c, pk[f]);
         }
         if (kz != kz0) __syncthreads();  // every wave is done with the previous split's x
-        // Stage x: float4 q of the range (input q / (64 nu), columns 4 (q % (64 nu)) ..), read
-        // coalesced (consecutive lanes, consecutive 16 bytes), as hi and lo in the lanes' k order
-        // (within each 8 columns: 0, 2, 1, 3, 4, 6, 5, 7, so a float4's four values stay
-        // together); (SUM) a group's sum over the 8 lanes that hold it, in a fixed tree.
-        const uint32_t q4 = 64 * nu;  // float4s an input row of the range
-        constexpr int XB = W == 8 ? 4 : 8;  // loads in flight a thread (eight waves: a split's all)
-        for (uint32_t q0 = tid; q0 < 8 * q4; q0 += XB * NT) {
-            float4 v[XB];
+        // Stage x, an input row a wave and a unit (64 float4s, consecutive lanes) a load, as scaled
+        // hi and lo in the lanes' k order (within each 8 columns: 0, 2, 1, 3, 4, 6, 5, 7, so a
+        // float4's four values stay together); (SUM) a group's sum over the 8 lanes that hold it,
+        // in a fixed tree.
+        constexpr uint32_t XB = 4;  // loads in flight a thread
+        // (Inputs past the batch are left as they are: their D rows are not used.)
+        const uint32_t ni = min((uint32_t)NI, p.n - i0);
+        for (uint32_t i = w; i < ni; i += W) {
+            const float* xrow = p.x + (size_t)(i0 + i) * p.cols + (size_t)ua * 256 + 4 * lane;
+            for (uint32_t v0 = 0; v0 < nu; v0 += XB) {
+                float4 v[XB];
 #pragma unroll
-            for (int t = 0; t < XB; t++) {
-                const uint32_t q = q0 + t * NT, in = i0 + q / q4;
-                v[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (q < 8 * q4 && in < p.n)
-                    v[t] = *(const float4*)(p.x + (size_t)in * p.cols + (size_t)ua * 256 + 4 * (q % q4));
-            }
+                for (uint32_t t = 0; t < XB; t++) v[t] = *(const float4*)(xrow + 256 * min(v0 + t, nu - 1));
 #pragma unroll
-            for (int t = 0; t < XB; t++) {
-                const uint32_t q = q0 + t * NT, i = q / q4, cq = q % q4;
-                if (q >= 8 * q4) break;  // uniform: 8 q4 is a multiple of NT
-                if constexpr (SUM) {
-                    float sg = ((v[t].x + v[t].y) + v[t].z) + v[t].w;
-                    sg += __shfl_xor(sg, 1, 64);
-                    sg += __shfl_xor(sg, 2, 64);
-                    sg += __shfl_xor(sg, 4, 64);
-                    if ((cq & 7) == 0) {
-                        ss[(cq / 8) * 16 + i] = sg;
-                        ss[(cq / 8) * 16 + 8 + i] = 0.0f;
+                for (uint32_t t = 0; t < XB; t++) {
+                    const uint32_t lu = v0 + t, cq = 64 * lu + lane;
+                    if (lu >= nu) break;
+                    const float x4[4] = {v[t].x, v[t].y, v[t].z, v[t].w};
+                    float sc, inv;
+                    unit_scale(x4, sc, inv);
+                    if (lane == 0) isc[lu * NI + i] = inv;
+                    if constexpr (SUM) {
+                        const float sg = group_sum(x4);
+                        if ((lane & 7) == 0) {
+                            f16 sp[3];
+                            sum_parts(sg, sc, sp);
+#pragma unroll
+                            for (int e = 0; e < 3; e++) ss[(lu * NI + i) * 32 + 8 * e + lane / 8] = sp[e];
+                        }
+                    }
+                    const float xs4[4] = {x4[0], KP ? x4[2] : x4[1], KP ? x4[1] : x4[2], x4[3]};
+                    half4 h, l;
+                    hi_lo(xs4, sc, h, l);
+                    if constexpr (TY == G_Q6K) {
+                        *(half8*)&xs[i * XR + 8 * cq] = __builtin_shufflevector(h, l, 0, 1, 2, 3, 4, 5, 6, 7);
+                    } else {
+                        *(half4*)&xs[i * XS + 4 * cq] = h;
+                        *(half4*)&xs[(NI + i) * XS + 4 * cq] = l;
                     }
                 }
-                const float xs4[4] = {v[t].x, KP ? v[t].z : v[t].y, KP ? v[t].y : v[t].z, v[t].w};
-                half4 h, l;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const f16 hv = (f16)xs4[e];
-                    h[e] = hv;
-                    l[e] = (f16)((xs4[e] - (float)hv) * MM_LO);
-                }
-                *(half4*)&xs[i * XS + 4 * cq] = h;
-                *(half4*)&xs[(8 + i) * XS + 4 * cq] = l;
             }
         }
         __syncthreads();
-        f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, accb = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         if (live) {
+            const uint32_t ra = rl & (NI - 1u);  // the lane's A row
             for (uint32_t u0 = 0; u0 < nu; u0 += PF) {
 #pragma unroll
                 for (int f = 0; f < PF; f++) {
@@ -820,46 +896,66 @@ __global__ __launch_bounds__(64 * MM_W<TY>, MM_W<TY> / 2) void k_matmul_mm(const
                         const uint8_t* qb = rowp + (size_t)(ua + lu) * MM_UB<TY>;   // its lane quad's
                         uint32_t dd[MWD<TY>];
                         mm_fix<TY>(pk[f], dd, wt, c, rl, (uint32_t)((uintptr_t)qb & 15u), (uint32_t)((uintptr_t)ub & 15u));
-                        const MMUnit m = mm_unit<TY>(dd, c, fl);
-                        if constexpr (SUM) {  // sum_g b_g s_g over the unit's groups, 4 at a time
-                            const float s0 = ss[(lu * 8 + c) * 16 + rl], s1 = ss[(lu * 8 + 4 + c) * 16 + rl];
-                            accb = __builtin_amdgcn_mfma_f32_16x16x4f32(s0, m.b0, accb, 0, 0, 0);
-                            accb = __builtin_amdgcn_mfma_f32_16x16x4f32(s1, m.b1, accb, 0, 0, 0);
-                        }
-                        f32x4 accu = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, accu2 = accu;  // even, odd groups
+                        const MMUnit m = mm_unit<TY>(dd);
+                        const f32x4 z4 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                        f32x4 t4 = z4, t5 = z4;  // hi and lo apart (NI 8: in lanes c < 2 and c >= 2 of t4)
 #pragma unroll
                         for (int j = 0; j < 8; j++) {
                             const uint32_t col = lu * 256 + 32 * j;
                             half8 q;
-                            half4 q4[2];
+                            half4 qh[2];
                             float a0 = 0.0f, a1 = 0.0f;
-                            mm_group<TY>(dd, m, ub, wt + rl * MM_WT<TY>, j, c, fl, q, q4, a0, a1);
-                            if constexpr (TY == G_Q4K || TY == G_Q5K) {
-                                const half8 xa = *(const half8*)&xs[rl * XS + col + 8 * c];
-                                if (j % 2 == 0) accu = mfma16(xa, q, accu);
-                                else accu2 = mfma16(xa, q, accu2);
-                            } else if constexpr (TY == G_F16) {
-                                const half8 xa = *(const half8*)&xs[rl * XS + col + 8 * c];
-                                acc = mfma16(xa, q, acc);
-                            } else if constexpr (TY == G_Q6K) {
-                                const half4 x0 = *(const half4*)&xs[rl * XS + col + 4 * c];
-                                const half4 x1 = *(const half4*)&xs[rl * XS + col + 16 + 4 * c];
-                                const f32x4 z = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                                const f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x16f16(x0, q4[0], z, 0, 0, 0);
-                                const f32x4 d1 = __builtin_amdgcn_mfma_f32_16x16x16f16(x1, q4[1], z, 0, 0, 0);
+                            mm_group<TY>(dd, m, ub, wt + rl * MM_WT<TY>, j, c, q, qh, a0, a1);
+                            if constexpr (TY == G_Q6K) {
+                                const half8 x0 = *(const half8*)&xs[ra * XR + 2 * col + 8 * c];
+                                const half8 x1 = *(const half8*)&xs[ra * XR + 2 * col + 32 + 8 * c];
+                                const f32x4 d0 = mfma16(x0, __builtin_shufflevector(qh[0], qh[0], 0, 1, 2, 3, 4, 5, 6, 7), z4);
+                                const f32x4 d1 = mfma16(x1, __builtin_shufflevector(qh[1], qh[1], 0, 1, 2, 3, 4, 5, 6, 7), z4);
 #pragma unroll
-                                for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(a1, d1[i], __builtin_fmaf(a0, d0[i], acc[i]));
+                                for (int i = 0; i < 4; i++) t4[i] = __builtin_fmaf(a1, d1[i], __builtin_fmaf(a0, d0[i], t4[i]));
                             } else {
-                                const half8 xa = *(const half8*)&xs[rl * XS + col + 8 * c];
-                                const f32x4 dv = mfma16(xa, q, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                                const half8 xh = *(const half8*)&xs[rl * XS + col + 8 * c];
+                                half8 xo;
+                                if constexpr (NI == 16) xo = *(const half8*)&xs[(16 + rl) * XS + col + 8 * c];
+                                if constexpr (UT) {
+                                    t4 = mfma16(xh, q, t4);
+                                    if constexpr (NI == 16) t5 = mfma16(xo, q, t5);
+                                } else {
+                                    const f32x4 dv = mfma16(xh, q, z4);
 #pragma unroll
-                                for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(a0, dv[i], acc[i]);
+                                    for (int i = 0; i < 4; i++) t4[i] = __builtin_fmaf(a0, dv[i], t4[i]);
+                                    if constexpr (NI == 16) {
+                                        const f32x4 dw = mfma16(xo, q, z4);
+#pragma unroll
+                                        for (int i = 0; i < 4; i++) t5[i] = __builtin_fmaf(a0, dw[i], t5[i]);
+                                    }
+                                }
                             }
                         }
-                        if constexpr (TY == G_Q4K || TY == G_Q5K) {
+                        if constexpr (TY != G_Q6K) {  // hi + lo
+                            if constexpr (NI == 16) {
+                                t4 += t5;
+                            } else {
 #pragma unroll
-                            for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(m.dl, accu[i] + accu2[i], acc[i]);
+                                for (int i = 0; i < 4; i++) {
+                                    const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(t4[i]), __float_as_uint(t4[i]), false, false);
+                                    t4[i] = __uint_as_float(r2[0]) + __uint_as_float(r2[1]);
+                                }
+                            }
                         }
+                        const float4 is = *(const float4*)&isc[lu * NI + 4 * (c & (NI / 4 - 1u))];
+                        const float i4[4] = {is.x, is.y, is.z, is.w};
+                        if constexpr (TY == G_Q4K || TY == G_Q5K) t4 *= m.dl;
+                        if constexpr (SUM) {
+                            half8 mv;
+                            if constexpr (TY == G_Q4K || TY == G_Q5K) mv = mins_f16(m.mnA, m.mnB);
+                            else mv = __builtin_bit_cast(half8, u32x4{dd[0], dd[1], dd[2], dd[3]});
+                            const f32x4 tb = mfma16(*(const half8*)&ss[(lu * NI + ra) * 32 + 8 * c], mv, z4);
+#pragma unroll
+                            for (int i = 0; i < 4; i++) t4[i] = __builtin_fmaf(m.bl, tb[i], t4[i]);
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(i4[i], t4[i], acc[i]);
                     }
                     // the unit's registers are free: load into them directly (a load hoisted
                     // above their last use would land in other registers and wait to be copied)
@@ -868,21 +964,12 @@ __global__ __launch_bounds__(64 * MM_W<TY>, MM_W<TY> / 2) void k_matmul_mm(const
                 }
             }
         }
-        if constexpr (TY == G_F16) {
+        // the split's partial (input 4c + i in lanes c < NI / 4); then the splits in order
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[i] *= fl;
-        }
-        // the split's partial in lanes c < 2 (input 4c + i): hi + lo, then the b terms; then
-        // the splits in order
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float pt = acc[i] + __shfl_xor(acc[i], 32, 64);
-            if constexpr (SUM) pt += accb[i];
-            tot[i] = kz == kz0 ? pt : tot[i] + pt;
-        }
+        for (int i = 0; i < 4; i++) tot[i] = kz == kz0 ? acc[i] : tot[i] + acc[i];
     }
     if (!p.par) {
-        if (c < 2 && r < p.rows) {
+        if (c < NI / 4 && r < p.rows) {
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 if (i0 + 4 * c + i < p.n) p.out[(size_t)(i0 + 4 * c + i) * p.rows + r] = tot[i];
@@ -891,7 +978,7 @@ __global__ __launch_bounds__(64 * MM_W<TY>, MM_W<TY> / 2) void k_matmul_mm(const
     }
     // Parallel splits: the partial to device memory (write-through stores), then the tile's
     // arrival count; the last workgroup of the tile adds the partials in split order.
-    if (c < 2 && r < p.rows) {
+    if (c < NI / 4 && r < p.rows) {
 #pragma unroll
         for (int i = 0; i < 4; i++)
             __hip_atomic_store(&p.part[((size_t)blockIdx.z * p.npad + i0 + 4 * c + i) * p.rows + r], tot[i],
@@ -906,36 +993,668 @@ __global__ __launch_bounds__(64 * MM_W<TY>, MM_W<TY> / 2) void k_matmul_mm(const
     }
     __syncthreads();
     if (!last) return;
-    // The tile's 8 x 16 W outputs, two a thread; eight splits' loads in flight at a time.
+    // The tile's NI x 16 W outputs, two a thread and pass; eight splits' loads in flight at a time.
     const size_t stride = (size_t)p.npad * p.rows;
-    float sum[2] = {0.0f, 0.0f};
-    bool ok[2];
-    const float* src[2];
+    for (uint32_t q = 0; q < NI * 16 * W; q += 2 * NT) {
+        float sum[2] = {0.0f, 0.0f};
+        bool ok[2];
+        const float* src[2];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const uint32_t e = tid + h * NT, rr = blockIdx.x * (16 * W) + e % (16 * W), in = i0 + e / (16 * W);
-        ok[h] = rr < p.rows && in < p.n;
-        src[h] = p.part + (size_t)min(in, p.npad - 1) * p.rows + min(rr, p.rows - 1);
+        for (int h = 0; h < 2; h++) {
+            const uint32_t e = q + tid + h * NT, rr = blockIdx.x * (16 * W) + e % (16 * W), in = i0 + e / (16 * W);
+            ok[h] = rr < p.rows && in < p.n;
+            src[h] = p.part + (size_t)min(in, p.npad - 1) * p.rows + min(rr, p.rows - 1);
+        }
+        for (uint32_t k0 = 0; k0 < p.ks; k0 += 8) {
+            float v[2][8];
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int t = 0; t < 8; t++)
+                    v[h][t] = k0 + t < p.ks ? __hip_atomic_load(src[h] + (k0 + t) * stride, __ATOMIC_RELAXED,
+                                                                 __HIP_MEMORY_SCOPE_AGENT)
+                                            : 0.0f;
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int t = 0; t < 8; t++)
+                    if (k0 + t < p.ks) sum[h] = k0 + t == 0 ? v[h][t] : sum[h] + v[h][t];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t e = q + tid + h * NT, rr = blockIdx.x * (16 * W) + e % (16 * W), in = i0 + e / (16 * W);
+            if (ok[h]) p.out[(size_t)in * p.rows + rr] = sum[h];
+        }
     }
-    for (uint32_t k0 = 0; k0 < p.ks; k0 += 8) {
-        float v[2][8];
+    if (tid == 0) __hip_atomic_store(&p.cnt[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---------------------------------------------------------------------------------------
+// Batched product of many input rows (prompts). k_matmul_mm's workgroups hold 8 input rows,
+// so a batch of n unpacks every weight n / 8 times and is bound by that VALU work (512 rows
+// of 14336 x 4096 Q4K: 480 us). Here a workgroup of eight waves takes MT input rows x 128
+// weight rows and walks its K range in steps of 64 columns (two groups): the step's packed
+// weights are loaded by four threads a row (one step ahead), unpacked once into f16 in LDS
+// and read back as the B operands of every input tile; x comes from k_mm_prep as scaled hi
+// and lo parts in the operands' order (the conversion once a call instead of once a
+// workgroup). Each wave owns TM x TN 16 x 16 output tiles.
+//
+// Every output element sees k_matmul_mm's operations in k_matmul_mm's order, so an input
+// row's bits stay those of the same row in a batch of 2. Formats of 32-weight blocks also
+// come here when cols is no multiple of 256 (the last unit is then shorter): those shapes
+// have no k_matmul_mm form and took the VALU.
+constexpr int TL_NT = 128;       // weight rows a workgroup
+constexpr int TL_THREADS = 512;  // eight waves; four threads a weight row
+
+template <uint32_t TY>
+constexpr bool tl_kq() {
+    return TY == G_Q4K || TY == G_Q5K;
+}
+// x's order: 0 as it is (F16), 1 k_matmul_mm's pairs (0, 2, 1, 3 of each four), 2 the same
+// with hi and lo of each four columns together (Q6K).
+template <uint32_t TY>
+constexpr int tl_order() {
+    return TY == G_F16 ? 0 : TY == G_Q6K ? 2 : 1;
+}
+
+// Prepared x of one unit of one input row, a wave: per step 256 bytes, hi of its 64 columns
+// then lo (order 2: 16-byte pieces of four columns' hi and lo); the inverse scale; (SUM) the
+// A operand of the b sum x terms. Rows past n and columns past cols are zeros.
+template <int ORDER, bool SUM>
+__global__ __launch_bounds__(256) void k_mm_prep(const float* __restrict__ x, f16* __restrict__ xp,
+                                                 float* __restrict__ ip, f16* __restrict__ sp, uint32_t n,
+                                                 uint32_t cols, uint32_t npad, uint32_t steps) {
+    const uint32_t lane = threadIdx.x & 63u, row = blockIdx.y * 4 + (threadIdx.x >> 6), u = blockIdx.x;
+    const uint32_t col = 256 * u + 4 * lane;
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (row < n && col < cols) v = *(const float4*)(x + (size_t)row * cols + col);
+    const float x4[4] = {v.x, v.y, v.z, v.w};
+    float sc, inv;
+    unit_scale(x4, sc, inv);
+    const size_t at = (size_t)u * npad + row;
+    if (lane == 0) ip[at] = inv;
+    if constexpr (SUM) {
+        const float sg = group_sum(x4);
+        if ((lane & 7u) == 0) {
+            f16 p[3];
+            sum_parts(sg, sc, p);
 #pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int t = 0; t < 8; t++)
-                v[h][t] = k0 + t < p.ks ? __hip_atomic_load(src[h] + (k0 + t) * stride, __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT)
-                                        : 0.0f;
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int t = 0; t < 8; t++)
-                if (k0 + t < p.ks) sum[h] = k0 + t == 0 ? v[h][t] : sum[h] + v[h][t];
+            for (int e = 0; e < 4; e++) sp[at * 32 + 8 * e + lane / 8] = e < 3 ? p[e] : (f16)0.0f;
+        }
     }
+    const float xo[4] = {v.x, ORDER ? v.z : v.y, ORDER ? v.y : v.z, v.w};
+    half4 h, l;
+    hi_lo(xo, sc, h, l);
+    const uint32_t step = 4 * u + lane / 16, q = lane % 16;
+    if (step >= steps) return;
+    f16* dst = xp + ((size_t)step * npad + row) * 128;
+    if constexpr (ORDER == 2) {
+        *(half8*)(dst + 8 * q) = __builtin_shufflevector(h, l, 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+        *(half4*)(dst + 4 * q) = h;
+        *(half4*)(dst + 64 + 4 * q) = l;
+    }
+}
+
+struct TLParams {
+    const uint8_t* w;
+    const f16* xp;    // [steps][npad][128]
+    const float* ip;  // [units][npad]: inverse scales
+    const f16* sp;    // [units][npad][32]: the group sums' parts
+    float* out;
+    float* part;
+    uint32_t* cnt;
+    uint32_t rows, n, npad, row_bytes, units, groups, ks, par, nyt;
+};
+
+// Bytes at an address that may be 2-byte aligned only (the hardware takes such loads).
+template <typename T>
+__device__ __forceinline__ T ldu(const uint8_t* p) {
+    T v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), sizeof(T));
+    return v;
+}
+
+// A thread's packed bytes of one step: row r, quarter qd. Groups 2s and 2s + 1 of the row
+// are g = 0, 1. K-quants and Q6K: bytes 8 qd .. of each 32-byte run; 32-weight formats and
+// F16: half qd & 1 of group qd >> 1. Every byte loaded is used (a load's unused register
+// would be taken for something else, which waits for the load).
+template <uint32_t TY>
+constexpr int TLP = TY == G_F16 ? 8 : TY == G_Q4K ? 2 : TY == G_Q5K ? 4 : TY == G_Q6K ? 6 : 6;
+// Load instructions of a step at least.
+template <uint32_t TY>
+constexpr int TLN = TY == G_Q4K ? 1 : 2;
+// A K-quant unit's header: d, dmin and the scale bytes; Q6K's 16 scales and d.
+template <uint32_t TY>
+constexpr int TLH = tl_kq<TY>() ? 4 : TY == G_Q6K ? 5 : 1;
+
+template <uint32_t TY>
+__device__ __forceinline__ void tl_load(const uint8_t* __restrict__ row, uint32_t step, uint32_t qd, uint32_t groups,
+                                        uint32_t (&d)[TLP<TY>]) {
+    if constexpr (tl_kq<TY>()) {
+        const uint8_t* b = row + (size_t)(step / 4) * (TY == G_Q4K ? 144 : 176) + 8 * qd;
+        const u32x2 v = *(const u32x2*)(b + (TY == G_Q4K ? 16 : 48) + 32 * (step % 4));
+        d[0] = v[0]; d[1] = v[1];
+        if constexpr (TY == G_Q5K) {
+            const u32x2 q = *(const u32x2*)(b + 16);
+            d[2] = q[0]; d[3] = q[1];
+        }
+    } else if constexpr (TY == G_Q6K) {
+        const uint32_t hh = (step % 4) / 2;
+        const uint8_t* b = row + (size_t)(step / 4) * 210 + 8 * qd;
+        const u32x2 v0 = ldu<u32x2>(b + 64 * hh), v1 = ldu<u32x2>(b + 64 * hh + 32), v2 = ldu<u32x2>(b + 128 + 32 * hh);
+        d[0] = v0[0]; d[1] = v0[1];  // group 2c
+        d[2] = v1[0]; d[3] = v1[1];  // group 2c + 1
+        d[4] = v2[0]; d[5] = v2[1];
+    } else {
+        const uint32_t g = min(2 * step + (qd >> 1), groups - 1), hf = qd & 1;  // (past the row: its last group)
+        if constexpr (TY == G_F16) {
+            const u32x4* b = (const u32x4*)(row + (size_t)g * 64 + 32 * hf);
+            const u32x4 v0 = b[0], v1 = b[1];
+            d[0] = v0[0]; d[1] = v0[1]; d[2] = v0[2]; d[3] = v0[3];
+            d[4] = v1[0]; d[5] = v1[1]; d[6] = v1[2]; d[7] = v1[3];
+        } else {
+            constexpr uint32_t BS = TY == G_Q8_0 ? 34 : TY == G_Q4_0 ? 18 : TY == G_Q4_1 ? 20 : TY == G_Q5_0 ? 22 : 24;
+            constexpr uint32_t QS = TY == G_Q8_0 || TY == G_Q4_0 ? 2 : TY == G_Q4_1 ? 4 : TY == G_Q5_0 ? 6 : 8;
+            const uint8_t* b = row + (size_t)g * BS;
+            const u32x4 v = ldu<u32x4>(b + QS + (TY == G_Q8_0 ? 16 * hf : 0));
+            d[0] = v[0]; d[1] = v[1]; d[2] = v[2]; d[3] = v[3];
+            d[4] = (TY == G_Q4_1 || TY == G_Q5_1) ? ldu<uint32_t>(b) : (uint32_t)*(const uint16_t*)b;
+            if constexpr (TY == G_Q5_0 || TY == G_Q5_1) d[5] = ldu<uint32_t>(b + (TY == G_Q5_0 ? 2 : 4));
+        }
+    }
+}
+
+template <uint32_t TY>
+__device__ __forceinline__ void tl_head(const uint8_t* __restrict__ row, uint32_t u, uint32_t (&h)[TLH<TY>]) {
+    if constexpr (tl_kq<TY>()) {
+        const u32x4 v = *(const u32x4*)(row + (size_t)u * (TY == G_Q4K ? 144 : 176));
+        h[0] = v[0]; h[1] = v[1]; h[2] = v[2]; h[3] = v[3];
+    } else if constexpr (TY == G_Q6K) {
+        const uint8_t* b = row + (size_t)u * 210 + 192;
+        const u32x4 v = ldu<u32x4>(b);
+        h[0] = v[0]; h[1] = v[1]; h[2] = v[2]; h[3] = v[3];
+        h[4] = *(const uint16_t*)(b + 16);
+    }
+}
+
+// Unpacks a thread's share of a step (its unit's step c) into LDS: its bytes of its row's B
+// operands (piece 4 g + c': group g's k slots 8c' ..; Q6K: the four weights of each half of
+// lane c'), the group scales (sa), and at a unit's first step the unit's factors: d and b
+// (uf) and the eight m's (um). h: the unit's header as loaded (c == 0), kept as m.
+template <uint32_t TY, bool FULL, int NT = TL_NT>
+__device__ __forceinline__ void tl_stash(const uint32_t (&d)[TLP<TY>], const uint32_t (&h)[TLH<TY>], MMUnit& m,
+                                         uint32_t step, uint32_t c, uint32_t r, uint32_t qd, uint32_t groups,
+                                         uint8_t* wl, float* sa, float* uf, f16* um) {
+    auto at = [&](uint32_t piece) { return wl + r * 128 + 16 * (piece ^ ((r >> 1) & 7u)); };
+    auto put = [&](uint32_t piece, half8 v) { *(half8*)at(piece) = v; };
+    if constexpr (tl_kq<TY>()) {
+        if (c == 0) {
+            const uint32_t dd[MWD<TY>] = {h[0], h[1], h[2], h[3]};
+            m = mm_unit<TY>(dd);
+            if (qd == 0) *(float2*)(uf + 2 * r) = float2{m.dl, m.bl};
+            if (qd == 1) *(half8*)(um + 8 * r) = mins_f16(m.mnA, m.mnB);
+        }
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const uint32_t e = tid + h * NT, rr = blockIdx.x * (16 * W) + e % (16 * W), in = i0 + e / (16 * W);
-        if (ok[h]) p.out[(size_t)in * p.rows + rr] = sum[h];
+        for (uint32_t hi = 0; hi < 2; hi++) {
+            const uint32_t j = 2 * c + hi, sc = ((j < 4 ? m.scA : m.scB) >> (8 * (j & 3u))) & 255u;
+            const half2 e = __builtin_bit_cast(half2, sc * 0x00010001u | 0x64006400u);
+            const f16 s16 = (TY == G_Q4K && hi) ? (f16)0.0625f : (f16)1.0f;
+            const half2 c1 = __builtin_elementwise_fma(e, half2{s16, s16}, half2{(f16)-1024.0f * s16, (f16)-1024.0f * s16});
+            const half2 c2 = c1 * half2{(f16)-1024.0f, (f16)-1024.0f};
+            const uint32_t v0 = d[0], v1 = d[1];
+            if constexpr (TY == G_Q4K) {
+                const uint32_t mk = hi ? 0x00f000f0u : 0x000f000fu;
+                put(4 * hi + qd, __builtin_bit_cast(half8, u32x4{field_pair_sc(v0, mk, c1, c2), field_pair_sc(v0 >> 8, mk, c1, c2),
+                                                                 field_pair_sc(v1, mk, c1, c2), field_pair_sc(v1 >> 8, mk, c1, c2)}));
+            } else {
+                const uint32_t h0 = d[2] >> j, h1 = d[3] >> j, n0 = hi ? v0 >> 4 : v0, n1 = hi ? v1 >> 4 : v1;
+                const uint32_t m4 = 0x000f000fu, b4 = 0x00010001u;
+                put(4 * hi + qd, __builtin_bit_cast(half8, u32x4{field_pair_sc(n0, m4, c1, c2, (h0 & b4) << 4),
+                                                                 field_pair_sc(n0 >> 8, m4, c1, c2, ((h0 >> 8) & b4) << 4),
+                                                                 field_pair_sc(n1, m4, c1, c2, (h1 & b4) << 4),
+                                                                 field_pair_sc(n1 >> 8, m4, c1, c2, ((h1 >> 8) & b4) << 4)}));
+            }
+        }
+    } else if constexpr (TY == G_Q6K) {
+        // The row's 16 scales, a dword a step, and d.
+        if (c == 0) {
+            m.scA = h[0];
+            m.scB = h[1];
+            m.mnA = h[2];
+            m.mnB = h[3];
+            m.dl = h2f(h[4]);
+        }
+        const half2 o = half2{(f16)1056.0f, (f16)1056.0f};
+#pragma unroll
+        for (uint32_t g = 0; g < 2; g++) {
+            const uint32_t qr = 2 * (c % 2) + g, ns = (c % 2) * 4;
+            const uint32_t v0 = ((d[2 * g] >> ns) & 0x0f0f0f0fu) | (((d[4] >> (2 * qr)) & 0x03030303u) << 4);
+            const uint32_t v1 = ((d[2 * g + 1] >> ns) & 0x0f0f0f0fu) | (((d[5] >> (2 * qr)) & 0x03030303u) << 4);
+            // weights 8 qd .. 8 qd + 7: half qd >> 1, lanes 2 (qd & 1) and the next
+            const uint32_t c2 = 2 * (qd & 1u);
+            *(half4*)(at(4 * g + c2) + 8 * (qd >> 1)) = __builtin_bit_cast(half4, bytes_f16(v0, o));
+            *(half4*)(at(4 * g + c2 + 1) + 8 * (qd >> 1)) = __builtin_bit_cast(half4, bytes_f16(v1, o));
+        }
+        const uint32_t sw = c == 0 ? m.scA : c == 1 ? m.scB : c == 2 ? m.mnA : m.mnB;  // the step's four scales
+        sa[qd * NT + r] = m.dl * (float)(int8_t)(uint8_t)(sw >> (8 * qd));
+    } else {
+        const uint32_t gi = qd >> 1, hf = qd & 1, piece = 4 * gi + 2 * hf;
+        if constexpr (TY == G_F16) {
+            put(piece, __builtin_bit_cast(half8, u32x4{d[0], d[1], d[2], d[3]}));
+            put(piece + 1, __builtin_bit_cast(half8, u32x4{d[4], d[5], d[6], d[7]}));
+        } else {
+            if (hf == 0) sa[gi * NT + r] = h2f(d[4] & 0xffffu);
+            if constexpr (TY == G_Q4_1 || TY == G_Q5_1) {
+                // m of the step's groups; at the unit's first step 0 for those past the row
+                const uint32_t g = 2 * step + gi;
+                if (!FULL && c == 0)
+#pragma unroll
+                    for (uint32_t k = 0; k < 2; k++)
+                        if (2 * step + 2 * qd + k >= groups) um[8 * r + 2 * qd + k] = (f16)0.0f;
+                if (hf == 1 && g < groups) um[8 * r + (g & 7u)] = __builtin_bit_cast(f16, (uint16_t)(d[4] >> 16));
+            }
+            if constexpr (TY == G_Q8_0) {
+                const half2 o = half2{(f16)1152.0f, (f16)1152.0f};
+                put(piece, bytes8_f16(d[0] ^ 0x80808080u, d[1] ^ 0x80808080u, o));
+                put(piece + 1, bytes8_f16(d[2] ^ 0x80808080u, d[3] ^ 0x80808080u, o));
+            } else {
+                const uint32_t ns = 4 * hf;
+                constexpr bool FIVE = TY == G_Q5_0 || TY == G_Q5_1;
+                const f16 off = TY == G_Q4_0 ? (f16)1032.0f : TY == G_Q5_0 ? (f16)1040.0f : (f16)1024.0f;
+#pragma unroll
+                for (uint32_t k = 0; k < 2; k++) {
+                    if constexpr (FIVE) {
+                        const uint32_t qh = (d[5] >> (16 * hf + 8 * k)) & 255u;
+                        put(piece + k, bytes8_f16(((d[2 * k] >> ns) & 0x0f0f0f0fu) | bit4_spread(qh & 15u),
+                                                  ((d[2 * k + 1] >> ns) & 0x0f0f0f0fu) | bit4_spread(qh >> 4), half2{off, off}));
+                    } else {
+                        put(piece + k, fields8(d[2 * k] >> ns, d[2 * k + 1] >> ns, 0x000f000fu, half2{off, off}));
+                    }
+                }
+            }
+        }
+    }
+}
+
+// Small batches whose cols is no multiple of 256, in one launch: a workgroup is 16 weight rows x
+// 8 input rows, its W waves (four for at most four units: more workgroups then share a CU, else
+// eight) take the units in turn, each staging its own unit's x (as k_matmul_mm does) and weights
+// (as the tile kernel does) in its own LDS without a barrier, and the units' sums meet in order.
+// Bound by latency: Q8_0 4864 x 896 at 2 / 6 / 16 rows 5.3 / 6.2 / 9.2 us (the VALU pass of 8
+// rows 7.8 / 14 / 31; the tile kernel and its preparation 13).
+constexpr uint32_t WV_UNITS = 56;  // units whose sums fit the workgroup's LDS
+
+template <uint32_t TY, int W>
+__global__ __launch_bounds__(64 * W) void k_matmul_units(const TLParams p, const float* __restrict__ x, uint32_t cols) {
+    constexpr bool SUM = mm_sum<TY>(), UT = TY == G_F16;
+    constexpr int XS = 264;  // halves an x row
+    static_assert(!tl_kq<TY>() && TY != G_Q6K, "formats of 32-weight blocks");
+    __shared__ __attribute__((aligned(16))) f16 xs[W][16 * XS];  // inputs' hi, then lo
+    __shared__ __attribute__((aligned(16))) uint8_t wl[W][2][16 * 128];
+    __shared__ float sa[W][2][UT ? 1 : 2 * 16];
+    __shared__ __attribute__((aligned(16))) f16 um[W][SUM ? 8 * 16 : 1];
+    __shared__ __attribute__((aligned(16))) f16 ss[W][SUM ? 8 * 32 : 1];
+    __shared__ float ps[WV_UNITS][8][16], isc[WV_UNITS][8];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t c = lane >> 4, l = lane & 15, tr = lane >> 2, qd = lane & 3;
+    const uint32_t r0 = blockIdx.x * 16, i0 = blockIdx.y * 8, ni = min(8u, p.n - i0);
+    const uint8_t* wrow = p.w + (size_t)min(r0 + tr, p.rows - 1) * p.row_bytes;
+    const f32x4 z4 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t nsteps = (p.groups + 1) / 2;
+    // LDS written and read by one wave only: in order, no barrier.
+    auto own = [&]() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+    if constexpr (SUM)
+        if (lane < 8) *(half8*)&ss[w][32 * lane + 24] = half8{};
+    for (uint32_t u = w; u < p.units; u += W) {
+        uint32_t pk[4][TLP<TY>], hd[TLH<TY>];
+        MMUnit mu;
+        const uint32_t ns = min(4u, nsteps - 4 * u);
+#pragma unroll
+        for (uint32_t s = 0; s < 4; s++) tl_load<TY>(wrow, min(4 * u + s, nsteps - 1), qd, p.groups, pk[s]);
+        const uint32_t col = 256 * u + 4 * lane;
+        float4 v[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; i++)
+            v[i] = *(const float4*)(x + (size_t)(i0 + min(i, ni - 1)) * cols + min(col, cols - 4));
+#pragma unroll
+        for (uint32_t i = 0; i < 8; i++) {
+            if (i >= ni) break;
+            const bool in = col < cols;
+            const float x4[4] = {in ? v[i].x : 0.0f, in ? v[i].y : 0.0f, in ? v[i].z : 0.0f, in ? v[i].w : 0.0f};
+            float sc, inv;
+            unit_scale(x4, sc, inv);
+            if (lane == 0) isc[u][i] = inv;
+            if constexpr (SUM) {
+                const float sg = group_sum(x4);
+                if ((lane & 7) == 0) {
+                    f16 sp[3];
+                    sum_parts(sg, sc, sp);
+#pragma unroll
+                    for (int e = 0; e < 3; e++) ss[w][i * 32 + 8 * e + lane / 8] = sp[e];
+                }
+            }
+            const float xo[4] = {x4[0], UT ? x4[1] : x4[2], UT ? x4[2] : x4[1], x4[3]};
+            half4 h, o;
+            hi_lo(xo, sc, h, o);
+            *(half4*)&xs[w][i * XS + 4 * lane] = h;
+            *(half4*)&xs[w][(8 + i) * XS + 4 * lane] = o;
+        }
+        f32x4 t = z4;  // hi in lanes c < 2, lo in c >= 2
+#pragma unroll
+        for (uint32_t s = 0; s < 4; s++) {
+            if (s >= ns) break;
+            tl_stash<TY, false, 16>(pk[s], hd, mu, 4 * u + s, s, tr, qd, p.groups, wl[w][s & 1], sa[w][s & 1], nullptr, um[w]);
+            own();
+#pragma unroll
+            for (uint32_t g = 0; g < 2; g++) {
+                if (8 * u + 2 * s + g >= p.groups) break;
+                const half8 b = *(const half8*)(wl[w][s & 1] + l * 128 + 16 * ((4 * g + c) ^ ((l >> 1) & 7u)));
+                const half8 xa = *(const half8*)&xs[w][l * XS + 64 * s + 32 * g + 8 * c];
+                if constexpr (UT) {
+                    t = mfma16(xa, b, t);
+                } else {
+                    const f32x4 d = mfma16(xa, b, z4);
+                    const float a = sa[w][s & 1][g * 16 + l];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) t[e] = __builtin_fmaf(a, d[e], t[e]);
+                }
+            }
+            own();
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[e]), __float_as_uint(t[e]), false, false);
+            t[e] = __uint_as_float(r2[0]) + __uint_as_float(r2[1]);
+        }
+        if constexpr (SUM) {
+            const f32x4 tb = mfma16(*(const half8*)&ss[w][(l & 7u) * 32 + 8 * c], *(const half8*)&um[w][8 * l], z4);
+#pragma unroll
+            for (int e = 0; e < 4; e++) t[e] = __builtin_fmaf(32.0f, tb[e], t[e]);
+            own();
+        }
+        if (c < 2)
+#pragma unroll
+            for (int e = 0; e < 4; e++) ps[u][4 * c + e][l] = t[e];
+    }
+    __syncthreads();
+    // The units' sums in order, split by split (k_matmul_mm's accumulation).
+    if (tid >= 128) return;
+    const uint32_t i = tid >> 4, r = r0 + (tid & 15);
+    if (i >= ni || r >= p.rows) return;
+    float tot = 0.0f;
+    for (uint32_t kz = 0; kz < p.ks; kz++) {
+        const uint32_t ua = kz * p.units / p.ks, ue = (kz + 1) * p.units / p.ks;
+        float acc = 0.0f;
+        for (uint32_t u = ua; u < ue; u++) acc = __builtin_fmaf(isc[u][i], ps[u][i][tid & 15], acc);
+        tot = kz == 0 ? acc : tot + acc;
+    }
+    p.out[(size_t)(i0 + i) * p.rows + r] = tot;
+}
+
+// FULL: cols is a multiple of 256, so a unit is four whole steps of straight-line code.
+template <uint32_t TY, int TM, int TN, int WM, bool FULL>
+__global__ __launch_bounds__(TL_THREADS, 2) void k_matmul_tile(const TLParams p) {
+    constexpr int WN = 8 / WM, MT = 16 * TM * WM;
+    static_assert(16 * TN * WN == TL_NT, "eight waves cover the weight rows");
+    constexpr bool SUM = mm_sum<TY>(), KQ = tl_kq<TY>(), UT = KQ || TY == G_F16;
+    constexpr int XL = MT * 16 / TL_THREADS;  // 16-byte pieces of x a thread moves a step
+    static_assert(XL >= 1 && MT * 16 % TL_THREADS == 0 && 4 * MT <= TL_THREADS, "a step's x divides over the threads");
+    // One LDS object a stage: the compiler then waits only for the stage it reads.
+    __shared__ __attribute__((aligned(16))) uint8_t xl0[MT * 256], xl1[MT * 256], wl0[TL_NT * 128], wl1[TL_NT * 128];
+    __shared__ __attribute__((aligned(16))) float is[2][MT];
+    __shared__ float sa[2][UT ? 1 : (TY == G_Q6K ? 4 : 2) * TL_NT];
+    __shared__ __attribute__((aligned(16))) float uf[2][KQ ? 2 * TL_NT : 1];
+    __shared__ __attribute__((aligned(16))) f16 um[2][SUM ? 8 * TL_NT : 1];
+    __shared__ __attribute__((aligned(16))) f16 us[2][SUM ? 32 * MT : 1];
+    __shared__ uint32_t last;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t c = lane >> 4, l = lane & 15;
+    // Workgroups 8 apart share an XCD: consecutive ones there take the input tiles of one
+    // stretch of weight rows, so that its packed bytes come from the XCD's L2 after the first.
+    const uint32_t xcd = blockIdx.x % 8, tile = xcd * (gridDim.x / 8) + min(xcd, gridDim.x % 8) + blockIdx.x / 8;
+    const uint32_t wx = tile / p.nyt, wy = tile % p.nyt;
+    const uint32_t r0 = wx * TL_NT, i0 = wy * MT;
+    const uint32_t tr = tid >> 2, qd = tid & 3;  // the weight row and quarter this thread unpacks
+    const uint8_t* wrow = p.w + (size_t)min(r0 + tr, p.rows - 1) * p.row_bytes;
+    const uint32_t wm = wv / WN, wn = wv % WN;   // the wave's tiles: inputs 16 TM wm .., rows 16 TN wn ..
+    const f32x4 z4 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t kz0 = p.par ? blockIdx.z : 0, kz1 = p.par ? blockIdx.z + 1 : p.ks;
+    const uint32_t nsteps = (p.groups + 1) / 2;
+    // LDS offsets of the lane's operands: piece 4 g + c of row l of a tile; x rows are 16
+    // pieces swizzled by the row, weight rows 8 pieces swizzled by the row pair.
+    const uint32_t xa = (16 * TM * wm + l) * 256, wa = (16 * TN * wn + l) * 128, wsw = (l >> 1) & 7u;
+    uint32_t pk[2][TLP<TY>];  // packed weights of the next step and the one after
+    uint32_t hd[TLH<TY>];     // the next unit's header
+    MMUnit mu;
+    u32x4 sr = u32x4{};
+    float ir = 0.0f;
+    // A step's x straight into its LDS stage, 1 KB (four rows) a wave and load; lane i fetches
+    // the piece that belongs in its 16 bytes.
+    auto fetch_x = [&](uint32_t s, uint8_t* dst) {
+#pragma unroll
+        for (int i = 0; i < XL; i++) {
+            const uint32_t blk = wv * XL + i, row = 4 * blk + c;
+            const uint8_t* base = (const uint8_t*)p.xp + ((size_t)s * p.npad + i0) * 256;  // uniform
+            const uint32_t off = row * 256 + 16 * (l ^ (row & 15u));
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + off),
+                                             (__attribute__((address_space(3))) void*)(dst + blk * 1024), 16, 0, 0);
+        }
+    };
+    auto fetch_unit = [&](uint32_t u) {
+        const size_t at = (size_t)u * p.npad + i0;
+        tl_head<TY>(wrow, u, hd);
+        ir = p.ip[at + min(tid, (uint32_t)MT - 1u)];
+        if constexpr (SUM) sr = *(const u32x4*)(p.sp + at * 32 + 8 * min(tid, 4u * MT - 1u));
+    };
+    auto stash = [&](const uint32_t (&pw)[TLP<TY>], uint32_t s, uint32_t cc) {
+        const uint32_t ub = (s >> 2) & 1;
+        tl_stash<TY, FULL>(pw, hd, mu, s, cc, tr, qd, p.groups, cc & 1 ? wl1 : wl0, sa[cc & 1], uf[ub], um[ub]);
+        if (cc == 0) {
+            if (tid < (uint32_t)MT) is[ub][tid] = ir;
+            if constexpr (SUM)
+                if (tid < 4u * MT) *(u32x4*)(us[ub] + 8 * (tid ^ ((tid >> 4) & 3u))) = sr;
+        }
+    };
+    f32x4 tot[TM][TN];
+    for (uint32_t kz = kz0; kz < kz1; kz++) {
+        const uint32_t ua = kz * p.units / p.ks, ue = (kz + 1) * p.units / p.ks;
+        const uint32_t s1 = min(4 * ue, nsteps);
+        // t and to: hi and lo (Q6K: both in t)
+        f32x4 ac[TM][TN], t[TM][TN], to[TY == G_Q6K ? 1 : TM][TY == G_Q6K ? 1 : TN];
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) ac[i][j] = z4;
+        if (kz != kz0) __syncthreads();  // the previous split's last step is read
+        fetch_unit(ua);
+        tl_load<TY>(wrow, 4 * ua, qd, p.groups, pk[0]);
+        fetch_x(4 * ua, xl0);
+        tl_load<TY>(wrow, min(4 * ua + 1, s1 - 1), qd, p.groups, pk[1]);
+        stash(pk[0], 4 * ua, 0);
+        __syncthreads();
+        for (uint32_t u = ua; u < ue; u++) {
+#pragma unroll
+            for (uint32_t cc = 0; cc < 4; cc++) {
+                const uint32_t s = 4 * u + cc;
+                if (!FULL && s >= s1) break;
+                // Step s + 1's x into the other stage, its packed weights (loaded a step ago)
+                // unpacked beside this step's MFMAs, step s + 2's packed weights on their way.
+                // (FULL: past the range's end its last step again into the stage no one reads any
+                // more, so that no branch splits the unit: across one the compiler gathers every
+                // step's FMAs at the unit's end and spills.)
+                const uint8_t *xb = (cc & 1 ? xl1 : xl0) + xa, *wb = (cc & 1 ? wl1 : wl0) + wa;
+                // The first operand before the new loads go out: the compiler waits for every load in
+                // flight at a stage's first read, which then are only those of a step ago.
+                const half8 xf = *(const half8*)(xb + 16 * (c ^ l));
+                __builtin_amdgcn_sched_barrier(0);
+                const bool more = FULL || s + 1 < s1;
+                const uint32_t sn = min(s + 1, s1 - 1);
+                if (more) {
+                    if (cc == 2) fetch_unit(min(u + 1, ue - 1));
+                    fetch_x(sn, cc & 1 ? xl0 : xl1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    tl_load<TY>(wrow, min(s + 2, s1 - 1), qd, p.groups, pk[cc & 1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (uint32_t g = 0; g < 2; g++) {
+                    if (!FULL && 2 * s + g >= p.groups) break;
+                    half8 b[TN];
+                    float a0[TN], a1[TN];
+#pragma unroll
+                    for (int j = 0; j < TN; j++) {
+                        b[j] = *(const half8*)(wb + 2048 * j + 16 * ((4 * g + c) ^ wsw));
+                        const uint32_t r = 16 * (TN * wn + j) + l;
+                        if constexpr (TY == G_Q6K) {
+                            a0[j] = sa[cc & 1][(2 * g) * TL_NT + r];
+                            a1[j] = sa[cc & 1][(2 * g + 1) * TL_NT + r];
+                        } else if constexpr (!UT) {
+                            a0[j] = sa[cc & 1][g * TL_NT + r];
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < TM; i++) {
+                        const uint32_t p0 = TY == G_Q6K ? 8 * g + c : 4 * g + c, p1 = TY == G_Q6K ? p0 + 4 : p0 + 8;
+                        const half8 x0 = g == 0 && i == 0 ? xf : *(const half8*)(xb + 4096 * i + 16 * (p0 ^ l));
+                        const half8 x1 = *(const half8*)(xb + 4096 * i + 16 * (p1 ^ l));
+#pragma unroll
+                        for (int j = 0; j < TN; j++) {
+                            if constexpr (UT) {
+                                t[i][j] = mfma16(x0, b[j], cc == 0 && g == 0 ? z4 : t[i][j]);
+                                to[i][j] = mfma16(x1, b[j], cc == 0 && g == 0 ? z4 : to[i][j]);
+                            } else if constexpr (TY == G_Q6K) {
+                                const f32x4 h0 = mfma16(x0, __builtin_shufflevector(b[j], b[j], 0, 1, 2, 3, 0, 1, 2, 3), z4);
+                                const f32x4 h1 = mfma16(x1, __builtin_shufflevector(b[j], b[j], 4, 5, 6, 7, 4, 5, 6, 7), z4);
+#pragma unroll
+                                for (int e = 0; e < 4; e++)
+                                    t[i][j][e] = __builtin_fmaf(a1[j], h1[e], __builtin_fmaf(a0[j], h0[e], cc == 0 && g == 0 ? 0.0f : t[i][j][e]));
+                            } else {
+                                const f32x4 h = mfma16(x0, b[j], z4), o = mfma16(x1, b[j], z4);
+#pragma unroll
+                                for (int e = 0; e < 4; e++) {
+                                    t[i][j][e] = __builtin_fmaf(a0[j], h[e], cc == 0 && g == 0 ? 0.0f : t[i][j][e]);
+                                    to[i][j][e] = __builtin_fmaf(a0[j], o[e], cc == 0 && g == 0 ? 0.0f : to[i][j][e]);
+                                }
+                            }
+                        }
+                        // The FMAs stay here: the compiler otherwise sinks a unit's to its end, every
+                        // MFMA's result kept until then, and spills.
+                        if constexpr (!UT)
+#pragma unroll
+                            for (int j = 0; j < TN; j++) {
+                                asm volatile("" : "+v"(t[i][j]));
+                                if constexpr (TY != G_Q6K) asm volatile("" : "+v"(to[i][j]));
+                            }
+                    }
+                }
+                if (cc == 3 || (!FULL && s + 1 == s1)) {  // the unit's end
+                    const uint32_t ub = u & 1;
+                    float dl[TN], bl[TN];
+                    half8 mv[TN];
+#pragma unroll
+                    for (int j = 0; j < TN; j++) {
+                        const uint32_t r = 16 * (TN * wn + j) + l;
+                        dl[j] = 1.0f;
+                        bl[j] = 32.0f;
+                        if constexpr (KQ) {
+                            const float2 f = *(const float2*)(uf[ub] + 2 * r);
+                            dl[j] = f.x;
+                            bl[j] = f.y;
+                        }
+                        if constexpr (SUM) mv[j] = *(const half8*)(um[ub] + 8 * r);
+                    }
+#pragma unroll
+                    for (int i = 0; i < TM; i++) {
+                        const f32x4 i4 = *(const f32x4*)&is[ub][16 * (TM * wm + i) + 4 * c];
+                        half8 sv;
+                        if constexpr (SUM) {
+                            const uint32_t e = 4 * (16 * (TM * wm + i) + l) + c;
+                            sv = *(const half8*)(us[ub] + 8 * (e ^ ((e >> 4) & 3u)));
+                        }
+#pragma unroll
+                        for (int j = 0; j < TN; j++) {
+                            f32x4 v = t[i][j];
+                            if constexpr (TY != G_Q6K) v += to[i][j];
+                            if constexpr (KQ) v *= dl[j];
+                            if constexpr (SUM) {
+                                const f32x4 tb = mfma16(sv, mv[j], z4);
+#pragma unroll
+                                for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf(bl[j], tb[e], v[e]);
+                            }
+#pragma unroll
+                            for (int e = 0; e < 4; e++) ac[i][j][e] = __builtin_fmaf(i4[e], v[e], ac[i][j][e]);
+                        }
+                    }
+                }
+                if (more) stash(pk[(cc + 1) & 1], sn, (cc + 1) & 3);
+                // The next step's x has landed (of the loads in flight only the last weight loads,
+                // TLN or more, may be left) and its LDS writes are done. (__syncthreads would wait
+                // for every load.)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(TLN<TY>) : "memory");
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) tot[i][j][e] = kz == kz0 ? ac[i][j][e] : tot[i][j][e] + ac[i][j][e];
+    }
+    // Element e of tile (i, j) in lane (c, l): input 4c + e, weight row l.
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t in = i0 + 16 * (TM * wm + i) + 4 * c + e;
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const uint32_t r = r0 + 16 * (TN * wn + j) + l;
+                if (r >= p.rows) continue;
+                if (p.par)
+                    __hip_atomic_store(&p.part[((size_t)blockIdx.z * p.npad + in) * p.rows + r], tot[i][j][e],
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else if (in < p.n)
+                    p.out[(size_t)in * p.rows + r] = tot[i][j][e];
+            }
+        }
+    if (!p.par) return;
+    // Parallel splits, as k_matmul_mm's: the tile's last workgroup adds the partials in order.
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (tid == 0) {
+        const uint32_t old = __hip_atomic_fetch_add(&p.cnt[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = old == p.ks - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    const size_t stride = (size_t)p.npad * p.rows;
+    const uint32_t rr = r0 + tid % TL_NT;
+    constexpr uint32_t IP = TL_THREADS / TL_NT;  // inputs a pass of the workgroup
+    for (uint32_t q = 0; q < (uint32_t)MT; q += 2 * IP) {
+        float sum[2] = {0.0f, 0.0f};
+        for (uint32_t k0 = 0; k0 < p.ks; k0 += 8) {
+            float v[2][8];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const float* src = p.part + (size_t)(i0 + q + IP * h + tid / TL_NT) * p.rows + min(rr, p.rows - 1);
+#pragma unroll
+                for (int t = 0; t < 8; t++)
+                    v[h][t] = k0 + t < p.ks ? __hip_atomic_load(src + (k0 + t) * stride, __ATOMIC_RELAXED,
+                                                                 __HIP_MEMORY_SCOPE_AGENT)
+                                            : 0.0f;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int t = 0; t < 8; t++)
+                    if (k0 + t < p.ks) sum[h] = k0 + t == 0 ? v[h][t] : sum[h] + v[h][t];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t in = i0 + q + IP * h + tid / TL_NT;
+            if (in < p.n && rr < p.rows) p.out[(size_t)in * p.rows + rr] = sum[h];
+        }
     }
     if (tid == 0) __hip_atomic_store(&p.cnt[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -947,8 +1666,9 @@ static uint32_t mm_rows(uint32_t type) {
 // K splits of a product: about two workgroups a CU from the rows alone (never from n), each
 // split at most MM_K units.
 static uint32_t mm_ks(uint32_t type, uint32_t rows, uint32_t cols) {
-    const uint32_t rt = (rows + mm_rows(type) - 1) / mm_rows(type), units = cols / 256;
+    const uint32_t rt = (rows + mm_rows(type) - 1) / mm_rows(type), units = (cols + 255) / 256;
     const uint32_t kmax = type == G_F16 ? MM_K<G_F16> : MM_K<G_Q4K>;
+    if (cols % 256 != 0 && units <= 16) return 1;  // (no k_matmul_mm form: short ranges stay whole)
     uint32_t ks = max(512u / rt, 1u);
     ks = max(ks, (units + kmax - 1) / kmax);
     ks = min(ks, units);
@@ -959,29 +1679,142 @@ static bool mm_par(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n) {
     return mm_ks(type, rows, cols) > 1 && (uint64_t)rt * nt <= MM_PAR;
 }
 
-bool matmul_uses_mm(uint32_t type, uint32_t cols, uint32_t n) {
+static bool mm_types(uint32_t type) {
     switch (type) {
         case G_F16: case G_Q8_0: case G_Q4_0: case G_Q4_1: case G_Q5_0: case G_Q5_1: case G_Q4K: case G_Q5K:
-        case G_Q6K: return n >= MM_MIN && cols % 256 == 0;
+        case G_Q6K: return true;
         default: return false;
     }
 }
 
-size_t matmul_scratch_bytes(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n) {
+static bool matmul_uses_mm(uint32_t type, uint32_t cols, uint32_t n) {
+    return mm_types(type) && n >= MM_MIN && cols % 256 == 0;
+}
+
+// Which kernel takes a batch of the matrix-core formats; all give an input row the same bits.
+// Batches of 17 rows and 2^29.5 multiply-adds take the tile kernel over k_matmul_mm (Q8_0 896 x
+// 4864 at 67 rows, 0.29 G: 20 us there, 38 here; Q4K 14336 x 4096 at 17, 1.0 G: 31 us there, 26
+// here); with cols no multiple of 256 over k_matmul_units, from 2^27 (Q8_0 4864 x 896 at 16
+// rows, 0.07 G: 9.2 us there, 15.8 here; at 67, 0.29 G: about 35 there, 20 here).
+constexpr uint32_t TL_MIN = 17;
+constexpr uint64_t TL_MACS = 760000000, TL_MACS_RAGGED = 134000000;
+// Bytes of prepared x a launch takes at most; longer batches go in slabs of input rows.
+constexpr size_t TL_SLAB_BYTES = (size_t)256 << 20;
+
+static bool matmul_uses_units(uint32_t type, uint32_t cols, uint32_t n) {
+    return mm_types(type) && cols % 256 != 0 && n >= MM_MIN && (cols + 255) / 256 <= WV_UNITS;
+}
+bool matmul_uses_tile(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n) {
+    const uint64_t macs = (uint64_t)rows * cols * n;
+    if (!mm_types(type)) return false;
+    if (cols % 256 == 0) return n >= TL_MIN && macs >= TL_MACS;
+    return n >= MM_MIN && (!matmul_uses_units(type, cols, n) || (n >= TL_MIN && macs >= TL_MACS_RAGGED));
+}
+
+struct TilePlan {
+    uint32_t mt, slab, npad, units, groups, ks, nxt, nyt, par;  // npad, nyt, par: of a whole slab
+    size_t xp_bytes, ip_bytes, sp_bytes, part_bytes;
+};
+static TilePlan tile_plan(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n) {
+    TilePlan t{};
+    t.units = (cols + 255) / 256;
+    t.groups = cols / 32;
+    t.nxt = (rows + TL_NT - 1) / TL_NT;
+    const size_t row_bytes = (size_t)(t.groups + 1) / 2 * 256;
+    t.slab = (uint32_t)std::max<size_t>(TL_SLAB_BYTES / row_bytes / 128 * 128, 128);
+    const uint32_t m = min(n, t.slab);
+    // Input rows a workgroup: 128 where that still gives every CU one.
+    t.mt = m <= 32 ? 32 : (m > 64 && (uint64_t)t.nxt * ((m + 127) / 128) >= 256) ? 128 : 64;
+    t.npad = (m + t.mt - 1) / t.mt * t.mt;
+    t.nyt = t.npad / t.mt;
+    t.ks = mm_ks(type, rows, cols);
+    // K splits in parallel where the tiles alone would leave half the CUs without work.
+    t.par = t.ks > 1 && (uint64_t)t.nxt * t.nyt <= 128;
+    t.xp_bytes = (size_t)t.npad * row_bytes;
+    t.ip_bytes = ((size_t)t.units * t.npad * sizeof(float) + 255) / 256 * 256;
+    t.sp_bytes = (size_t)t.units * t.npad * 64;
+    t.part_bytes = t.par ? (size_t)t.ks * t.npad * rows * sizeof(float) : 0;
+    return t;
+}
+
+size_t matmul_scratch_bytes(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n, bool tile) {
+    if (tile) {
+        const TilePlan t = tile_plan(type, rows, cols, n);
+        return t.xp_bytes + t.ip_bytes + t.sp_bytes + t.part_bytes;
+    }
     if (!matmul_uses_mm(type, cols, n) || !mm_par(type, rows, cols, n)) return 0;
-    return (size_t)mm_ks(type, rows, cols) * ((n + 7) / 8 * 8) * rows * sizeof(float);
+    return (size_t)mm_ks(type, rows, cols) * ((n + 15) / 16 * 16) * rows * sizeof(float);
 }
 
 template <uint32_t TY>
 static hipError_t matmul_mm_go(const MatmulParams& mp, void* scratch, uint32_t* counters, hipStream_t s) {
     const uint32_t ks = mm_ks(TY, mp.rows, mp.cols), rt = (mp.rows + 16 * MM_W<TY> - 1) / (16 * MM_W<TY>);
-    const uint32_t nt = (mp.n + 7) / 8;
     const bool par = mm_par(TY, mp.rows, mp.cols, mp.n);
     if (par && (!scratch || !counters)) return hipErrorInvalidValue;
-    const MMParams q{mp.w, mp.x, mp.out, (float*)scratch, counters, mp.rows, mp.cols, mp.n, nt * 8, mp.row_bytes,
-                     mp.cols / 256, ks, par ? 1u : 0u};
-    hipLaunchKernelGGL((k_matmul_mm<TY>), dim3(rt, nt, par ? ks : 1), dim3(64 * MM_W<TY>), 0, s, q);
+    const MMParams q{mp.w, mp.x, mp.out, (float*)scratch, counters, mp.rows, mp.cols, mp.n, (mp.n + 15) / 16 * 16,
+                     mp.row_bytes, mp.cols / 256, ks, par ? 1u : 0u};
+    // Sixteen inputs a workgroup for one such block over a matrix large enough to fill the GPU with
+    // half the workgroups (Q6K 4096 x 14336 at 16 rows: 29 us against 31; Q8_0 896 x 4864 at 17:
+    // 16 against 12). F16's x of 16 inputs would take most of the LDS.
+    if constexpr (TY != G_F16) {
+        if (mp.n > 8 && mp.n <= 16 && (uint64_t)mp.rows * mp.cols >= (1u << 23)) {
+            const dim3 grid(rt, (mp.n + 15) / 16, par ? ks : 1);
+            hipLaunchKernelGGL((k_matmul_mm<TY, 16>), grid, dim3(64 * MM_W<TY>), 0, s, q);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((k_matmul_mm<TY, 8>), dim3(rt, (mp.n + 7) / 8, par ? ks : 1), dim3(64 * MM_W<TY>), 0, s, q);
     return hipGetLastError();
+}
+
+template <uint32_t TY>
+static hipError_t matmul_units_go(const MatmulParams& mp, hipStream_t s) {
+    const uint32_t units = (mp.cols + 255) / 256;
+    const TLParams q{mp.w, nullptr, nullptr, nullptr, mp.out, nullptr, nullptr, mp.rows, mp.n, 0, mp.row_bytes,
+                     units, mp.cols / 32, mm_ks(TY, mp.rows, mp.cols), 0, 0};
+    const dim3 grid((mp.rows + 15) / 16, (mp.n + 7) / 8);
+    if (units <= 4)
+        hipLaunchKernelGGL((k_matmul_units<TY, 4>), grid, dim3(256), 0, s, q, mp.x, mp.cols);
+    else
+        hipLaunchKernelGGL((k_matmul_units<TY, 8>), grid, dim3(512), 0, s, q, mp.x, mp.cols);
+    return hipGetLastError();
+}
+
+template <uint32_t TY>
+static hipError_t matmul_tile_go(const MatmulParams& mp, void* scratch, uint32_t* counters, hipStream_t s) {
+    const TilePlan t = tile_plan(TY, mp.rows, mp.cols, mp.n);
+    if (!scratch || !counters) return hipErrorInvalidValue;
+    f16* xp = (f16*)scratch;
+    float* ip = (float*)((char*)scratch + t.xp_bytes);
+    f16* sp = (f16*)((char*)ip + t.ip_bytes);
+    float* part = (float*)((char*)sp + t.sp_bytes);
+    for (uint32_t n0 = 0; n0 < mp.n; n0 += t.slab) {
+        const uint32_t m = min(mp.n - n0, t.slab), nyt = (m + t.mt - 1) / t.mt, npad = nyt * t.mt;
+        hipLaunchKernelGGL((k_mm_prep<tl_order<TY>(), mm_sum<TY>()>), dim3(t.units, npad / 4), dim3(256), 0, s,
+                           mp.x + (size_t)n0 * mp.cols, xp, ip, sp, m, mp.cols, npad, (t.groups + 1) / 2);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        const TLParams q{mp.w, xp, ip, sp, mp.out + (size_t)n0 * mp.rows, part, counters, mp.rows, m, npad, mp.row_bytes,
+                         t.units, t.groups, t.ks, t.par, nyt};
+        const dim3 grid(t.nxt * nyt, 1, t.par ? t.ks : 1);
+        auto go = [&](auto full) {
+            constexpr bool FULL = decltype(full)::value;
+            if (t.mt == 128)
+                hipLaunchKernelGGL((k_matmul_tile<TY, 2, 4, 4, FULL>), grid, dim3(TL_THREADS), 0, s, q);
+            else if (t.mt == 64)
+                hipLaunchKernelGGL((k_matmul_tile<TY, 2, 2, 2, FULL>), grid, dim3(TL_THREADS), 0, s, q);
+            else
+                hipLaunchKernelGGL((k_matmul_tile<TY, 2, 1, 1, FULL>), grid, dim3(TL_THREADS), 0, s, q);
+        };
+        if (mp.cols % 256 == 0) {
+            go(std::true_type{});
+        } else if constexpr (!tl_kq<TY>() && TY != G_Q6K) {
+            go(std::false_type{});
+        }
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <uint32_t TY, int NBT, int R>
@@ -996,8 +1829,11 @@ static void matmul_go(const MatmulParams& mp, hipStream_t s) {
 // the matrix still gives 256+ workgroups (measured: the 14336 x 4096 Q4K product 21.3 ->
 // 14.2 µs), else four. Batches: four rows a wave, eight input rows a pass.
 template <uint32_t TY>
-static hipError_t matmul_t(const MatmulParams& mp, void* scratch, uint32_t* counters, hipStream_t s) {
+static hipError_t matmul_t(const MatmulParams& mp, bool tile, void* scratch, uint32_t* counters, hipStream_t s) {
     if constexpr (mm_type<TY>()) {
+        if (tile) return matmul_tile_go<TY>(mp, scratch, counters, s);
+        if constexpr (!tl_kq<TY>() && TY != G_Q6K)
+            if (matmul_uses_units(TY, mp.cols, mp.n)) return matmul_units_go<TY>(mp, s);
         if (matmul_uses_mm(TY, mp.cols, mp.n)) return matmul_mm_go<TY>(mp, scratch, counters, s);
     }
     if (mp.n == 1) {
@@ -1012,20 +1848,20 @@ static hipError_t matmul_t(const MatmulParams& mp, void* scratch, uint32_t* coun
 }
 
 hipError_t matmul_launch(const void* w, uint32_t type, const float* x, float* out, uint32_t rows, uint32_t cols,
-                         uint32_t n, uint32_t row_bytes, void* scratch, uint32_t* counters, hipStream_t s) {
+                         uint32_t n, uint32_t row_bytes, bool tile, void* scratch, uint32_t* counters, hipStream_t s) {
     const MatmulParams mp{(const uint8_t*)w, x, out, rows, cols, n, row_bytes};
     switch (type) {
-        case G_F32: return matmul_t<G_F32>(mp, scratch, counters, s);
-        case G_F16: return matmul_t<G_F16>(mp, scratch, counters, s);
-        case G_BF16: return matmul_t<G_BF16>(mp, scratch, counters, s);
-        case G_Q4_0: return matmul_t<G_Q4_0>(mp, scratch, counters, s);
-        case G_Q4_1: return matmul_t<G_Q4_1>(mp, scratch, counters, s);
-        case G_Q5_0: return matmul_t<G_Q5_0>(mp, scratch, counters, s);
-        case G_Q5_1: return matmul_t<G_Q5_1>(mp, scratch, counters, s);
-        case G_Q8_0: return matmul_t<G_Q8_0>(mp, scratch, counters, s);
-        case G_Q4K: return matmul_t<G_Q4K>(mp, scratch, counters, s);
-        case G_Q5K: return matmul_t<G_Q5K>(mp, scratch, counters, s);
-        case G_Q6K: return matmul_t<G_Q6K>(mp, scratch, counters, s);
+        case G_F32: return matmul_t<G_F32>(mp, tile, scratch, counters, s);
+        case G_F16: return matmul_t<G_F16>(mp, tile, scratch, counters, s);
+        case G_BF16: return matmul_t<G_BF16>(mp, tile, scratch, counters, s);
+        case G_Q4_0: return matmul_t<G_Q4_0>(mp, tile, scratch, counters, s);
+        case G_Q4_1: return matmul_t<G_Q4_1>(mp, tile, scratch, counters, s);
+        case G_Q5_0: return matmul_t<G_Q5_0>(mp, tile, scratch, counters, s);
+        case G_Q5_1: return matmul_t<G_Q5_1>(mp, tile, scratch, counters, s);
+        case G_Q8_0: return matmul_t<G_Q8_0>(mp, tile, scratch, counters, s);
+        case G_Q4K: return matmul_t<G_Q4K>(mp, tile, scratch, counters, s);
+        case G_Q5K: return matmul_t<G_Q5K>(mp, tile, scratch, counters, s);
+        case G_Q6K: return matmul_t<G_Q6K>(mp, tile, scratch, counters, s);
         default: return hipErrorInvalidValue;
     }
 }

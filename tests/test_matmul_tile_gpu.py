@@ -1,0 +1,84 @@
+"""bchip_matmul's kernels for large batches (k_matmul_tile) and for 32-weight formats whose
+cols is no multiple of 256 (k_matmul_units, k_matmul_tile) against the small batches of
+k_matmul_mm and each other: the same bits, since all run an output's operations in one order. Sizes sit at the
+edges of its tiles: 32 and 64 input rows, 128 weight rows, steps of 64 columns (odd groups
+too), K splits run in parallel and in turn, one unit and several a split."""
+import numpy as np
+import pytest
+
+import bchip
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+BLOCK32 = [O.F16, O.Q8_0, O.Q4_0, O.Q4_1, O.Q5_0, O.Q5_1]
+TILE_TYPES = BLOCK32 + [O.Q4K, O.Q5K, O.Q6K]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = bchip.Ctx(0)
+    yield c
+    c.close()
+
+
+def product(ctx, ty, data, rows, cols, x):
+    return products(ctx, ty, data, rows, cols, [x])[0]
+
+
+def products(ctx, ty, data, rows, cols, batches):
+    """The product of each batch of input rows, the weights uploaded once."""
+    wb, got = ctx.upload(data), []
+    for x in batches:
+        xb, ob = ctx.upload(np.ascontiguousarray(x, np.float32)), ctx.zeros(len(x) * rows * 4)
+        ctx.matmul(wb, ty, xb, ob, rows, cols, len(x))
+        got.append(ctx.read(ob, (len(x), rows)))
+        xb.free()
+        ob.free()
+    wb.free()
+    return got
+
+
+# rows x cols x n of at least 0.76 G (the tile kernel's threshold): 32 and 64 and 128 input rows a
+# workgroup; K splits in parallel and in turn; one unit, a few, remainders of every size.
+@pytest.mark.parametrize("ty", TILE_TYPES, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,n", [(11650, 4096, 17), (5801, 4096, 32), (301, 1280, 2000), (8300, 1536, 65),
+                                         (33000, 256, 100), (32900, 768, 129)])
+def test_tile_gives_the_small_batches_bits(ctx, ty, rows, cols, n):
+    # (a block of random rows repeated: random_tensor draws slowly)
+    some = 257
+    data = np.resize(np.asarray(O.random_tensor(ty, some, cols, rows + n), np.uint8).reshape(some, -1),
+                     (rows, O.row_bytes(ty, cols))).reshape(-1)
+    x = np.random.default_rng(cols + n).standard_normal((n, cols)).astype(np.float32)
+    at = [0, 15, n - 16] + ([n // 2] if n > 64 else [])  # batches of 16, 2 and 9 rows at the ends and inside
+    cuts = [(k, k + size) for k, size in zip(at, (16, 2, 16, 9))]
+    whole, *parts = products(ctx, ty, data, rows, cols, [x] + [x[a:b] for a, b in cuts])
+    assert np.isfinite(whole).all()
+    for (a, b), part in zip(cuts, parts):
+        np.testing.assert_array_equal(part, whole[a:b], err_msg=f"rows {a}..{b}")
+
+
+@pytest.mark.parametrize("ty", BLOCK32, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols", [(3, 32), (130, 96), (65, 896), (128, 864), (31, 2080), (17, 4384)])
+def test_cols_off_a_multiple_of_256(ctx, ty, rows, cols):
+    """One launch up to 16 input rows, the tile kernel beyond: a row's bits do not depend on
+    its batch, and its error against the f64 product stays below what its roundings can add
+    up to: x in two f16 parts (2^-22 of a term), f32 sums of a group's 32 products in some
+    order (32 x 2^-24 of their sizes), two roundings a group and unit after that."""
+    n = 70
+    data = O.random_tensor(ty, rows, cols, 5 * rows + n)
+    x = np.random.default_rng(cols).standard_normal((n, cols)).astype(np.float32)
+    x[1] *= 1e-6
+    x[2] *= 3e7
+    whole = product(ctx, ty, data, rows, cols, x)
+    for lo, hi in ((0, 2), (1, 4), (0, 8), (3, 19), (60, 70), (5, 38)):
+        np.testing.assert_array_equal(product(ctx, ty, data, rows, cols, x[lo:hi]), whole[lo:hi], err_msg=f"rows {lo}..{hi}")
+    w = O.dequant(ty, np.asarray(data, np.uint8).reshape(-1), rows, cols).astype(np.float64)
+    sizes = np.abs(x.astype(np.float64)) @ np.abs(w).T
+    # (SUM formats: |a q| and |b| of a weight can each exceed |a q + b|, at most 31-fold)
+    if ty in (O.Q4_1, O.Q5_1):
+        sizes = sizes.max(axis=1, keepdims=True) * 32
+    bound = (2.0 ** -22 + (32 + 4 + cols / 16) * 2.0 ** -24) * sizes
+    err = np.abs(whole - O.matmul_f64(ty, data, rows, cols, x, n))
+    print(f"{O.TYPE_NAMES[ty]} {rows}x{cols}: at most {np.max(err / bound):.3g} of the bound", flush=True)
+    assert (err <= bound).all()
