@@ -2,23 +2,29 @@
 // own f32 cache (crates/bc-infer/src/gpu/mod.rs:409-421) and want its results to f32
 // rounding, as the reference's end-to-end tests demand (model.rs:531, 548, 642: 1e-4).
 //
-// The reference per (row, head) (model.rs:448-481): scores dot(q, k) * scale with
-// quant::dot's eight lane sums (quant.rs:617-631), one softmax over the whole list, then
-// o += (p / sum) v in slot order. Here the scores are the same dot (eight lanes summed in
-// the same order, no fused multiply-add), times scale * log2(e); the softmax is online, over
-// blocks of F32_BLK list entries in exp2 units: per block and slot, the block's max, the new
-// running max, P = 2^(s - max), the block's sum of P and of P v (each in entry order), and
+// The reference per (row, head) (model.rs:448-481): scores dot(q, k) * scale, one softmax over
+// the whole list, then o += (p / sum) v in slot order. Here both contractions run on the f32
+// matrix cores (v_mfma_f32_16x16x4_f32: f32 operands, products and sums): a dot as eight chains of
+// hd / 8 products, added in pairs, times scale * log2(e); the softmax is online, over blocks of
+// F32_BLK list entries in exp2 units: per block and slot, the block's max, the new running
+// max, P = 2^(s - max), the block's sum of P and of P v (a chain over its entries), and
 // the running state scaled by 2^(old max - new max). Lists go in chunks of CHUNK_MULTI
 // entries, each an online softmax from a fresh state, folded left to right (merge_coef, the
 // fold every other kernel and attn_combine use). A row's bits therefore depend only on its q
 // and its list: the same in any batch, as a tree node or a line token, split over
 // workgroups or not, and a one-row pass gives the bits of the same row in a batch.
 //
-// A workgroup holds F32_SLOTS query slots of one KV head (rows x heads of the group; one row
-// for a tree), stages q and each block's K and V in LDS once for all of them, and walks its
-// list's chunks (all of them, folding as it goes, or one, its state then folded by
-// attn_combine when there are few workgroups). Bound: latency and LDS for the shapes this
-// path serves (the reference's tests, config 1's decode); f16 caches take the MFMA kernels.
+// A tile is 16 query slots of one KV head (rows x heads of the group; one row of a tree). S^T =
+// K Q^T leaves entry 4 (l / 16) + i of a 16-entry tile and slot l % 16 in lane l, register i,
+// which is the second product's operand (O^T = V^T P^T) as it stands: no move between lanes,
+// and a slot's max, sum and scale sit in the lanes that hold its outputs. The contractions' order
+// within a step of four is free (dims 16 j + 4 g + c, entries 4 g + i for lane group g = l / 16),
+// so that every operand is a 16-byte read.
+//
+// Two forms, the same bits. attn_f32_step: a workgroup per (tile, chunk), its waves each three
+// of the chunk's 16-entry score tiles and a quarter of the output dims; K and V go straight to
+// registers, a chunk's K all in flight at once. attn_f32_line: a workgroup of four
+// tiles walks the whole list, K and V blocks staged in LDS for all four.
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -28,8 +34,9 @@
 namespace bchip {
 
 constexpr int F32_BLK = 32;      // list entries per block
-constexpr int F32_SLOTS = 16;    // query slots a workgroup
+constexpr int F32_SLOTS = 16;    // query slots a tile
 constexpr int F32_THREADS = 256;
+constexpr int F32_WAVES = F32_THREADS / 64;
 
 struct F32Params {
     const float* q;
@@ -44,12 +51,12 @@ struct F32Params {
     uint32_t pos;     // line: slot of row 0; tree: the tree's first slot
     uint64_t slot_limit;  // slots the caches hold (tree slots past it read as zeros)
     float sc;         // scale * log2(e)
-    uint32_t rb, nrb; // rows a workgroup (1 for trees), row blocks
+    uint32_t rb, nrb; // rows a tile (1 for trees), tiles of a KV head
     uint32_t nchunk;  // chunks of the farthest list
-    uint32_t split;   // a workgroup per chunk
+    uint32_t split;   // attn_f32_step: more than one chunk, the states go to attn_combine
     const float* zero;  // ZERO_BYTES of zeros: the loads of rows past a list
     // A line call fused with RoPE and the K/V append of its rows at slots pos .. pos + rows - 1
-    // (attn_f32<HD, NR, MS>, NR > 0: at most NR rows): q is unrotated on entry and rotated as it
+    // (attn_f32_step<HD, NR>, NR > 0: at most NR rows): q is unrotated on entry and rotated as it
     // is staged; the new K rows (knew, rotated here) and V rows (vnew) go to the caches and
     // stand in for those slots' cache entries. q is left rotated: by the workgroup itself when
     // unsplit, else by the fold.
@@ -61,182 +68,188 @@ struct F32Params {
     float* qw;
 };
 
-// The dot's and P v's loops: two steps a trip at hd <= 64 (their LDS reads then go out
-// together; configs[0]'s step 24.9 -> 22.7 us a layer), one at hd 128 (there the same
-// measured slower, 76 -> 77-80 us: the registers cost more than the overlap gives).
-template <int HD>
-constexpr int F32_LU = HD <= 64 ? 2 : 1;
-
-// Rows a fused line call of several rows takes (their K and V rows sit in LDS: at 8 rows and
-// hd 128 three workgroups still fit a CU; 16 rows left two, and a verify pass's 704
-// workgroups then took two turns of the GPU, 73 -> 96 us a layer-step).
+// Rows a fused line call of several rows takes.
 constexpr uint32_t F32_FUSE_ROWS = 8;
 
-template <int HD, int NR, bool MS>
-__global__ __launch_bounds__(F32_THREADS) void attn_f32(const F32Params p) {
+// Lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and D[4 (l / 16) + i][l % 16].
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The max of a slot's four lanes (l, l ^ 16, l ^ 32, l ^ 48), to each of them; their sum.
+__device__ __forceinline__ float slot_max(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float slot_sum(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// A score tile from its eight chains: entries first .. first + 3 of the list in a lane; -inf at
+// or past the slot's list.
+__device__ __forceinline__ f32x4 score_tile(const f32x4 (&a)[8], float sc, uint32_t first, uint32_t len) {
+    f32x4 s;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float d = ((a[0][i] + a[1][i]) + (a[2][i] + a[3][i])) + ((a[4][i] + a[5][i]) + (a[6][i] + a[7][i]));
+        s[i] = first + i < len ? d * sc : -INFINITY;
+    }
+    return s;
+}
+
+// A slot's running max and this lane's share of its sum, taken over a block: s becomes P; returns
+// the scale of what came before.
+__device__ __forceinline__ float softmax_block(f32x4 (&s)[2], float& m, float& l) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; t++) mx = fmaxf(mx, fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3])));
+    const float mn = fmaxf(m, slot_max(mx)), ms = (mn == -INFINITY) ? 0.0f : mn;
+    const float cr = exp2_hw(m - ms);
+    float bl[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) s[t][i] = exp2_hw(s[t][i] - ms);
+        bl[t] = (s[t][0] + s[t][1]) + (s[t][2] + s[t][3]);
+    }
+    l = l * cr + (bl[0] + bl[1]);
+    m = mn;
+    return cr;
+}
+
+typedef __amdgpu_buffer_rsrc_t f32_rsrc;
+
+template <int N>
+struct VecN {
+    typedef float T __attribute__((ext_vector_type(N)));
+};
+template <>
+struct VecN<1> {
+    typedef float T;
+};
+__device__ __forceinline__ float vec_at(float v, int) { return v; }
+template <typename V>
+__device__ __forceinline__ float vec_at(V v, int i) {
+    return v[i];
+}
+
+// Bound: HBM for long lists (llama-8B heads, 32768 slots: 268 MB in 59 us a layer, 67 with VALU
+// dots; 6001 slots 14.5 against 19), else the fixed time of a launch. K goes out first and V as
+// K's registers free up, a third after each score tile: with V's loads queued beside K's the
+// first scores came later and the products after them were not hidden (12000 slots: 8 layers
+// 255 us, so 237). Steps and verify rows run best two workgroups a CU with these registers;
+// trees and short prompts, whose rows read one prefix from cache, three (33 rows at 3001: 265
+// us, 236).
+template <int HD, int NR>
+__global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void attn_f32_step(const F32Params p) {
     constexpr bool FUSE = NR > 0;
-    // q and K rows in LDS in lane order: element d = j + 8i at j * NI + i, so that the
-    // elements of quant::dot's lane j (d = j, j + 8, ...) are contiguous and read 16 bytes at a
-    // time. Rows are KS floats apart, 4 more than a multiple of 32 banks, so that the eight
-    // lanes LDS serves together (eight entries, one offset) hit eight groups of banks.
-    constexpr int NI = HD / 8;     // elements of one dot lane
-    constexpr int KS = HD + 4;     // LDS row of q or K
-    static_assert(NI % 4 == 0, "a lane's run is whole 16-byte reads");
-    constexpr int NL = F32_BLK * (HD / 4) / F32_THREADS;  // 16-byte pieces of K (and of V) a thread loads a block
-    static_assert(NL >= 1 && F32_BLK * (HD / 4) % F32_THREADS == 0, "a block's rows divide over the threads");
-    // Each wave takes slots wave, wave + W, ...: their scores, softmax and P v within the wave.
-    constexpr int W = F32_THREADS / 64;            // waves
-    constexpr int SPW = F32_SLOTS / W;             // slots a wave at most
-    constexpr int DPL = HD >= 64 ? HD / 64 : 1;    // dims a lane holds in P v
-    constexpr int DL = HD / DPL;                   // lanes holding dims
-    static_assert(F32_BLK == 32, "a block's entries are the wave's lanes 0..31");
-    __shared__ __attribute__((aligned(16))) float qs[F32_SLOTS][KS];
-    __shared__ __attribute__((aligned(16))) float ks[F32_BLK][KS];
-    __shared__ __attribute__((aligned(16))) float vs[F32_BLK][HD];
+    constexpr int NJ = HD / 16;                      // 16-byte reads of a K row a lane
+    constexpr int QS = HD + 4;                       // LDS row of q
+    constexpr int NT = CHUNK_MULTI / 16;             // score tiles of a chunk
+    constexpr int TPW = NT / F32_WAVES;              // of a wave
+    constexpr int VW = HD >= 64 ? HD / F32_WAVES : 16;  // output dims of a wave (hd 32: of two waves)
+    constexpr int VC = VW / 16;                      // tiles of them: dim VW w + VC m + c is row m of tile c
+    static_assert(NT % F32_WAVES == 0 && F32_BLK == 32, "");
+    typedef typename VecN<VC>::T vvec;
+    __shared__ __attribute__((aligned(16))) float qs[F32_SLOTS][QS];
+    __shared__ __attribute__((aligned(16))) f32x4 ss[NT][64];
     __shared__ uint32_t tail[MAX_ITEMS];
-    // hd >= 128: each wave's P of a block (its slots of a pass), read back 16 bytes at a time for
-    // the block sum and P v (eight reads a block where readlane took 32 VALU instructions:
-    // configs[1] over f32 77.7 -> 75.5 us a call, its verify loop 70.8 -> 66.4 us a
-    // layer-step; at hd 64 readlane measured slightly faster).
-    constexpr bool PL = HD >= 128;
-    constexpr int PS = MS ? F32_SLOTS / (F32_THREADS / 64) : 1;  // slots of a pass at most (one without MS)
-    __shared__ __attribute__((aligned(16))) float pw[PL ? F32_THREADS / 64 : 1][PL ? PS : 1][PL ? F32_BLK : 4];
     // FUSE: the new K rows (rotated) and V rows as the caches hold them.
     __shared__ __attribute__((aligned(16))) float nrow[FUSE ? 2 : 1][FUSE ? NR : 1][FUSE ? HD : 4];
 
-    const uint32_t tid = threadIdx.x;
-    const uint32_t gi = p.split ? blockIdx.x / p.nchunk : blockIdx.x;
-    const uint32_t c_one = p.split ? blockIdx.x % p.nchunk : 0u;
-    const uint32_t kvh = gi % p.nkv;
-    const uint32_t rbi = p.nrb - 1u - gi / p.nkv;  // latest rows (longest lists) first
-    const uint32_t grp = kvh * p.nrb + rbi;        // canonical group of the chunk states
-    const uint32_t r0 = rbi * p.rb;
-    const uint32_t hd = p.hd, kvd = p.nkv * hd;
-    const float* kcb = p.kc + (size_t)kvh * hd;
-    const float* vcb = p.vc + (size_t)kvh * hd;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t n = lane & 15u, g = lane >> 4;    // n: an entry, a slot or a dim's place
+    // The tiles of a chunk of a KV head side by side in launch order, so that they find its K and V
+    // in cache.
+    const uint32_t kvh = blockIdx.x % p.nkv, b0 = blockIdx.x / p.nkv;
+    const uint32_t rbi = b0 % p.nrb, c = b0 / p.nrb;
+    const uint32_t grp = kvh * p.nrb + rbi;          // canonical group of the chunk states
+    const uint32_t r0 = rbi * p.rb, hd = p.hd, kvd = p.nkv * hd;
 
-    // A tree's workgroup is one row: its list is the slots below pos, then pos + j for each
-    // set bit j of its mask, in order (kernels.h:266-278).
+    // A tree's tile is one row: its list is the slots below pos, then pos + j for each set bit j
+    // of its mask, in order (kernels.h:266-278).
     uint32_t ntail = 0;
     if (p.tree) {
         const uint32_t lo = p.masks[2 * r0], hi = p.masks[2 * r0 + 1];
         ntail = __popc(lo) + __popc(hi);
         if (tid < ntail) tail[tid] = p.pos + nth_set_bit(lo, hi, tid);
+        __syncthreads();
     }
     // Slot n: head kvh * G + n / rb of row r0 + n % rb.
-    auto slot_valid = [&](uint32_t n) { return n / p.rb < p.G && r0 + n % p.rb < p.rows; };
-    auto slot_len = [&](uint32_t n) -> uint32_t {
-        if (!slot_valid(n)) return 0u;
-        return p.tree ? p.pos + ntail : p.pos + r0 + n % p.rb + 1u;
-    };
+    auto slot_valid = [&](uint32_t k) { return k / p.rb < p.G && r0 + k % p.rb < p.rows; };
     const uint32_t rlast = min(r0 + p.rb, p.rows) - 1u;
     const uint32_t maxlen = p.tree ? p.pos + ntail : p.pos + rlast + 1u;
-    // Slots at or past G * rb hold no query (a one-row step at G = 4 fills 4 of 16): the P v
-    // products, the folds and the stores skip them, whole iterations at a time (uniform).
-    const uint32_t used_e = min((uint32_t)F32_SLOTS, p.G * p.rb) * HD;
+    const uint32_t len = !slot_valid(n) ? 0u : p.tree ? maxlen : p.pos + r0 + n % p.rb + 1u;
+    const uint32_t kb0 = c * CHUNK_MULTI, kb1 = min(kb0 + CHUNK_MULTI, maxlen);
 
-
-    const uint32_t lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // Slot wave + W s's running state: m, l, and the folded RM, RL (wave-uniform), and its
-    // dims lane * DPL .. + DPL - 1 of o and R.
-    float m[SPW], l[SPW], RM[SPW], RL[SPW], o[SPW][DPL], R[SPW][DPL];
+    // K and V through buffer descriptors from the chunk's first slot on: entries past the list and
+    // dims past hd are sent past the end, as slots past the cache are, and read as 0. (A list's
+    // slots lie at most MAX_ITEMS past its entries' numbers.)
+    const uint64_t slots = p.slot_limit > kb0 ? min(p.slot_limit - kb0, (uint64_t)(CHUNK_MULTI + MAX_ITEMS)) : 0;
+    const size_t at = ((size_t)kb0 * p.nkv + kvh) * hd;
+    const int bytes = slots ? (int)((slots * kvd - (size_t)kvh * hd) * 4) : 0;
+    const f32_rsrc kr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.kc + at), 0, bytes, 0x00020000);
+    const f32_rsrc vr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.vc + at), 0, bytes, 0x00020000);
+    constexpr uint32_t NONE = 0x80000000u;
+    auto row_at = [&](uint32_t e) -> uint32_t {  // bytes from the chunk's first slot to entry e
+        const uint32_t kk = kb0 + e;
+        uint32_t s = e;
+        if (p.tree && kk >= p.pos) s = tail[min(kk - p.pos, (uint32_t)MAX_ITEMS - 1u)] - kb0;
+        return kk < kb1 ? s * kvd * 4u : NONE;
+    };
+    f32x4 kx[TPW][NJ];
 #pragma unroll
-    for (int s = 0; s < SPW; s++) {
-        m[s] = RM[s] = -INFINITY;
-        l[s] = RL[s] = 0.0f;
+    for (int t = 0; t < TPW; t++) {
+        const uint32_t ro = row_at(16u * (wave + F32_WAVES * t) + n) + 16u * g;
 #pragma unroll
-        for (int dd = 0; dd < DPL; dd++) o[s][dd] = R[s][dd] = 0.0f;
+        for (int j = 0; j < NJ; j++) {
+            const uint32_t o = (hd == (uint32_t)HD || 16u * j + 4u * g < hd) ? ro + 64u * j : NONE;
+            kx[t][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(kr, o, 0, 0));
+        }
     }
-    const uint32_t dl = lane % DL;  // this lane's dims in P v: dl * DPL .. (lanes past DL repeat them)
-
-    // This thread's share of a block's K and V rows (NL 16-byte pieces of each), loaded one
-    // block ahead: the next block's loads are in flight while this block computes. Entries
-    // past the chunk or the cache, and dims past hd, load the zero page.
-    f32x4 kr[NL], vr[NL];
-    auto fetch = [&](uint32_t key0, uint32_t kb1) {
+    const uint32_t vd = VW * wave + VC * n;
+    vvec vx[NT][4];
+    auto load_v = [&](int t) {
 #pragma unroll
-        for (int i = 0; i < NL; i++) {
-            const uint32_t e = tid + F32_THREADS * i, k = e / (HD / 4), d = 4 * (e % (HD / 4)), kk = key0 + k;
-            const uint32_t s = (p.tree && kk >= p.pos) ? tail[min(kk - p.pos, (uint32_t)MAX_ITEMS - 1u)] : kk;
-            const bool ok = kk < kb1 && d < hd && (uint64_t)s < p.slot_limit;
-            // One load each from a selected address (the asm keeps the compiler from
-            // splitting it into a load on each side of a branch, each followed by a wait).
-            uintptr_t ka = ok ? (uintptr_t)(kcb + (size_t)s * kvd + d) : (uintptr_t)p.zero;
-            uintptr_t va = ok ? (uintptr_t)(vcb + (size_t)s * kvd + d) : (uintptr_t)p.zero;
-            asm("" : "+v"(ka), "+v"(va));
-            typedef __attribute__((address_space(1))) const f32x4 gf4;
-            kr[i] = *(gf4*)ka;
-            vr[i] = *(gf4*)va;
+        for (int i = 0; i < 4; i++) {
+            const uint32_t ro = row_at(16u * t + 4u * g + i), o = vd < hd ? ro + 4u * vd : NONE;
+            if constexpr (VC == 1)
+                vx[t][i] = __builtin_bit_cast(vvec, __builtin_amdgcn_raw_buffer_load_b32(vr, o, 0, 0));
+            else if constexpr (VC == 2)
+                vx[t][i] = __builtin_bit_cast(vvec, __builtin_amdgcn_raw_buffer_load_b64(vr, o, 0, 0));
+            else
+                vx[t][i] = __builtin_bit_cast(vvec, __builtin_amdgcn_raw_buffer_load_b128(vr, o, 0, 0));
         }
     };
-    auto stash = [&](uint32_t key0) {
-#pragma unroll
-        for (int i = 0; i < NL; i++) {
-            const uint32_t e = tid + F32_THREADS * i, k = e / (HD / 4), d = 4 * (e % (HD / 4));
-            f32x4 kx = kr[i], vx = vr[i];
-            if constexpr (FUSE) {
-                // A new row's slot: its K and V as this kernel wrote them to the caches.
-                const uint32_t j = key0 + k - p.pos;
-                if (key0 + k >= p.pos && j < p.rows) {
-                    kx = *(const f32x4*)&nrow[0][j][d];
-                    vx = *(const f32x4*)&nrow[1][j][d];
-                }
-            }
-            float* kd = &ks[k][(d % 8) * NI + d / 8];  // d % 8 is 0 or 4: elements d .. d + 3 are lanes' runs apart
-            kd[0] = kx[0];
-            kd[NI] = kx[1];
-            kd[2 * NI] = kx[2];
-            kd[3 * NI] = kx[3];
-            *(f32x4*)&vs[k][d] = vx;
-        }
-    };
-    const uint32_t nused = used_e / HD;  // slots that may hold a query
-    // Cross-lane moves: the value 32 lanes up; the max over 16- and 32-lane groups.
-    auto up32 = [](float x) {
-        return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);
-    };
-    auto wave_max = [](float x) {
-        x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false)));  // row_ror:8
-        x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false)));  // row_ror:4
-        x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false)));  // row_ror:2
-        x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false)));  // row_ror:1
-        const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-        x = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
-        const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-        return fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
-    };
-
-    // The first block's loads go out before q is staged, so that the two latencies overlap
-    // (a tree's loads name slots from tail: every thread's entries of it are in first). Each
-    // chunk's last block loads the next chunk's first (chunks past the list are empty, and
-    // only they).
-    if (p.tree) __syncthreads();
-    const uint32_t cend = p.split ? c_one + 1u : max(1u, (maxlen + CHUNK_MULTI - 1u) / CHUNK_MULTI);
-    if (c_one * CHUNK_MULTI < maxlen) fetch(c_one * CHUNK_MULTI, min(c_one * CHUNK_MULTI + CHUNK_MULTI, maxlen));
+    const bool has_new = FUSE && kb1 > p.pos && kb0 < p.pos + p.rows;  // a new row's slot is in this chunk
     if constexpr (FUSE) {
         // Row j's new slot is pos + j, its angles from positions[j]; pair pp of a head is (a, b)
         // by rope_pair, rotated when pp < rope_dim / 2 by k_rope_append's expressions (the
         // same bits).
-        const size_t kvd_s = kvd;
-        const uint32_t lo = max(c_one * CHUNK_MULTI, p.pos), hi = min(cend * CHUNK_MULTI, p.pos + p.rows);
+        const uint32_t lo = max(kb0, p.pos), hi = min(kb0 + CHUNK_MULTI, p.pos + p.rows);
         if (lo < hi) {
-            // This workgroup streams new slots lo .. hi - 1: their K rows rotated and V rows,
-            // into the caches and nrow (row blocks of the same chunk write the same values).
+            // This workgroup reads new slots lo .. hi - 1: their K rows rotated and V rows, into
+            // the caches and nrow (tiles of the same chunk write the same values).
             for (uint32_t e = tid; e < (hi - lo) * (HD / 2); e += F32_THREADS) {
                 const uint32_t j = lo - p.pos + e / (HD / 2), pp = e % (HD / 2);
                 uint32_t a, b;
                 const bool rot = rope_pair(pp, p.rope_dim, p.neox, a, b);
                 float k0 = 0.0f, k1 = 0.0f, v0 = 0.0f, v1 = 0.0f;
                 if (pp < hd / 2) {
-                    const float* kx = p.knew + ((size_t)j * p.nkv + kvh) * hd;
-                    const float* vx = p.vnew + ((size_t)j * p.nkv + kvh) * hd;
-                    k0 = kx[a];
-                    k1 = kx[b];
-                    if (rot) rotate(kx[a], kx[b], (float)p.positions[j] * p.inv_freq[pp], k0, k1);
-                    v0 = vx[2 * pp];
-                    v1 = vx[2 * pp + 1];
-                    float* kdst = (float*)p.kc + (size_t)(p.pos + j) * kvd_s + (size_t)kvh * hd;
-                    float* vdst = (float*)p.vc + (size_t)(p.pos + j) * kvd_s + (size_t)kvh * hd;
+                    const float* kn = p.knew + ((size_t)j * p.nkv + kvh) * hd;
+                    const float* vn = p.vnew + ((size_t)j * p.nkv + kvh) * hd;
+                    k0 = kn[a];
+                    k1 = kn[b];
+                    if (rot) rotate(kn[a], kn[b], (float)p.positions[j] * p.inv_freq[pp], k0, k1);
+                    v0 = vn[2 * pp];
+                    v1 = vn[2 * pp + 1];
+                    float* kdst = (float*)p.kc + (size_t)(p.pos + j) * kvd + (size_t)kvh * hd;
+                    float* vdst = (float*)p.vc + (size_t)(p.pos + j) * kvd + (size_t)kvh * hd;
                     kdst[a] = k0;
                     kdst[b] = k1;
                     vdst[2 * pp] = v0;
@@ -250,283 +263,312 @@ __global__ __launch_bounds__(F32_THREADS) void attn_f32(const F32Params p) {
         }
         // q rotated as it is staged, a pair a thread (dims past hd and empty slots: zeros).
         for (uint32_t e = tid; e < F32_SLOTS * (HD / 2); e += F32_THREADS) {
-            const uint32_t n = e / (HD / 2), pp = e % (HD / 2);
+            const uint32_t k = e / (HD / 2), pp = e % (HD / 2);
             uint32_t a, b;
             const bool rot = rope_pair(pp, p.rope_dim, p.neox, a, b);
             float y0 = 0.0f, y1 = 0.0f;
-            if (pp < hd / 2 && slot_valid(n)) {
-                const uint32_t r = r0 + n % p.rb, h = kvh * p.G + n / p.rb;
+            if (pp < hd / 2 && slot_valid(k)) {
+                const uint32_t r = r0 + k % p.rb, h = kvh * p.G + k / p.rb;
                 const float* qh = p.q + ((size_t)r * p.nh + h) * hd;
                 y0 = qh[a];
                 y1 = qh[b];
                 if (rot) rotate(qh[a], qh[b], (float)p.positions[r] * p.inv_freq[pp], y0, y1);
             }
-            qs[n][(a % 8) * NI + a / 8] = y0;
-            qs[n][(b % 8) * NI + b / 8] = y1;
+            qs[k][a] = y0;
+            qs[k][b] = y1;
         }
+    } else {
+        for (uint32_t e = tid; e < F32_SLOTS * (HD / 4); e += F32_THREADS) {
+            const uint32_t k = e / (HD / 4), d = 4 * (e % (HD / 4));
+            f32x4 v = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (d < hd && slot_valid(k)) {
+                const uint32_t r = r0 + k % p.rb, h = kvh * p.G + k / p.rb;
+                v = *(const f32x4*)&p.q[((size_t)r * p.nh + h) * hd + d];
+            }
+            *(f32x4*)&qs[k][d] = v;
+        }
+    }
+    // The fences order LDS only: __syncthreads' would also wait for the K and V loads.
+    auto lds_barrier = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    lds_barrier();
+    if constexpr (FUSE) {
         if (!p.split) {
             // q stays rotated, as k_rope_append leaves it: this workgroup is the only reader of
             // its heads, and every read of them is done at the barrier. (A split launch's fold
             // writes them once every chunk's workgroup has read them.)
-            __syncthreads();
             for (uint32_t e = tid; e < F32_SLOTS * HD; e += F32_THREADS) {
-                const uint32_t n = e / HD, d = e % HD;
-                if (d < hd && slot_valid(n)) {
-                    const uint32_t r = r0 + n % p.rb, h = kvh * p.G + n / p.rb;
-                    p.qw[((size_t)r * p.nh + h) * hd + d] = qs[n][(d % 8) * NI + d / 8];
+                const uint32_t k = e / HD, d = e % HD;
+                if (d < hd && slot_valid(k)) {
+                    const uint32_t r = r0 + k % p.rb, h = kvh * p.G + k / p.rb;
+                    p.qw[((size_t)r * p.nh + h) * hd + d] = qs[k][d];
                 }
             }
-        }
-    } else {
-        for (uint32_t e = tid; e < F32_SLOTS * HD; e += F32_THREADS) {
-            const uint32_t n = e / HD, d = e % HD;
-            float v = 0.0f;
-            if (d < hd && slot_valid(n)) {
-                const uint32_t r = r0 + n % p.rb, h = kvh * p.G + n / p.rb;
-                v = p.q[((size_t)r * p.nh + h) * hd + d];
-            }
-            qs[n][(d % 8) * NI + d / 8] = v;
         }
     }
-    for (uint32_t c = c_one; c < cend; c++) {
-        const uint32_t kb0 = c * CHUNK_MULTI, kb1 = min(kb0 + CHUNK_MULTI, maxlen);
-        for (uint32_t key0 = kb0; key0 < kb1; key0 += F32_BLK) {
-            __syncthreads();  // the previous block's K, V and P are consumed (and q is in)
-            stash(key0);
-            if (key0 + F32_BLK < kb1) {
-                fetch(key0 + F32_BLK, kb1);
-            } else if (c + 1 < cend && kb1 < maxlen) {
-                const uint32_t nb0 = (c + 1) * CHUNK_MULTI;
-                fetch(nb0, min(nb0 + CHUNK_MULTI, maxlen));
-            }
-            // K and V in for everyone. The fences order LDS only: __syncthreads' would also
-            // wait for the next block's loads just issued.
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-            // Per slot of this wave: scores, softmax and P v. Lane k < 32 and lane k + 32 take
-            // entry k: each sums quant::dot's lanes 4h .. 4h + 3 (h its half) over their
-            // elements in order, and lane k adds the eight to 0 in lane order (the upper four
-            // from lane k + 32), times sc; -inf at or past the slot's list. The block's max
-            // across the wave; P of entry k in lane k; the block sum and P v entry by entry
-            // in order, P taken from its lane.
-            const uint32_t k = lane & 31u, h = lane >> 5;
-            // Slots s0 .. s0 + NS - 1 of the wave together: each slot's operations as alone,
-            // in the same order; K's and V's LDS reads serve all of them.
-            auto pass = [&](auto S0, auto NSc) {
-                constexpr int s0 = decltype(S0)::value, NS = decltype(NSc)::value;
-                static_assert(s0 + NS <= SPW && (!PL || NS <= PS), "a pass's slots are the wave's, its P rows in pw");
-                uint32_t nn[NS];
-                float a[NS][4];
+    f32x4 qx[NJ];
 #pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    nn[s] = wave + W * (s0 + s);
+    for (int j = 0; j < NJ; j++) qx[j] = *(const f32x4*)&qs[n][16 * j + 4 * g];
+
+    const uint32_t nblk = kb0 < kb1 ? (kb1 - kb0 + F32_BLK - 1) / F32_BLK : 0u;
 #pragma unroll
-                    for (int jj = 0; jj < 4; jj++) a[s][jj] = 0.0f;
-                }
-                // d = j + 8 (i + t) in order; past hd (a head dim below HD) no term.
-                auto dot_lanes = [&](auto FULL) {
-#pragma unroll F32_LU<HD>
-                    for (uint32_t i = 0; i < (uint32_t)NI; i += 4) {
+    for (int t = 0; t < TPW; t++) {
+        const uint32_t tile = wave + F32_WAVES * t, e = kb0 + 16 * tile + n;
+        if constexpr (FUSE) {
+            // A new row's slot: its K as this kernel wrote it to the cache.
+            if (has_new && e >= p.pos && e < p.pos + p.rows) {
 #pragma unroll
-                        for (uint32_t jj = 0; jj < 4; jj++) {
-                            const uint32_t j = 4 * h + jj;
-                            const f32x4 kv = *(const f32x4*)&ks[k][j * NI + i];
-#pragma unroll
-                            for (int s = 0; s < NS; s++) {
-                                const f32x4 qv = *(const f32x4*)&qs[nn[s]][j * NI + i];
-#pragma unroll
-                                for (uint32_t t = 0; t < 4; t++)
-                                    if (decltype(FULL)::value || 8 * (i + t) < hd) a[s][jj] += qv[t] * kv[t];
-                            }
-                        }
-                    }
-                };
-                if (hd == (uint32_t)HD)
-                    dot_lanes(std::true_type{});
-                else
-                    dot_lanes(std::false_type{});
-                float pe[NS], mn[NS], cr[NS];
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    float dsum = 0.0f + a[s][0];
-                    dsum += a[s][1];
-                    dsum += a[s][2];
-                    dsum += a[s][3];
-#pragma unroll
-                    for (int jj = 0; jj < 4; jj++) dsum += up32(a[s][jj]);
-                    const float sc = (lane < 32u && key0 + k < slot_len(nn[s])) ? dsum * p.sc : -INFINITY;
-                    const float mx = wave_max(sc);
-                    mn[s] = fmaxf(m[s0 + s], mx);
-                    const float ms = (mn[s] == -INFINITY) ? 0.0f : mn[s];
-                    cr[s] = exp2_hw(m[s0 + s] - ms);
-                    pe[s] = exp2_hw(sc - ms);
-                }
-                float bl[NS], acc[NS][DPL];
-                if constexpr (PL) {
-#pragma unroll
-                    for (int s = 0; s < NS; s++)
-                        if (lane < 32u) pw[wave][s][lane] = pe[s];
-                }
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    bl[s] = 0.0f;
-#pragma unroll
-                    for (int dd = 0; dd < DPL; dd++) acc[s][dd] = 0.0f;
-                }
-#pragma unroll F32_LU<HD>
-                for (int k8 = 0; k8 < F32_BLK; k8 += 8) {
-                    f32x4 pq[NS][2];
-                    if constexpr (PL) {
-#pragma unroll
-                        for (int s = 0; s < NS; s++) {
-                            pq[s][0] = *(const f32x4*)&pw[wave][s][k8];
-                            pq[s][1] = *(const f32x4*)&pw[wave][s][k8 + 4];
-                        }
-                    }
-#pragma unroll
-                    for (int kj = 0; kj < 8; kj++) {
-                        const int kk = k8 + kj;
-                        float v[DPL];
-                        if constexpr (DPL == 1) {
-                            v[0] = vs[kk][dl];
-                        } else if constexpr (DPL == 2) {
-                            const float2 v2 = *(const float2*)&vs[kk][2 * dl];
-                            v[0] = v2.x;
-                            v[1] = v2.y;
-                        } else {
-                            const f32x4 v4 = *(const f32x4*)&vs[kk][4 * dl];
-#pragma unroll
-                            for (int dd = 0; dd < 4; dd++) v[dd] = v4[dd];
-                        }
-#pragma unroll
-                        for (int s = 0; s < NS; s++) {
-                            const float pk = PL ? pq[s][kj / 4][kj % 4]
-                                                : __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pe[s]), kk));
-                            bl[s] += pk;
-#pragma unroll
-                            for (int dd = 0; dd < DPL; dd++) acc[s][dd] += pk * v[dd];
-                        }
-                    }
-                }
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    l[s0 + s] = l[s0 + s] * cr[s] + bl[s];
-                    m[s0 + s] = mn[s];
-#pragma unroll
-                    for (int dd = 0; dd < DPL; dd++) o[s0 + s][dd] = o[s0 + s][dd] * cr[s] + acc[s][dd];
-                }
-            };
-            using i0 = std::integral_constant<int, 0>;
-            using i1 = std::integral_constant<int, 1>;
-            using i2 = std::integral_constant<int, 2>;
-            using i3 = std::integral_constant<int, 3>;
-            static_assert(SPW == 4, "four slots a wave at most");
-            // The wave's slots that may hold a query: wave, wave + W, ... below nused.
-            const uint32_t nact = wave < nused ? min((uint32_t)SPW, (nused - wave + W - 1) / W) : 0u;
-            if constexpr (MS && HD > 64) {
-                // A launch whose waves hold several slots (MS: more than four in a workgroup):
-                // four a pass where a wave has four, else two.
-                if (nact == 4) {
-                    pass(i0{}, std::integral_constant<int, 4>{});
-                } else {
-                    if (nact >= 2)
-                        pass(i0{}, i2{});
-                    else if (nact == 1)
-                        pass(i0{}, i1{});
-                    if (nact == 3) pass(i2{}, i1{});
-                }
-            } else if constexpr (HD <= 64) {
-                // Two slots a pass: the shared reads and the two slots' chains side by side
-                // (configs[0], seven slots over four waves: 22.7 -> 21.9 us a layer-step).
-                if (nact >= 2)
-                    pass(i0{}, i2{});
-                else if (nact == 1)
-                    pass(i0{}, i1{});
-                if (nact >= 4)
-                    pass(i2{}, i2{});
-                else if (nact == 3)
-                    pass(i2{}, i1{});
-            } else {
-                if (nact >= 1) pass(i0{}, i1{});
-                if (nact >= 2) pass(i1{}, i1{});
-                if (nact >= 3) pass(i2{}, i1{});
-                if (nact >= 4) pass(i3{}, i1{});
+                for (int j = 0; j < NJ; j++) kx[t][j] = *(const f32x4*)&nrow[0][e - p.pos][16 * j + 4 * g];
             }
         }
-        if (p.split) break;
-        // The chunk's state folded into the running one (merge_coef, R = R a + c b).
+        if (tile / 2 < nblk) {
+            f32x4 a[8] = {};
 #pragma unroll
-        for (int sw = 0; sw < SPW; sw++) {
-            float fa, fb, mn;
-            merge_coef(RM[sw], m[sw], fa, fb, mn);
-            RL[sw] = RL[sw] * fa + l[sw] * fb;
-            RM[sw] = mn;
+            for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int dd = 0; dd < DPL; dd++) {
-                R[sw][dd] = R[sw][dd] * fa + o[sw][dd] * fb;
-                o[sw][dd] = 0.0f;
-            }
-            m[sw] = -INFINITY;
-            l[sw] = 0.0f;
+                for (int k = 0; k < 4; k++) a[4 * (j % 2) + k] = mfma4(kx[t][j][k], qx[j][k], a[4 * (j % 2) + k]);
+            ss[tile][lane] = score_tile(a, p.sc, kb0 + 16 * tile + 4 * g, len);
         }
+#pragma unroll
+        for (int v = 0; v < NT / TPW; v++) load_v(NT / TPW * t + v);
     }
+    lds_barrier();
+
+    float m = -INFINITY, l = 0.0f;
+    f32x4 o[VC];
+#pragma unroll
+    for (int k = 0; k < VC; k++) o[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int b = 0; b < NT / 2; b++) {
+        if ((uint32_t)b >= nblk) break;
+        f32x4 s[2] = {ss[2 * b][lane], ss[2 * b + 1][lane]};
+        const float cr = softmax_block(s, m, l);
+        f32x4 acc[VC] = {};
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                vvec v = vx[2 * b + t][i];
+                if constexpr (FUSE) {
+                    const uint32_t e = kb0 + 16 * (2 * b + t) + 4 * g + i;
+                    if (has_new && e >= p.pos && e < p.pos + p.rows && vd < (uint32_t)HD)
+                        v = *(const vvec*)&nrow[1][e - p.pos][vd];
+                }
+#pragma unroll
+                for (int k = 0; k < VC; k++) acc[k] = mfma4(vec_at(v, k), s[t][i], acc[k]);
+            }
+#pragma unroll
+        for (int k = 0; k < VC; k++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[k][i] = __builtin_fmaf(o[k][i], cr, acc[k][i]);
+    }
+    l = slot_sum(l);
+    // Lane (n, g): dims vb .. vb + 4 VC - 1 of slot n, dim vb + VC i + k in o[k][i].
+    const uint32_t vb = VW * wave + 4 * VC * g;
     if (p.split) {
-        const size_t u = (size_t)grp * p.nchunk + c_one;
+        const size_t u = (size_t)grp * p.nchunk + c;
+        if (n >= min((uint32_t)F32_SLOTS, p.G * p.rb)) return;  // attn_combine reads no slot past them
+        if (vb < (uint32_t)HD) {
+            float* dst = p.part_o + (u * F32_SLOTS + n) * HD + vb;
 #pragma unroll
-        for (int sw = 0; sw < SPW; sw++) {
-            const uint32_t n = wave + W * sw;
-            if (n >= nused) break;  // attn_combine reads no slot past them
-            if (lane < (uint32_t)DL) {
+            for (int q4 = 0; q4 < VC; q4++) {
+                f32x4 v;
 #pragma unroll
-                for (int dd = 0; dd < DPL; dd++) p.part_o[(u * F32_SLOTS + n) * HD + DPL * dl + dd] = o[sw][dd];
+                for (int x = 0; x < 4; x++) v[x] = o[(4 * q4 + x) % VC][(4 * q4 + x) / VC];
+                *(f32x4*)(dst + 4 * q4) = v;
             }
-            if (lane == 0) *(float2*)(p.part_ml + (u * F32_SLOTS + n) * 2) = float2{m[sw], l[sw]};
         }
+        if (wave == 0 && g == 0) *(float2*)(p.part_ml + (u * F32_SLOTS + n) * 2) = float2{m, l};
         return;
     }
+    if (!slot_valid(n)) return;
+    float* dst = p.out + ((size_t)(r0 + n % p.rb) * p.nh + kvh * p.G + n / p.rb) * hd + vb;
 #pragma unroll
-    for (int sw = 0; sw < SPW; sw++) {
-        const uint32_t n = wave + W * sw;
-        if (n >= nused) break;
-        if (!slot_valid(n) || lane >= (uint32_t)DL) continue;
-        const uint32_t r = r0 + n % p.rb, hh = kvh * p.G + n / p.rb;
+    for (int q4 = 0; q4 < VC; q4++)
+        if (vb + 4 * q4 < hd) {
+            f32x4 v;
 #pragma unroll
-        for (int dd = 0; dd < DPL; dd++) {
-            const uint32_t d = DPL * dl + dd;
-            if (d < hd) p.out[((size_t)r * p.nh + hh) * hd + d] = R[sw][dd] / RL[sw];
+            for (int x = 0; x < 4; x++) v[x] = o[(4 * q4 + x) % VC][(4 * q4 + x) / VC] / l;
+            *(f32x4*)(dst + 4 * q4) = v;
         }
+}
+
+// A block of K or V in LDS, 16-byte units: K's unit u of entry e at u ^ (e % 8), so that the eight
+// entries LDS serves together are in eight groups of banks; V's in order.
+template <int HD>
+struct F32Stage {
+    f32x4 k[F32_BLK][HD / 4];
+    f32x4 v[F32_BLK][HD / 4];
+};
+
+// Bound: the matrix cores (777 rows at 300, llama-8B heads: 8.8 GFLOP in 127 us, 361 with VALU
+// dots; 57 at the rate of a large f32 product). A block's products take 4096 cycles of a
+// SIMD at hd 128, so one barrier a block and two workgroups a CU hide the loads. What is left
+// is the tail: 392 workgroups of unequal lists over 256 CUs.
+// TREE: a row's list by its mask, a tile (one row) a workgroup: only slots too wide for
+// attn_f32_step come here.
+template <int HD, bool TREE>
+__global__ __launch_bounds__(F32_THREADS, HD <= 128 ? 2 : 1) void attn_f32_line(const F32Params p) {
+    constexpr int NJ = HD / 16;
+    constexpr int VC = HD >= 64 ? 4 : HD / 16;       // a dims tile's lanes are VC dims apart
+    constexpr int NH = HD / (16 * VC);               // dim 16 VC h + VC m + c is row m of tile (h, c)
+    constexpr int UN = HD / 4;                       // 16-byte units of a row
+    constexpr int NL = F32_BLK * UN / F32_THREADS;   // of K (and of V) a thread loads a block
+    static_assert(NL >= 1 && F32_BLK * UN % F32_THREADS == 0 && CHUNK_MULTI % (2 * F32_BLK) == 0, "");
+    typedef typename VecN<VC>::T vvec;
+    typedef __attribute__((address_space(3))) void lds_t;
+    // Two stages, an object each: the compiler then knows that reads of one don't wait for loads
+    // into the other.
+    __shared__ __attribute__((aligned(16))) F32Stage<HD> st0;
+    __shared__ __attribute__((aligned(16))) F32Stage<HD> st1;
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t n = lane & 15u, g = lane >> 4;
+    const uint32_t per = TREE ? 1u : F32_WAVES;  // tiles of the workgroup
+    const uint32_t kvh = blockIdx.x % p.nkv, nwg = (p.nrb + per - 1) / per;
+    const uint32_t wi = nwg - 1u - blockIdx.x / p.nkv;  // latest rows (longest lists) first
+    const uint32_t rbi = wave < per ? per * wi + wave : p.nrb, r0 = rbi * p.rb, hd = p.hd, kvd = p.nkv * hd;
+    const float* kcb = p.kc + (size_t)kvh * hd;
+    const float* vcb = p.vc + (size_t)kvh * hd;
+    const uint32_t nrow = n % p.rb, head = n / p.rb;
+    const bool valid = head < p.G && r0 + nrow < p.rows;
+    uint32_t lo = 0, hi = 0;  // a tree's workgroup: its row's mask
+    if (TREE) {
+        lo = p.masks[2 * wi];
+        hi = p.masks[2 * wi + 1];
     }
+    const uint32_t maxlen = TREE ? p.pos + __popc(lo) + __popc(hi) : p.pos + min((wi + 1) * per * p.rb, p.rows);
+    const uint32_t len = !valid ? 0u : TREE ? maxlen : p.pos + r0 + nrow + 1u;
+    const uint32_t wlen = r0 >= p.rows ? 0u : TREE ? maxlen : p.pos + min(r0 + p.rb, p.rows);  // the wave's longest list
+
+    // This thread's units of a block.
+    auto load = [&](F32Stage<HD>& st, uint32_t key0) {
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const uint32_t u0 = F32_THREADS * i + 64 * wave, e = (u0 + lane) / UN, u = (u0 + lane) % UN;
+            const uint32_t kk = key0 + e, uk = u ^ (e & 7u);
+            const uint32_t s = TREE && kk >= p.pos && kk < maxlen ? p.pos + nth_set_bit(lo, hi, kk - p.pos) : kk;
+            const bool ok = kk < maxlen && (uint64_t)s < p.slot_limit;
+            const float* ks = ok && 4 * uk < hd ? kcb + (size_t)s * kvd + 4 * uk : p.zero;
+            const float* vs = ok && 4 * u < hd ? vcb + (size_t)s * kvd + 4 * u : p.zero;
+            __builtin_amdgcn_global_load_lds((const void*)ks, (lds_t*)(&st.k[0][0] + u0), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const void*)vs, (lds_t*)(&st.v[0][0] + u0), 16, 0, 0);
+        }
+    };
+    load(st0, 0);
+    f32x4 qx[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        qx[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (valid && 16 * j + 4 * g < hd)
+            qx[j] = *(const f32x4*)&p.q[((size_t)(r0 + nrow) * p.nh + kvh * p.G + head) * hd + 16 * j + 4 * g];
+    }
+    float m = -INFINITY, l = 0.0f, RM = -INFINITY, RL = 0.0f;
+    f32x4 o[NH * VC], R[NH * VC];
+#pragma unroll
+    for (int k = 0; k < NH * VC; k++) o[k] = R[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    auto block = [&](F32Stage<HD>& st, F32Stage<HD>& next, uint32_t key0) {
+        // This stage's loads are in for everyone, and everyone is done with the other's.
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        const bool mine = key0 < wlen;
+        f32x4 a0;
+        if (mine) a0 = st.k[n][g ^ (n & 7u)];  // before the loads below: it would wait for them
+        asm volatile("" : "+v"(a0));
+        if (key0 + F32_BLK < maxlen) load(next, key0 + F32_BLK);
+        if (!mine) return;
+        f32x4 s[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            f32x4 a[8] = {};
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                const f32x4 kx = t == 0 && j == 0 ? a0 : st.k[16 * t + n][(4 * j + g) ^ (n & 7u)];
+#pragma unroll
+                for (int k = 0; k < 4; k++) a[4 * (j % 2) + k] = mfma4(kx[k], qx[j][k], a[4 * (j % 2) + k]);
+            }
+            s[t] = score_tile(a, p.sc, key0 + 16 * t + 4 * g, len);
+        }
+        const float cr = softmax_block(s, m, l);
+        f32x4 acc[NH * VC] = {};
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int h = 0; h < NH; h++) {
+                    const vvec v = *((const vvec*)&st.v[16 * t + 4 * g + i][0] + 16 * h + n);
+#pragma unroll
+                    for (int k = 0; k < VC; k++) acc[VC * h + k] = mfma4(vec_at(v, k), s[t][i], acc[VC * h + k]);
+                }
+#pragma unroll
+        for (int k = 0; k < NH * VC; k++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[k][i] = __builtin_fmaf(o[k][i], cr, acc[k][i]);
+    };
+    for (uint32_t kb0 = 0; kb0 < maxlen; kb0 += CHUNK_MULTI) {
+#pragma unroll 1
+        for (uint32_t key0 = kb0; key0 < min(kb0 + CHUNK_MULTI, maxlen); key0 += 2 * F32_BLK) {
+            block(st0, st1, key0);
+            if (key0 + F32_BLK < maxlen) block(st1, st0, key0 + F32_BLK);
+        }
+        // The chunk's state folded into the running one (merge_coef, R = R a + c b).
+        float fa, fb, mn;
+        merge_coef(RM, m, fa, fb, mn);
+        RL = RL * fa + slot_sum(l) * fb;
+        RM = mn;
+#pragma unroll
+        for (int k = 0; k < NH * VC; k++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                R[k][i] = R[k][i] * fa + o[k][i] * fb;
+                o[k][i] = 0.0f;
+            }
+        m = -INFINITY;
+        l = 0.0f;
+    }
+    if (!valid) return;
+    float* dst = p.out + ((size_t)(r0 + nrow) * p.nh + kvh * p.G + head) * hd;
+#pragma unroll
+    for (int h = 0; h < NH; h++)
+#pragma unroll
+        for (int q4 = 0; q4 < VC; q4++) {
+            // Lane (n, g): dims 16 VC h + 4 VC g + VC i + k of slot n in o[VC h + k][i].
+            const uint32_t d = 16 * VC * h + 4 * VC * g + 4 * q4;
+            f32x4 v;
+#pragma unroll
+            for (int x = 0; x < 4; x++) v[x] = R[VC * h + (4 * q4 + x) % VC][(4 * q4 + x) / VC] / RL;
+            if (d < hd) *(f32x4*)(dst + d) = v;
+        }
 }
 
 static uint32_t ceil_div32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-template <int HD, bool MS>
-static void launch_f32_ms(const F32Params& fp, uint32_t blocks, const AttnCall& a, hipStream_t s, bool fuse) {
-    if (fuse && fp.rows == 1)
-        hipExtLaunchKernelGGL((attn_f32<HD, 1, MS>), dim3(blocks), dim3(F32_THREADS), 0, s, a.ev_before, a.ev_after, 0,
-                              fp);
-    else if (fuse)
-        hipExtLaunchKernelGGL((attn_f32<HD, (int)F32_FUSE_ROWS, MS>), dim3(blocks), dim3(F32_THREADS), 0, s,
-                              a.ev_before, a.ev_after, 0, fp);
-    else
-        hipExtLaunchKernelGGL((attn_f32<HD, 0, MS>), dim3(blocks), dim3(F32_THREADS), 0, s, a.ev_before, a.ev_after, 0,
-                              fp);
-}
-
-// MS: a launch whose workgroups hold more than four query slots (a wave then has several);
-// its own kernels, so that the one-slot-a-wave step keeps the registers of one pass.
 template <int HD>
-static hipError_t launch_f32_t(const F32Params& fp, uint32_t blocks, const AttnCall& a, hipStream_t s, bool fuse) {
-    if constexpr (HD > 64) {
-        if (fp.G * fp.rb > (uint32_t)(F32_THREADS / 64)) {
-            launch_f32_ms<HD, true>(fp, blocks, a, s, fuse);
-            return hipGetLastError();
-        }
-    }
-    launch_f32_ms<HD, false>(fp, blocks, a, s, fuse);
+static hipError_t launch_f32(const F32Params& fp, uint32_t blocks, const AttnCall& a, hipStream_t s, bool fuse, bool line) {
+    const dim3 grid(blocks), wg(F32_THREADS);
+    if (line && fp.tree)
+        hipExtLaunchKernelGGL((attn_f32_line<HD, true>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+    else if (line)
+        hipExtLaunchKernelGGL((attn_f32_line<HD, false>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+    else if (fuse && fp.rows == 1)
+        hipExtLaunchKernelGGL((attn_f32_step<HD, 1>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+    else if (fuse)
+        hipExtLaunchKernelGGL((attn_f32_step<HD, (int)F32_FUSE_ROWS>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+    else
+        hipExtLaunchKernelGGL((attn_f32_step<HD, 0>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
     return hipGetLastError();
 }
+
+// Tiles from which a line takes the line form: below it the states that a split launch writes
+// and the fold reads cost less than CUs left idle or on lists of unequal length (llama-8B heads, 200 rows at
+// 300, 400 tiles: 40 us split; 400 rows at 0, 800 tiles: 41 us unsplit).
+constexpr uint64_t F32_LINE_TILES = 512;
+// Elements of a slot up to which attn_f32_step's 32-bit offsets reach a chunk's slots.
+constexpr uint64_t F32_STEP_KVD = 1u << 20;
 
 hipError_t f32_attention(const AttnCall& a, uint64_t kvoff, Workspace& ws, hipStream_t s, const RopeArgs* rope) {
     if (a.rows == 0 || a.nkv == 0 || a.nh % a.nkv != 0 || a.hd == 0 || a.hd % 8 != 0 || a.hd > MAX_HD)
@@ -569,7 +611,25 @@ hipError_t f32_attention(const AttnCall& a, uint64_t kvoff, Workspace& ws, hipSt
     const uint64_t far = a.tree ? (uint64_t)a.pos + MAX_ITEMS : (uint64_t)a.pos + a.rows;
     fp.nchunk = ceil_div32(far, CHUNK_MULTI);
     const uint64_t groups = (uint64_t)a.nkv * fp.nrb;
-    fp.split = groups < 512 && fp.nchunk > 1;
+    const bool wide = kvd > F32_STEP_KVD;
+    bool line = wide || (!a.tree && !rope && groups >= F32_LINE_TILES);
+    if (a.tree && !wide && groups >= F32_LINE_TILES && fp.nchunk > 1 && a.rows > 1) {
+        // A tree's rows share no list, so the line form (a row a workgroup, one wave of it at work)
+        // is not for them: half the rows at a time bounds the states.
+        AttnCall h = a;
+        h.rows = a.rows / 2;
+        h.ev_after = nullptr;
+        hipError_t e = f32_attention(h, kvoff, ws, s);
+        if (e != hipSuccess) return e;
+        h = a;
+        h.rows = a.rows - a.rows / 2;
+        h.ev_before = nullptr;
+        h.q += (size_t)(a.rows / 2) * a.nh * a.hd;
+        h.out += (size_t)(a.rows / 2) * a.nh * a.hd;
+        h.masks += 2 * (a.rows / 2);
+        return f32_attention(h, kvoff, ws, s);
+    }
+    fp.split = !line && fp.nchunk > 1;
     const uint32_t hdp = a.hd <= 32 ? 32u : a.hd <= 64 ? 64u : a.hd <= 128 ? 128u : 256u;
     if (fp.split) {
         hipError_t e = ws.reserve((size_t)groups * fp.nchunk * F32_SLOTS, hdp);
@@ -577,19 +637,26 @@ hipError_t f32_attention(const AttnCall& a, uint64_t kvoff, Workspace& ws, hipSt
             fp.part_o = ws.o;
             fp.part_ml = ws.ml;
         } else if (ws.fixed) {
-            fp.split = 0;  // a fixed workspace too small for the states: unsplit, the same bits
+            fp.split = 0;  // a fixed workspace too small for the states: the line form, the same bits
+            line = true;
         } else {
             return e;
         }
     }
-    const uint64_t blocks = groups * (fp.split ? fp.nchunk : 1u);
+    const uint64_t blocks = line ? (uint64_t)a.nkv * ceil_div32(fp.nrb, a.tree ? 1 : F32_WAVES) : groups * fp.nchunk;
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
     hipError_t e;
+    if (line && rope) {  // the line form is not fused
+        e = rope_append_launch(rope->q, rope->k, rope->v, (void*)a.kc, (void*)a.vc, 0, rope->inv_freq, rope->positions,
+                               a.rows, a.nh, a.nkv, a.hd, rope->rope_dim, rope->neox, a.pos, s);
+        if (e != hipSuccess) return e;
+        rope = nullptr;
+    }
     switch (hdp) {
-        case 32: e = launch_f32_t<32>(fp, (uint32_t)blocks, a, s, rope != nullptr); break;
-        case 64: e = launch_f32_t<64>(fp, (uint32_t)blocks, a, s, rope != nullptr); break;
-        case 128: e = launch_f32_t<128>(fp, (uint32_t)blocks, a, s, rope != nullptr); break;
-        default: e = launch_f32_t<256>(fp, (uint32_t)blocks, a, s, rope != nullptr); break;
+        case 32: e = launch_f32<32>(fp, (uint32_t)blocks, a, s, rope != nullptr, line); break;
+        case 64: e = launch_f32<64>(fp, (uint32_t)blocks, a, s, rope != nullptr, line); break;
+        case 128: e = launch_f32<128>(fp, (uint32_t)blocks, a, s, rope != nullptr, line); break;
+        default: e = launch_f32<256>(fp, (uint32_t)blocks, a, s, rope != nullptr, line); break;
     }
     if (e != hipSuccess || !fp.split) return e;
     CombineParams cp{};
