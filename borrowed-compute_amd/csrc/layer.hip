@@ -1029,6 +1029,140 @@ __global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_
     if (tid == 0) __hip_atomic_store(&p.cnt[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// One input row (decode) of the block formats, cols a multiple of 256: a workgroup is 16 weight
+// rows, its W waves take the units in turn (one loaded ahead; ONE: a wave has one unit at most),
+// each staging its own unit's x and weights in its own LDS without a barrier. A unit's end and
+// the units' sum are in 64 bits (a few operations a unit), so the error stays at or below the
+// vector-unit pass's, whose f32 chains were shorter. Every A row 0 .. 7 is x's hi
+// and 8 .. 15 its lo (Q6K: both together), so staging is one row and the reads are broadcasts.
+// The vector-unit pass (k_matmul) held 1.75 waves a SIMD on this work, each waiting for a column
+// tile and then converting and multiplying it; here the products go to the matrix cores and the
+// waves are seven a SIMD, which leaves the unpacking (Q6K) and the loads (the others).
+// One row, us a call with the weights from HBM, k_matmul -> here: Q4K 14336 x 4096 14.1 -> 11.3,
+// 4096 x 14336 18.0 -> 11.0; Q6K 22.0 -> 18.0, 26.5 -> 16.4; Q8_0 21.6 -> 15.2, 24.3 -> 15.5;
+// Q4K 1024 x 4096 5.9 -> 3.9. 32 rows a workgroup (x staged once for both) were 6% faster at Q4K
+// 28672 x 8192 and 9-18% slower for Q8_0 and Q4_0. Error against 64 bits at 14336 columns:
+// Q4_0 2.4e-7 -> 0.8e-7, Q8_0 1.2 -> 0.9, Q4K 1.8 -> 1.7, Q5K 1.8 -> 1.6, Q6K 2.4 -> 1.0.
+constexpr uint32_t ROW_UNITS = 256;  // units whose sums fit the workgroup's LDS
+
+template <uint32_t TY, int W, bool ONE>
+__global__ __launch_bounds__(64 * W) void k_matmul_row(const MMParams p) {
+    constexpr bool SUM = mm_sum<TY>(), UT = TY == G_Q4K || TY == G_Q5K;
+    static_assert(MM_LDSP<TY>, "block formats");
+    constexpr uint32_t XL = 288;  // halves from hi to lo: other banks
+    __shared__ __attribute__((aligned(16))) f16 xs[W][XL + 256];
+    __shared__ __attribute__((aligned(16))) uint8_t wtb[W][16 * MM_WT<TY>];
+    __shared__ __attribute__((aligned(16))) f16 ss[W][SUM ? 32 : 8];
+    extern __shared__ __attribute__((aligned(16))) double ps[];  // [units][16], then [units] inverse scales
+    float* isc = (float*)(ps + p.units * 16);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t c = lane >> 4, rl = lane & 15;
+    const uint32_t r0 = blockIdx.x * 16;
+    // the lane's matrix-core row and its lane quad's
+    const uint8_t* mrow = p.w + (size_t)min(r0 + rl, p.rows - 1) * p.row_bytes;
+    const uint8_t* qrow = p.w + (size_t)min(r0 + (lane >> 2), p.rows - 1) * p.row_bytes;
+    uint8_t* wt = wtb[w];
+    // LDS written and read by one wave only: in order, no barrier.
+    auto own = [&]() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+    if constexpr (SUM)
+        if (lane == 0) *(half8*)&ss[w][24] = half8{};
+    constexpr int PF = ONE ? 1 : 2;
+    uint32_t pk[PF][MW<TY>];
+    float4 xv[PF];
+    // Past the wave's last unit the loads are of the first row's first unit, the same few lines for
+    // every wave, so that each use waits for a fixed number of loads.
+    auto load = [&](uint32_t u, uint32_t (&d)[MW<TY>], float4& x) {
+        const bool in = u < p.units;
+        const uint32_t uu = in ? u : 0;
+        x = *(const float4*)(p.x + (size_t)uu * 256 + 4 * lane);
+        mm_load<TY>(in ? qrow : p.w, uu, c, d);
+    };
+    load(w, pk[0], xv[0]);
+    if constexpr (!ONE) load(w + W, pk[1], xv[1]);
+    for (uint32_t u0 = w; u0 < p.units; u0 += PF * W) {
+#pragma unroll
+        for (int f = 0; f < PF; f++) {
+            const uint32_t u = u0 + f * W;
+            if (u < p.units) {
+                const float x4[4] = {xv[f].x, xv[f].y, xv[f].z, xv[f].w};
+                float sc, inv;
+                unit_scale(x4, sc, inv);
+                if (lane == 0) isc[u] = inv;
+                if constexpr (SUM) {
+                    const float sg = group_sum(x4);
+                    if ((lane & 7) == 0) {
+                        f16 sp[3];
+                        sum_parts(sg, sc, sp);
+#pragma unroll
+                        for (int e = 0; e < 3; e++) ss[w][8 * e + lane / 8] = sp[e];
+                    }
+                }
+                const float xo[4] = {x4[0], x4[2], x4[1], x4[3]};
+                half4 h, o;
+                hi_lo(xo, sc, h, o);
+                if constexpr (TY == G_Q6K) {
+                    *(half8*)&xs[w][8 * lane] = __builtin_shufflevector(h, o, 0, 1, 2, 3, 4, 5, 6, 7);
+                } else {
+                    *(half4*)&xs[w][4 * lane] = h;
+                    *(half4*)&xs[w][XL + 4 * lane] = o;
+                }
+                own();
+                const f16* xr = &xs[w][TY == G_Q6K || rl < 8 ? 0 : XL];
+                const f32x4 z4 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                const uint8_t* ub = mrow + (size_t)u * MM_UB<TY>;
+                const uint8_t* qb = qrow + (size_t)u * MM_UB<TY>;
+                uint32_t dd[MWD<TY>];
+                mm_fix<TY>(pk[f], dd, wt, c, rl, (uint32_t)((uintptr_t)qb & 15u), (uint32_t)((uintptr_t)ub & 15u));
+                const MMUnit m = mm_unit<TY>(dd);
+                f32x4 t4 = z4;
+                float s = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    half8 q;
+                    half4 qh[2];
+                    float a0 = 0.0f, a1 = 0.0f;
+                    mm_group<TY>(dd, m, ub, wt + rl * MM_WT<TY>, j, c, q, qh, a0, a1);
+                    if constexpr (TY == G_Q6K) {
+                        const half8 x0 = *(const half8*)&xr[64 * j + 8 * c], x1 = *(const half8*)&xr[64 * j + 32 + 8 * c];
+                        const f32x4 d0 = mfma16(x0, __builtin_shufflevector(qh[0], qh[0], 0, 1, 2, 3, 4, 5, 6, 7), z4);
+                        const f32x4 d1 = mfma16(x1, __builtin_shufflevector(qh[1], qh[1], 0, 1, 2, 3, 4, 5, 6, 7), z4);
+                        s = __builtin_fmaf(a1, d1[0], __builtin_fmaf(a0, d0[0], s));
+                    } else {
+                        const half8 xa = *(const half8*)&xr[32 * j + 8 * c];
+                        if constexpr (UT)
+                            t4 = mfma16(xa, q, t4);
+                        else
+                            s = __builtin_fmaf(a0, mfma16(xa, q, z4)[0], s);
+                    }
+                }
+                if constexpr (UT) s = t4[0];
+                double sum = s;
+                if constexpr (TY != G_Q6K) {  // hi + lo
+                    const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+                    sum = (double)__uint_as_float(r2[0]) + (double)__uint_as_float(r2[1]);
+                }
+                if constexpr (UT) sum *= (double)m.dl;
+                if constexpr (SUM) {
+                    half8 mv;
+                    if constexpr (UT) mv = mins_f16(m.mnA, m.mnB);
+                    else mv = __builtin_bit_cast(half8, u32x4{dd[0], dd[1], dd[2], dd[3]});
+                    sum = __builtin_fma((double)m.bl, (double)mfma16(*(const half8*)&ss[w][8 * c], mv, z4)[0], sum);
+                }
+                if (c == 0) ps[u * 16 + rl] = sum;
+                own();
+            }
+            // the unit's registers are free: load into them directly
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!ONE) load(u + 2 * W, pk[f], xv[f]);
+        }
+    }
+    __syncthreads();
+    if (tid >= 16 || r0 + tid >= p.rows) return;
+    double tot = 0.0;
+    for (uint32_t u = 0; u < p.units; u++) tot = __builtin_fma((double)isc[u], ps[u * 16 + tid], tot);
+    p.out[r0 + tid] = (float)tot;
+}
+
 // ---------------------------------------------------------------------------------------
 // Batched product of many input rows (prompts). k_matmul_mm's workgroups hold 8 input rows,
 // so a batch of n unpacks every weight n / 8 times and is bound by that VALU work (512 rows
@@ -1767,6 +1901,28 @@ static hipError_t matmul_mm_go(const MatmulParams& mp, void* scratch, uint32_t* 
     return hipGetLastError();
 }
 
+static bool matmul_uses_row(uint32_t type, uint32_t cols, uint32_t n) {
+    return n == 1 && mm_types(type) && type != G_F16 && cols % 256 == 0 && cols / 256 <= ROW_UNITS;
+}
+template <uint32_t TY>
+static hipError_t matmul_row_go(const MatmulParams& mp, hipStream_t s) {
+    const uint32_t units = mp.cols / 256;
+    const MMParams q{mp.w, mp.x, mp.out, nullptr, nullptr, mp.rows, mp.cols, 1, 1, mp.row_bytes, units, 1, 0};
+    const size_t lds = (size_t)units * (16 * sizeof(double) + sizeof(float));
+    const dim3 grid((mp.rows + 15) / 16);
+    // Sixteen waves a workgroup where there is at most one a CU, eight where there are more.
+    // (with f32 sums at the end) 4096 x 14336 at sixteen and eight: Q4K 13.1 and 14.3 us, Q6K 18.7
+    // and 20.1; 14336 x 4096: 15.5 and 11.9, 22.6 and 18.9; 8192 x 28672: 40.9 and 39.0. Up to sixteen
+    // units a wave has one: 3584 x 3584 Q4K 6.3 -> 5.8 us without the second load and the loop.
+    if (mp.rows > 4096)
+        hipLaunchKernelGGL((k_matmul_row<TY, 8, false>), grid, dim3(512), lds, s, q);
+    else if (units > 16)
+        hipLaunchKernelGGL((k_matmul_row<TY, 16, false>), grid, dim3(1024), lds, s, q);
+    else
+        hipLaunchKernelGGL((k_matmul_row<TY, 16, true>), grid, dim3(1024), lds, s, q);
+    return hipGetLastError();
+}
+
 template <uint32_t TY>
 static hipError_t matmul_units_go(const MatmulParams& mp, hipStream_t s) {
     const uint32_t units = (mp.cols + 255) / 256;
@@ -1825,7 +1981,8 @@ static void matmul_go(const MatmulParams& mp, hipStream_t s) {
     hipLaunchKernelGGL((k_matmul<TY, NBT, R>), grid, dim3(64 * MM_WAVES), lds, s, mp);
 }
 
-// One input row (decode): eight rows a wave when a group packs into at most 12 dwords and
+// One input row in the vector-unit pass (the plain types, and cols off a multiple of 256 or
+// beyond ROW_UNITS units): eight rows a wave when a group packs into at most 12 dwords and
 // the matrix still gives 256+ workgroups (measured: the 14336 x 4096 Q4K product 21.3 ->
 // 14.2 µs), else four. Batches: four rows a wave, eight input rows a pass.
 template <uint32_t TY>
@@ -1835,6 +1992,8 @@ static hipError_t matmul_t(const MatmulParams& mp, bool tile, void* scratch, uin
         if constexpr (!tl_kq<TY>() && TY != G_Q6K)
             if (matmul_uses_units(TY, mp.cols, mp.n)) return matmul_units_go<TY>(mp, s);
         if (matmul_uses_mm(TY, mp.cols, mp.n)) return matmul_mm_go<TY>(mp, scratch, counters, s);
+        if constexpr (MM_LDSP<TY>)
+            if (matmul_uses_row(TY, mp.cols, mp.n)) return matmul_row_go<TY>(mp, s);
     }
     if (mp.n == 1) {
         if (PK<TY> <= 12 && mp.rows >= 256u * MM_WAVES * 8)
