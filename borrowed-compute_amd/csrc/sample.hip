@@ -576,7 +576,8 @@ __device__ float segment_total(SmpScan& sc, const float* p, uint32_t vocab, cons
 // f32 mass of k shares p / total, each rounded, falls short of their true sum by less than (k +
 // 2) 2^-24 of it, so bins whose true mass M of K tokens gives M / total (1 - (K + 2) 2^-24) >=
 // top_p hold the whole kept prefix. Tokens of p = 0 move no sum and are never picked past the
-// first place (the largest p is 1), so they are left out.
+// first place (the largest p is 1), so they are left out. The bound's bins hold at least one
+// token, the most likely one, as the reference keeps at least one.
 // firsts[k]: the first place at or past k SMP_BUCKET at which a bin of the candidates begins (or
 // their end).
 __global__ __launch_bounds__(SMP_THREADS) void k_sample_bound(uint64_t* p_out, uint32_t vocab, SmpRow* __restrict__ info,
@@ -628,7 +629,9 @@ __global__ __launch_bounds__(SMP_THREADS) void k_sample_bound(uint64_t* p_out, u
         h->place[bin] = rc;
         rm += bm[k];
         rc += bc[k];
-        if ((double)rm * 9.094947017729282e-13 / (double)total * (1.0 - (double)(rc + 2u) * 5.960464477539063e-8) >= (double)top_p)
+        // (A bin above every token is no bound: at a top_p of 0 or less its mass of 0 would reach it.)
+        if (rc > 0 &&
+            (double)rm * 9.094947017729282e-13 / (double)total * (1.0 - (double)(rc + 2u) * 5.960464477539063e-8) >= (double)top_p)
             atomicMax(&bound_s, bin);
     }
     __syncthreads();

@@ -67,3 +67,20 @@ def test_rows_with_nans_infinities_and_zeros(ctx, vocab):
         got = ids_of(ctx, s, 1.0, top_p, 5, 40)
         want = [O.sample(s[r], 1.0, top_p, 5, 40 + r) for r in range(5)]
         np.testing.assert_array_equal(got, np.array(want, np.uint32), err_msg=f"top_p {top_p}")
+
+
+@pytest.mark.parametrize("vocab", [300, 8192, 8193, 40000])
+def test_top_p_at_or_below_zero_keeps_the_first_token(ctx, vocab):
+    """A running mass of nothing already reaches such a top_p, but at least one token is kept. The
+    scratch holds another call's keys, whose ids are not the answer. (NaN: no mass reaches it.)"""
+    rng = np.random.default_rng(vocab)
+    s = (rng.standard_normal((4, vocab)) * 2).astype(np.float32)
+    s[3] = -5.0
+    s[3, [vocab // 3, vocab - 1]] = 40.0  # two tokens of p = 1, all others next to 0
+    ids_of(ctx, s[:, ::-1] * np.float32(0.5), 0.7, 1.0, 1, 0)
+    for top_p in (0.0, -0.0, -1.0, -np.inf, np.nan, 2.0):
+        got = ids_of(ctx, s, 0.9, top_p, 11, 3)
+        want = [O.sample(s[r], 0.9, top_p, 11, 3 + r) for r in range(4)]
+        np.testing.assert_array_equal(got, np.array(want, np.uint32), err_msg=f"top_p {top_p}")
+        if top_p <= 0:
+            np.testing.assert_array_equal(got, s.argmax(axis=1))
