@@ -467,24 +467,24 @@ int bchip_matmul(bchip_ctx* c, const void* w, uint32_t type, const float* x, flo
     CHECK(check_span(c, w, sat_mul(row_bytes, rows), "weights"));
     CHECK(check_span(c, x, sat_mul(n, (uint64_t)cols * 4), "x"));
     CHECK(check_span(c, out, sat_mul(n, (uint64_t)rows * 4), "out"));
-    // The tile kernel's scratch may not be had: device memory may be full, and nothing can be
-    // allocated while the stream is captured. The call then runs without it.
-    bool tile = matmul_uses_tile(type, rows, cols, n);
-    if (tile) {
-        const size_t sb = matmul_scratch_bytes(type, rows, cols, n, true);
+    // Scratch may not be had: device memory may be full, and nothing can be allocated while the
+    // stream is captured. The call then runs without it, to the same bits.
+    auto scratch = [&](size_t bytes) -> void* {
+        if (bytes <= c->ws.vt_bytes) return c->ws.vt;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (sb > c->ws.vt_bytes &&
-            (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-             c->ws.reserve_vt(sb) != hipSuccess)) {
-            (void)hipGetLastError();
-            tile = false;
-        }
+        if (hipStreamIsCapturing(c->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+            c->ws.reserve_vt(bytes) == hipSuccess)
+            return c->ws.vt;
+        (void)hipGetLastError();
+        return nullptr;
+    };
+    bool tile = matmul_uses_tile(type, rows, cols, n);
+    void* work = tile ? scratch(matmul_scratch_bytes(type, rows, cols, n, true)) : nullptr;
+    if (!work) {
+        tile = false;
+        if (const size_t sb = matmul_scratch_bytes(type, rows, cols, n, false)) work = scratch(sb);
     }
-    if (!tile) {
-        const size_t sb = matmul_scratch_bytes(type, rows, cols, n, false);
-        if (sb) HIP_TRY(c->ws.reserve_vt(sb), "matmul scratch");
-    }
-    HIP_TRY(matmul_launch(w, type, x, out, rows, cols, n, (uint32_t)row_bytes, tile, c->ws.vt, c->mm_cnt, c->stream),
+    HIP_TRY(matmul_launch(w, type, x, out, rows, cols, n, (uint32_t)row_bytes, tile, work, c->mm_cnt, c->stream),
             "matmul");
     return BCHIP_OK;
 }

@@ -141,12 +141,12 @@ hipError_t sample_launch(const float* scores, uint32_t rows, uint32_t vocab, flo
 bool ggml_block(uint32_t type, uint32_t& weights, uint32_t& bytes);
 // Input rows one product call takes: passes of 8 rows over the grid's y dimension (65535).
 constexpr uint32_t MATMUL_MAX_N = 8u * 65535u;
-// Batches of n >= 2 input rows of the quantised formats and F16 run on the matrix cores; their K splits may need matmul_scratch_bytes of scratch (partial
-// sums) and a context's MATMUL_COUNTERS arrival counters (zero when no product runs).
+// Batches of n >= 2 input rows of the quantised formats and F16 run on the matrix cores; their K
+// splits may take matmul_scratch_bytes of scratch (partial sums) and a context's MATMUL_COUNTERS
+// arrival counters (zero when no product runs).
 constexpr uint32_t MATMUL_COUNTERS = 1024;
-// Larger batches, and batches whose cols is no multiple of 256, take the tile kernel (tile:
-// matmul_uses_tile), which needs scratch for the prepared input rows. Without it (tile false)
-// every call still runs.
+// Larger batches take the tile kernel (tile: matmul_uses_tile), which needs scratch for the
+// prepared input rows. scratch null: the call runs without (tile false, K splits in turn).
 bool matmul_uses_tile(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n);
 size_t matmul_scratch_bytes(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n, bool tile);
 hipError_t matmul_launch(const void* w, uint32_t type, const float* x, float* out, uint32_t rows, uint32_t cols,

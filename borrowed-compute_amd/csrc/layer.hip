@@ -1883,8 +1883,7 @@ size_t matmul_scratch_bytes(uint32_t type, uint32_t rows, uint32_t cols, uint32_
 template <uint32_t TY>
 static hipError_t matmul_mm_go(const MatmulParams& mp, void* scratch, uint32_t* counters, hipStream_t s) {
     const uint32_t ks = mm_ks(TY, mp.rows, mp.cols), rt = (mp.rows + 16 * MM_W<TY> - 1) / (16 * MM_W<TY>);
-    const bool par = mm_par(TY, mp.rows, mp.cols, mp.n);
-    if (par && (!scratch || !counters)) return hipErrorInvalidValue;
+    const bool par = scratch && counters && mm_par(TY, mp.rows, mp.cols, mp.n);  // (else in turn: the same bits)
     const MMParams q{mp.w, mp.x, mp.out, (float*)scratch, counters, mp.rows, mp.cols, mp.n, (mp.n + 15) / 16 * 16,
                      mp.row_bytes, mp.cols / 256, ks, par ? 1u : 0u};
     // Sixteen inputs a workgroup for one such block over a matrix large enough to fill the GPU with
