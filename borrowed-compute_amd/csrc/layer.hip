@@ -1417,9 +1417,11 @@ __device__ __forceinline__ void tl_stash(const uint32_t (&d)[TLP<TY>], const uin
 // (as the tile kernel does) in its own LDS without a barrier, and the units' sums meet in order.
 // Bound by latency: Q8_0 4864 x 896 at 2 / 6 / 16 rows 5.3 / 6.2 / 9.2 us (the VALU pass of 8
 // rows 7.8 / 14 / 31; the tile kernel and its preparation 13).
-constexpr uint32_t WV_UNITS = 56;  // units whose sums fit the workgroup's LDS
+// LONG: more units than the workgroup's LDS holds sums of go in stretches (the tile kernel's
+// work, but for a call whose scratch cannot be had; the loop over stretches cost the others 2%).
+constexpr uint32_t WV_UNITS = 56;
 
-template <uint32_t TY, int W>
+template <uint32_t TY, int W, bool LONG>
 __global__ __launch_bounds__(64 * W) void k_matmul_units(const TLParams p, const float* __restrict__ x, uint32_t cols) {
     constexpr bool SUM = mm_sum<TY>(), UT = TY == G_F16;
     constexpr int XS = 264;  // halves an x row
@@ -1440,88 +1442,108 @@ __global__ __launch_bounds__(64 * W) void k_matmul_units(const TLParams p, const
     auto own = [&]() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
     if constexpr (SUM)
         if (lane < 8) *(half8*)&ss[w][32 * lane + 24] = half8{};
-    for (uint32_t u = w; u < p.units; u += W) {
-        uint32_t pk[4][TLP<TY>], hd[TLH<TY>];
-        MMUnit mu;
-        const uint32_t ns = min(4u, nsteps - 4 * u);
+    auto stretch = [&](uint32_t u0, uint32_t ue) {
+        for (uint32_t u = u0 + w; u < ue; u += W) {
+            uint32_t pk[4][TLP<TY>], hd[TLH<TY>];
+            MMUnit mu;
+            const uint32_t ns = min(4u, nsteps - 4 * u);
 #pragma unroll
-        for (uint32_t s = 0; s < 4; s++) tl_load<TY>(wrow, min(4 * u + s, nsteps - 1), qd, p.groups, pk[s]);
-        const uint32_t col = 256 * u + 4 * lane;
-        float4 v[8];
+            for (uint32_t s = 0; s < 4; s++) tl_load<TY>(wrow, min(4 * u + s, nsteps - 1), qd, p.groups, pk[s]);
+            const uint32_t col = 256 * u + 4 * lane;
+            float4 v[8];
 #pragma unroll
-        for (uint32_t i = 0; i < 8; i++)
-            v[i] = *(const float4*)(x + (size_t)(i0 + min(i, ni - 1)) * cols + min(col, cols - 4));
+            for (uint32_t i = 0; i < 8; i++)
+                v[i] = *(const float4*)(x + (size_t)(i0 + min(i, ni - 1)) * cols + min(col, cols - 4));
 #pragma unroll
-        for (uint32_t i = 0; i < 8; i++) {
-            if (i >= ni) break;
-            const bool in = col < cols;
-            const float x4[4] = {in ? v[i].x : 0.0f, in ? v[i].y : 0.0f, in ? v[i].z : 0.0f, in ? v[i].w : 0.0f};
-            float sc, inv;
-            unit_scale(x4, sc, inv);
-            if (lane == 0) isc[u][i] = inv;
+            for (uint32_t i = 0; i < 8; i++) {
+                if (i >= ni) break;
+                const bool in = col < cols;
+                const float x4[4] = {in ? v[i].x : 0.0f, in ? v[i].y : 0.0f, in ? v[i].z : 0.0f, in ? v[i].w : 0.0f};
+                float sc, inv;
+                unit_scale(x4, sc, inv);
+                if (lane == 0) isc[u - u0][i] = inv;
+                if constexpr (SUM) {
+                    const float sg = group_sum(x4);
+                    if ((lane & 7) == 0) {
+                        f16 sp[3];
+                        sum_parts(sg, sc, sp);
+#pragma unroll
+                        for (int e = 0; e < 3; e++) ss[w][i * 32 + 8 * e + lane / 8] = sp[e];
+                    }
+                }
+                const float xo[4] = {x4[0], UT ? x4[1] : x4[2], UT ? x4[2] : x4[1], x4[3]};
+                half4 h, o;
+                hi_lo(xo, sc, h, o);
+                *(half4*)&xs[w][i * XS + 4 * lane] = h;
+                *(half4*)&xs[w][(8 + i) * XS + 4 * lane] = o;
+            }
+            f32x4 t = z4;  // hi in lanes c < 2, lo in c >= 2
+#pragma unroll
+            for (uint32_t s = 0; s < 4; s++) {
+                if (s >= ns) break;
+                tl_stash<TY, false, 16>(pk[s], hd, mu, 4 * u + s, s, tr, qd, p.groups, wl[w][s & 1], sa[w][s & 1], nullptr, um[w]);
+                own();
+#pragma unroll
+                for (uint32_t g = 0; g < 2; g++) {
+                    if (8 * u + 2 * s + g >= p.groups) break;
+                    const half8 b = *(const half8*)(wl[w][s & 1] + l * 128 + 16 * ((4 * g + c) ^ ((l >> 1) & 7u)));
+                    const half8 xa = *(const half8*)&xs[w][l * XS + 64 * s + 32 * g + 8 * c];
+                    if constexpr (UT) {
+                        t = mfma16(xa, b, t);
+                    } else {
+                        const f32x4 d = mfma16(xa, b, z4);
+                        const float a = sa[w][s & 1][g * 16 + l];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) t[e] = __builtin_fmaf(a, d[e], t[e]);
+                    }
+                }
+                own();
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[e]), __float_as_uint(t[e]), false, false);
+                t[e] = __uint_as_float(r2[0]) + __uint_as_float(r2[1]);
+            }
             if constexpr (SUM) {
-                const float sg = group_sum(x4);
-                if ((lane & 7) == 0) {
-                    f16 sp[3];
-                    sum_parts(sg, sc, sp);
+                const f32x4 tb = mfma16(*(const half8*)&ss[w][(l & 7u) * 32 + 8 * c], *(const half8*)&um[w][8 * l], z4);
 #pragma unroll
-                    for (int e = 0; e < 3; e++) ss[w][i * 32 + 8 * e + lane / 8] = sp[e];
-                }
+                for (int e = 0; e < 4; e++) t[e] = __builtin_fmaf(32.0f, tb[e], t[e]);
+                own();
             }
-            const float xo[4] = {x4[0], UT ? x4[1] : x4[2], UT ? x4[2] : x4[1], x4[3]};
-            half4 h, o;
-            hi_lo(xo, sc, h, o);
-            *(half4*)&xs[w][i * XS + 4 * lane] = h;
-            *(half4*)&xs[w][(8 + i) * XS + 4 * lane] = o;
+            if (c < 2)
+#pragma unroll
+                for (int e = 0; e < 4; e++) ps[u - u0][4 * c + e][l] = t[e];
         }
-        f32x4 t = z4;  // hi in lanes c < 2, lo in c >= 2
-#pragma unroll
-        for (uint32_t s = 0; s < 4; s++) {
-            if (s >= ns) break;
-            tl_stash<TY, false, 16>(pk[s], hd, mu, 4 * u + s, s, tr, qd, p.groups, wl[w][s & 1], sa[w][s & 1], nullptr, um[w]);
-            own();
-#pragma unroll
-            for (uint32_t g = 0; g < 2; g++) {
-                if (8 * u + 2 * s + g >= p.groups) break;
-                const half8 b = *(const half8*)(wl[w][s & 1] + l * 128 + 16 * ((4 * g + c) ^ ((l >> 1) & 7u)));
-                const half8 xa = *(const half8*)&xs[w][l * XS + 64 * s + 32 * g + 8 * c];
-                if constexpr (UT) {
-                    t = mfma16(xa, b, t);
-                } else {
-                    const f32x4 d = mfma16(xa, b, z4);
-                    const float a = sa[w][s & 1][g * 16 + l];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) t[e] = __builtin_fmaf(a, d[e], t[e]);
-                }
-            }
-            own();
-        }
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[e]), __float_as_uint(t[e]), false, false);
-            t[e] = __uint_as_float(r2[0]) + __uint_as_float(r2[1]);
-        }
-        if constexpr (SUM) {
-            const f32x4 tb = mfma16(*(const half8*)&ss[w][(l & 7u) * 32 + 8 * c], *(const half8*)&um[w][8 * l], z4);
-#pragma unroll
-            for (int e = 0; e < 4; e++) t[e] = __builtin_fmaf(32.0f, tb[e], t[e]);
-            own();
-        }
-        if (c < 2)
-#pragma unroll
-            for (int e = 0; e < 4; e++) ps[u][4 * c + e][l] = t[e];
-    }
-    __syncthreads();
+    };
     // The units' sums in order, split by split (k_matmul_mm's accumulation).
-    if (tid >= 128) return;
     const uint32_t i = tid >> 4, r = r0 + (tid & 15);
-    if (i >= ni || r >= p.rows) return;
-    float tot = 0.0f;
-    for (uint32_t kz = 0; kz < p.ks; kz++) {
-        const uint32_t ua = kz * p.units / p.ks, ue = (kz + 1) * p.units / p.ks;
-        float acc = 0.0f;
-        for (uint32_t u = ua; u < ue; u++) acc = __builtin_fmaf(isc[u][i], ps[u][i][tid & 15], acc);
-        tot = kz == 0 ? acc : tot + acc;
+    const bool folds = tid < 128 && i < ni && r < p.rows;
+    float acc = 0.0f, tot = 0.0f;
+    uint32_t kz = 0, kend = p.units / p.ks;
+    auto fold = [&](uint32_t u0, uint32_t ue) {
+        for (uint32_t u = u0; u < ue; u++) {
+            acc = __builtin_fmaf(isc[u - u0][i], ps[u - u0][i][tid & 15], acc);
+            if (u + 1 < kend) continue;
+            tot = kz == 0 ? acc : tot + acc;
+            acc = 0.0f;
+            kz++;
+            kend = (kz + 1) * p.units / p.ks;
+        }
+    };
+    if constexpr (LONG) {
+        for (uint32_t u0 = 0; u0 < p.units; u0 += WV_UNITS) {
+            const uint32_t ue = min(u0 + WV_UNITS, p.units);
+            stretch(u0, ue);
+            __syncthreads();
+            if (folds) fold(u0, ue);
+            __syncthreads();  // the next stretch's sums take their place
+        }
+        if (!folds) return;
+    } else {
+        stretch(0, p.units);
+        __syncthreads();
+        if (!folds) return;
+        fold(0, p.units);
     }
     p.out[(size_t)(i0 + i) * p.rows + r] = tot;
 }
@@ -1836,13 +1858,13 @@ constexpr uint64_t TL_MACS = 760000000, TL_MACS_RAGGED = 134000000;
 constexpr size_t TL_SLAB_BYTES = (size_t)256 << 20;
 
 static bool matmul_uses_units(uint32_t type, uint32_t cols, uint32_t n) {
-    return mm_types(type) && cols % 256 != 0 && n >= MM_MIN && (cols + 255) / 256 <= WV_UNITS;
+    return mm_types(type) && cols % 256 != 0 && n >= MM_MIN;
 }
 bool matmul_uses_tile(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n) {
     const uint64_t macs = (uint64_t)rows * cols * n;
     if (!mm_types(type)) return false;
     if (cols % 256 == 0) return n >= TL_MIN && macs >= TL_MACS;
-    return n >= MM_MIN && (!matmul_uses_units(type, cols, n) || (n >= TL_MIN && macs >= TL_MACS_RAGGED));
+    return n >= MM_MIN && ((cols + 255) / 256 > WV_UNITS || (n >= TL_MIN && macs >= TL_MACS_RAGGED));
 }
 
 struct TilePlan {
@@ -1929,9 +1951,11 @@ static hipError_t matmul_units_go(const MatmulParams& mp, hipStream_t s) {
                      units, mp.cols / 32, mm_ks(TY, mp.rows, mp.cols), 0, 0};
     const dim3 grid((mp.rows + 15) / 16, (mp.n + 7) / 8);
     if (units <= 4)
-        hipLaunchKernelGGL((k_matmul_units<TY, 4>), grid, dim3(256), 0, s, q, mp.x, mp.cols);
+        hipLaunchKernelGGL((k_matmul_units<TY, 4, false>), grid, dim3(256), 0, s, q, mp.x, mp.cols);
+    else if (units <= WV_UNITS)
+        hipLaunchKernelGGL((k_matmul_units<TY, 8, false>), grid, dim3(512), 0, s, q, mp.x, mp.cols);
     else
-        hipLaunchKernelGGL((k_matmul_units<TY, 8>), grid, dim3(512), 0, s, q, mp.x, mp.cols);
+        hipLaunchKernelGGL((k_matmul_units<TY, 8, true>), grid, dim3(512), 0, s, q, mp.x, mp.cols);
     return hipGetLastError();
 }
 

@@ -40,6 +40,15 @@ def test_a_captured_call_without_scratch(ty, rows, cols, n):
     run(ty, rows, cols, n)
 
 
+# Cols off a multiple of 256, on both sides of the 56 units whose sums k_matmul_units holds at
+# once, with one K split, a few and many.
+@pytest.mark.parametrize("ty", [O.F16, O.Q8_0, O.Q4_0, O.Q4_1, O.Q5_0, O.Q5_1], ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,n", [(4864, 896, 70), (333, 14304, 40), (333, 14368, 40), (65, 29568, 9),
+                                         (20000, 14368, 2), (17, 43040, 33)])
+def test_a_captured_call_off_a_multiple_of_256(ty, rows, cols, n):
+    run(ty, rows, cols, n)
+
+
 def run(ty, rows, cols, n):
     some = min(rows, 131)
     data = np.resize(np.asarray(O.random_tensor(ty, some, cols, rows + n), np.uint8).reshape(some, -1),
