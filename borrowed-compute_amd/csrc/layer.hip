@@ -1854,8 +1854,9 @@ static bool matmul_uses_mm(uint32_t type, uint32_t cols, uint32_t n) {
 // rows, 0.07 G: 9.2 us there, 15.8 here; at 67, 0.29 G: about 35 there, 20 here).
 constexpr uint32_t TL_MIN = 17;
 constexpr uint64_t TL_MACS = 760000000, TL_MACS_RAGGED = 134000000;
-// Bytes of prepared x a launch takes at most; longer batches go in slabs of input rows.
-constexpr size_t TL_SLAB_BYTES = (size_t)256 << 20;
+// Bytes of prepared x a launch takes at most, and its input rows (k_mm_prep's grid.y is a quarter of
+// them, of 65535); longer batches go in slabs of input rows.
+constexpr size_t TL_SLAB_BYTES = (size_t)256 << 20, TL_SLAB_ROWS = 4 * 65535;
 
 static bool matmul_uses_units(uint32_t type, uint32_t cols, uint32_t n) {
     return mm_types(type) && cols % 256 != 0 && n >= MM_MIN;
@@ -1877,7 +1878,7 @@ static TilePlan tile_plan(uint32_t type, uint32_t rows, uint32_t cols, uint32_t 
     t.groups = cols / 32;
     t.nxt = (rows + TL_NT - 1) / TL_NT;
     const size_t row_bytes = (size_t)(t.groups + 1) / 2 * 256;
-    t.slab = (uint32_t)std::max<size_t>(TL_SLAB_BYTES / row_bytes / 128 * 128, 128);
+    t.slab = (uint32_t)std::max<size_t>(std::min(TL_SLAB_BYTES / row_bytes, TL_SLAB_ROWS) / 128 * 128, 128);
     const uint32_t m = min(n, t.slab);
     // Input rows a workgroup: 128 where that still gives every CU one.
     t.mt = m <= 32 ? 32 : (m > 64 && (uint64_t)t.nxt * ((m + 127) / 128) >= 256) ? 128 : 64;

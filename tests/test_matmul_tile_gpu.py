@@ -82,3 +82,25 @@ def test_cols_off_a_multiple_of_256(ctx, ty, rows, cols):
     err = np.abs(whole - O.matmul_f64(ty, data, rows, cols, x, n))
     print(f"{O.TYPE_NAMES[ty]} {rows}x{cols}: at most {np.max(err / bound):.3g} of the bound", flush=True)
     assert (err <= bound).all()
+
+
+# Batches of more than one slab of input rows: 256 MiB of prepared x (4608 rows of 14336 columns),
+# and 262016 rows where narrow inputs would fit more.
+@pytest.mark.parametrize("ty,rows,cols,n,slab", [(O.Q4K, 256, 14336, 4700, 4608), (O.Q8_0, 130, 14336, 9300, 4608),
+                                                 (O.F16, 12, 256, 262500, 262016), (O.Q8_0, 17, 96, 524280, 262016)],
+                         ids=str)
+def test_slabs_give_the_small_batches_bits(ctx, ty, rows, cols, n, slab):
+    wb = ctx.upload(np.asarray(O.random_tensor(ty, rows, cols, 3), np.uint8))
+    xb, ob, part = ctx.zeros(n * cols * 4), ctx.zeros(n * rows * 4), ctx.zeros(16 * rows * 4)
+    ctx.fill_normal(xb, bchip.F32, n * cols, 5)
+    ctx.matmul(wb, ty, xb, ob, rows, cols, n)
+    for at in (0, slab - 16, slab - 5, slab, 2 * slab - 8, n - 16):
+        at = min(at, n - 16)
+        got = ctx.read(ob, (16, rows), off=at * rows * 4)
+        assert got.all() and np.isfinite(got).all()
+        xs = ctx.upload(ctx.read(xb, (16, cols), off=at * cols * 4))
+        ctx.matmul(wb, ty, xs, part, rows, cols, 16)
+        np.testing.assert_array_equal(got, ctx.read(part, (16, rows)), err_msg=f"rows from {at}")
+        xs.free()
+    for b in (wb, xb, ob, part):
+        b.free()
