@@ -359,9 +359,12 @@ __global__ __launch_bounds__(64 * MM_WAVES) void k_matmul(const MatmulParams p) 
 // In the affine form, group g of weight row r is w = a q + b, q a small integer; so
 // sum_k w x = a sum q x + b sum x. The MFMAs compute sum q x with x split into two f16 parts:
 // a unit of 256 columns of an input row is scaled by a power of two s that puts its largest
-// |x| in [2^14, 2^15), hi = f16(x s), lo = f16(x s - hi): 22 bits of every x within 2^-17 of
-// the unit's largest and an absolute error below 2^-39 of it for the rest, each product
-// exact in f32, f32-level sums. A unit's hi and lo sums meet at its end.
+// |x| in [2^14, 2^15), hi = f16(x s), lo = f16((x s - hi) 2^12): 22 bits of every x within 2^-29
+// of the unit's largest and an absolute error below 2^-51 of it for the rest (with lo unscaled
+// 2^-17 and 2^-39: columns 1e6 below others that met weights of 0 were 4e-7 off, so 1.1e-7), each
+// product exact in f32, f32-level sums. A unit's hi and lo sums meet at its end, the lo sum
+// times 2^-12. (Q6K, whose MFMAs add both, keeps lo unscaled: weights times 2^-12 over lo cost
+// its tile kernel 4%, and its vector-unit pass lost more in such columns, 4e-3.)
 //
 // k_matmul_mm: a workgroup is W waves of 16 weight rows, eight input rows and a K range of
 // at most MM_K units. The range's x is staged once in LDS as 16 A rows: rows 0 .. 7 the eight
@@ -380,7 +383,7 @@ __global__ __launch_bounds__(64 * MM_WAVES) void k_matmul(const MatmulParams p) 
 //   T_hi, T_lo = the MFMAs of a group over hi and over lo (Q4K, Q5K, F16: chained over the
 //   unit's groups; Q6K: one T of a half, hi and lo in one MFMA)
 //   t_hi += a T_hi, t_lo += a T_lo per group, zeroed each unit (Q4K, Q5K, F16: t = T)
-//   t = t_hi + t_lo (Q6K: t += a T per half)
+//   t = t_hi + 2^-12 t_lo, one FMA (Q6K: t += a T per half)
 //   t = d t (Q4K, Q5K), then t += the unit's b sum x terms; p += t / s per unit
 //   out = the K splits' p added in split order.
 // The b sum x terms (Q4_1, Q5_1: m; Q4K, Q5K: -dmin m_j) are one more MFMA a unit: A = the
@@ -643,13 +646,17 @@ __device__ __forceinline__ float group_sum(const float (&x)[4]) {
     return sg;
 }
 // Four columns' hi and lo parts, scaled, in the order of e (x s is exact, so lo's FMA gives
-// x s - hi).
+// x s - hi, at most 8).
+constexpr float MM_LO = 4096.0f, MM_LO_INV = 1.0f / 4096.0f;
+template <bool SCALED>
 __device__ __forceinline__ void hi_lo(const float (&x)[4], float s, half4& h, half4& l) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int e = 0; e < 4; e += 2) {
         const half2 hv = __builtin_convertvector((f32x2{x[e] * s, x[e + 1] * s}), half2);
-        const half2 lv = __builtin_convertvector((f32x2{__builtin_fmaf(x[e], s, -(float)hv[0]), __builtin_fmaf(x[e + 1], s, -(float)hv[1])}), half2);
+        const float k = SCALED ? MM_LO : 1.0f;
+        const half2 lv = __builtin_convertvector((f32x2{k * __builtin_fmaf(x[e], s, -(float)hv[0]),
+                                                        k * __builtin_fmaf(x[e + 1], s, -(float)hv[1])}), half2);
         h[e] = hv[0]; h[e + 1] = hv[1];
         l[e] = lv[0]; l[e + 1] = lv[1];
     }
@@ -873,7 +880,7 @@ __global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_
                     }
                     const float xs4[4] = {x4[0], KP ? x4[2] : x4[1], KP ? x4[1] : x4[2], x4[3]};
                     half4 h, l;
-                    hi_lo(xs4, sc, h, l);
+                    hi_lo<TY != G_Q6K>(xs4, sc, h, l);
                     if constexpr (TY == G_Q6K) {
                         *(half8*)&xs[i * XR + 8 * cq] = __builtin_shufflevector(h, l, 0, 1, 2, 3, 4, 5, 6, 7);
                     } else {
@@ -934,12 +941,13 @@ __global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_
                         }
                         if constexpr (TY != G_Q6K) {  // hi + lo
                             if constexpr (NI == 16) {
-                                t4 += t5;
+#pragma unroll
+                                for (int i = 0; i < 4; i++) t4[i] = __builtin_fmaf(MM_LO_INV, t5[i], t4[i]);
                             } else {
 #pragma unroll
                                 for (int i = 0; i < 4; i++) {
                                     const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(t4[i]), __float_as_uint(t4[i]), false, false);
-                                    t4[i] = __uint_as_float(r2[0]) + __uint_as_float(r2[1]);
+                                    t4[i] = __builtin_fmaf(MM_LO_INV, __uint_as_float(r2[1]), __uint_as_float(r2[0]));
                                 }
                             }
                         }
@@ -1099,7 +1107,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_row(const MMParams p) {
                 }
                 const float xo[4] = {x4[0], x4[2], x4[1], x4[3]};
                 half4 h, o;
-                hi_lo(xo, sc, h, o);
+                hi_lo<TY != G_Q6K>(xo, sc, h, o);
                 if constexpr (TY == G_Q6K) {
                     *(half8*)&xs[w][8 * lane] = __builtin_shufflevector(h, o, 0, 1, 2, 3, 4, 5, 6, 7);
                 } else {
@@ -1139,7 +1147,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_row(const MMParams p) {
                 double sum = s;
                 if constexpr (TY != G_Q6K) {  // hi + lo
                     const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false);
-                    sum = (double)__uint_as_float(r2[0]) + (double)__uint_as_float(r2[1]);
+                    sum = __builtin_fma((double)MM_LO_INV, (double)__uint_as_float(r2[1]), (double)__uint_as_float(r2[0]));
                 }
                 if constexpr (UT) sum *= (double)m.dl;
                 if constexpr (SUM) {
@@ -1218,7 +1226,7 @@ __global__ __launch_bounds__(256) void k_mm_prep(const float* __restrict__ x, f1
     }
     const float xo[4] = {v.x, ORDER ? v.z : v.y, ORDER ? v.y : v.z, v.w};
     half4 h, l;
-    hi_lo(xo, sc, h, l);
+    hi_lo<ORDER != 2>(xo, sc, h, l);
     const uint32_t step = 4 * u + lane / 16, q = lane % 16;
     if (step >= steps) return;
     f16* dst = xp + ((size_t)step * npad + row) * 128;
@@ -1473,7 +1481,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_units(const TLParams p, const
                 }
                 const float xo[4] = {x4[0], UT ? x4[1] : x4[2], UT ? x4[2] : x4[1], x4[3]};
                 half4 h, o;
-                hi_lo(xo, sc, h, o);
+                hi_lo<true>(xo, sc, h, o);
                 *(half4*)&xs[w][i * XS + 4 * lane] = h;
                 *(half4*)&xs[w][(8 + i) * XS + 4 * lane] = o;
             }
@@ -1502,7 +1510,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_units(const TLParams p, const
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[e]), __float_as_uint(t[e]), false, false);
-                t[e] = __uint_as_float(r2[0]) + __uint_as_float(r2[1]);
+                t[e] = __builtin_fmaf(MM_LO_INV, __uint_as_float(r2[1]), __uint_as_float(r2[0]));
             }
             if constexpr (SUM) {
                 const f32x4 tb = mfma16(*(const half8*)&ss[w][(l & 7u) * 32 + 8 * c], *(const half8*)&um[w][8 * l], z4);
@@ -1521,6 +1529,10 @@ __global__ __launch_bounds__(64 * W) void k_matmul_units(const TLParams p, const
     float acc = 0.0f, tot = 0.0f;
     uint32_t kz = 0, kend = p.units / p.ks;
     auto fold = [&](uint32_t u0, uint32_t ue) {
+        if (!LONG && p.ks == 1) {
+            for (uint32_t u = 0; u < ue; u++) tot = __builtin_fmaf(isc[u][i], ps[u][i][tid & 15], tot);
+            return;
+        }
         for (uint32_t u = u0; u < ue; u++) {
             acc = __builtin_fmaf(isc[u - u0][i], ps[u - u0][i][tid & 15], acc);
             if (u + 1 < kend) continue;
@@ -1731,7 +1743,9 @@ __global__ __launch_bounds__(TL_THREADS, 2) void k_matmul_tile(const TLParams p)
 #pragma unroll
                         for (int j = 0; j < TN; j++) {
                             f32x4 v = t[i][j];
-                            if constexpr (TY != G_Q6K) v += to[i][j];
+                            if constexpr (TY != G_Q6K)
+#pragma unroll
+                                for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf(MM_LO_INV, to[i][j][e], v[e]);
                             if constexpr (KQ) v *= dl[j];
                             if constexpr (SUM) {
                                 const f32x4 tb = mfma16(sv, mv[j], z4);
