@@ -387,7 +387,9 @@ __global__ __launch_bounds__(64 * MM_WAVES) void k_matmul(const MatmulParams p) 
 //   t = d t (Q4K, Q5K), then t += the unit's b sum x terms; p += t / s per unit
 //   out = the K splits' p added in split order.
 // The b sum x terms (Q4_1, Q5_1: m; Q4K, Q5K: -dmin m_j) are one more MFMA a unit: A = the
-// eight groups' sums of x s / 32 in three f16 parts (33 bits), B = the m's three times over.
+// eight groups' sums of (hi + lo) / 32 in three f16 parts (33 bits), B = the m's three times over
+// (Q4K, Q5K: the last two parts times 2^12 over m 2^-12, a floor of 2^-52 of the unit's largest
+// |x|, else 2^-40: small groups beside columns 1e6 larger, 2.5e-6 off without).
 // The units' bytes are loaded MM_PF units ahead. K splits: their number depends on rows and
 // cols only; one workgroup runs the splits one after another or ks workgroups run them at
 // once and the last to finish (a device counter per tile) adds them: an input row's bits
@@ -637,14 +639,6 @@ __device__ __forceinline__ void unit_scale(const float (&x)[4], float& s, float&
     s = e == 255u ? 1.0f : __uint_as_float((268u - e) << 23);
     inv = e == 255u ? 1.0f : __uint_as_float((e - 14u) << 23);
 }
-// The sum of a group of 32 columns over its 8 lanes.
-__device__ __forceinline__ float group_sum(const float (&x)[4]) {
-    float sg = ((x[0] + x[1]) + x[2]) + x[3];
-    sg += __shfl_xor(sg, 1, 64);
-    sg += __shfl_xor(sg, 2, 64);
-    sg += __shfl_xor(sg, 4, 64);
-    return sg;
-}
 // Four columns' hi and lo parts, scaled, in the order of e (x s is exact, so lo's FMA gives
 // x s - hi, at most 8).
 constexpr float MM_LO = 4096.0f, MM_LO_INV = 1.0f / 4096.0f;
@@ -661,14 +655,28 @@ __device__ __forceinline__ void hi_lo(const float (&x)[4], float s, half4& h, ha
         l[e] = lv[0]; l[e + 1] = lv[1];
     }
 }
-// A group's sum of x s / 32 in three parts.
-__device__ __forceinline__ void sum_parts(float sg, float s, f16 (&p)[3]) {
-    float r = sg * (s * 0.03125f);
+// The sum of a group of 32 columns over its 8 lanes, of hi + lo as they are: what x lost then meets
+// a weight a q + b, not a q alone.
+__device__ __forceinline__ float group_sum(half4 h, half4 l) {
+    float x[4];
 #pragma unroll
-    for (int e = 0; e < 3; e++) {
-        p[e] = (f16)r;
-        r -= (float)p[e];
-    }
+    for (int e = 0; e < 4; e++) x[e] = __builtin_fmaf(MM_LO_INV, (float)l[e], (float)h[e]);
+    float sg = ((x[0] + x[1]) + x[2]) + x[3];
+    // DPP moves (lanes i ^ 1, i ^ 2, 7 - i of eight): no LDS.
+    sg += __uint_as_float(__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(sg), 0xb1, 0xf, 0xf, false));
+    sg += __uint_as_float(__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(sg), 0x4e, 0xf, 0xf, false));
+    sg += __uint_as_float(__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(sg), 0x141, 0xf, 0xf, false));
+    return sg;
+}
+// A group's sum of x s / 32 in three parts; SCALED (K-quants, whose m's are small integers): the
+// last two times 2^12, over m's times 2^-12.
+template <bool SCALED>
+__device__ __forceinline__ void sum_parts(float sg, f16 (&p)[3]) {
+    float r = sg * 0.03125f;
+    p[0] = (f16)r;
+    r = (r - (float)p[0]) * (SCALED ? MM_LO : 1.0f);
+    p[1] = (f16)r;
+    p[2] = (f16)(r - (float)p[1]);
 }
 // What a unit's groups share: the scale factors and packed scale bytes (K-quants), the b
 // factor over x's scale and the eight groups' m's as f16.
@@ -676,11 +684,13 @@ struct MMUnit {
     float dl = 0.0f, bl = 0.0f;
     uint32_t scA = 0, scB = 0, mnA = 0, mnB = 0;
 };
-// The m bytes of a unit (K-quants) as f16 values, in group order.
-__device__ __forceinline__ half8 mins_f16(uint32_t a, uint32_t b) {
-    const half2 o = half2{(f16)1024.0f, (f16)1024.0f};
+// The m bytes of a unit (K-quants) as f16 values times k, in group order: (1024 + m) k - 1024 k,
+// exact for the k of lane c's part of the sums (1, or 2^-12 for the second and third).
+__device__ __forceinline__ f16 mins_scale(uint32_t c) { return c == 0 ? (f16)1.0f : (f16)MM_LO_INV; }
+__device__ __forceinline__ half8 mins_f16(uint32_t a, uint32_t b, f16 k) {
+    const half2 k2 = half2{k, k}, o = k2 * half2{(f16)-1024.0f, (f16)-1024.0f};
     auto two = [&](uint32_t v, uint32_t sel) {
-        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2, __builtin_amdgcn_perm(0x64646464u, v, sel)) - o);
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(half2, __builtin_amdgcn_perm(0x64646464u, v, sel)), k2, o));
     };
     return __builtin_bit_cast(half8, u32x4{two(a, 0x04010400u), two(a, 0x04030402u), two(b, 0x04010400u), two(b, 0x04030402u)});
 }
@@ -830,6 +840,7 @@ __global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_
     const uint32_t c = lane >> 4, rl = lane & 15;
     const uint32_t r0 = blockIdx.x * (16 * W) + 16 * w, r = r0 + rl, i0 = blockIdx.y * NI;
     const bool live = r0 < p.rows;  // the wave has rows
+    const f16 mk = mins_scale(c);
     // the rows a lane loads: its matrix-core row (mrowp), or (KQ) its lane quad's
     const uint8_t* mrowp = p.w + (size_t)min(r, p.rows - 1) * p.row_bytes;
     const uint8_t* rowp = KQ ? p.w + (size_t)min(r0 + (lane >> 2), p.rows - 1) * p.row_bytes : mrowp;
@@ -869,18 +880,18 @@ __global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_
                     float sc, inv;
                     unit_scale(x4, sc, inv);
                     if (lane == 0) isc[lu * NI + i] = inv;
+                    const float xs4[4] = {x4[0], KP ? x4[2] : x4[1], KP ? x4[1] : x4[2], x4[3]};
+                    half4 h, l;
+                    hi_lo<TY != G_Q6K>(xs4, sc, h, l);
                     if constexpr (SUM) {
-                        const float sg = group_sum(x4);
+                        const float sg = group_sum(h, l);
                         if ((lane & 7) == 0) {
                             f16 sp[3];
-                            sum_parts(sg, sc, sp);
+                            sum_parts<TY == G_Q4K || TY == G_Q5K>(sg, sp);
 #pragma unroll
                             for (int e = 0; e < 3; e++) ss[(lu * NI + i) * 32 + 8 * e + lane / 8] = sp[e];
                         }
                     }
-                    const float xs4[4] = {x4[0], KP ? x4[2] : x4[1], KP ? x4[1] : x4[2], x4[3]};
-                    half4 h, l;
-                    hi_lo<TY != G_Q6K>(xs4, sc, h, l);
                     if constexpr (TY == G_Q6K) {
                         *(half8*)&xs[i * XR + 8 * cq] = __builtin_shufflevector(h, l, 0, 1, 2, 3, 4, 5, 6, 7);
                     } else {
@@ -956,7 +967,7 @@ __global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_
                         if constexpr (TY == G_Q4K || TY == G_Q5K) t4 *= m.dl;
                         if constexpr (SUM) {
                             half8 mv;
-                            if constexpr (TY == G_Q4K || TY == G_Q5K) mv = mins_f16(m.mnA, m.mnB);
+                            if constexpr (TY == G_Q4K || TY == G_Q5K) mv = mins_f16(m.mnA, m.mnB, mk);
                             else mv = __builtin_bit_cast(half8, u32x4{dd[0], dd[1], dd[2], dd[3]});
                             const f32x4 tb = mfma16(*(const half8*)&ss[(lu * NI + ra) * 32 + 8 * c], mv, z4);
 #pragma unroll
@@ -1070,6 +1081,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_row(const MMParams p) {
     const uint8_t* mrow = p.w + (size_t)min(r0 + rl, p.rows - 1) * p.row_bytes;
     const uint8_t* qrow = p.w + (size_t)min(r0 + (lane >> 2), p.rows - 1) * p.row_bytes;
     uint8_t* wt = wtb[w];
+    const f16 mk = mins_scale(c);
     // LDS written and read by one wave only: in order, no barrier.
     auto own = [&]() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
     if constexpr (SUM)
@@ -1096,18 +1108,18 @@ __global__ __launch_bounds__(64 * W) void k_matmul_row(const MMParams p) {
                 float sc, inv;
                 unit_scale(x4, sc, inv);
                 if (lane == 0) isc[u] = inv;
+                const float xo[4] = {x4[0], x4[2], x4[1], x4[3]};
+                half4 h, o;
+                hi_lo<TY != G_Q6K>(xo, sc, h, o);
                 if constexpr (SUM) {
-                    const float sg = group_sum(x4);
+                    const float sg = group_sum(h, o);
                     if ((lane & 7) == 0) {
                         f16 sp[3];
-                        sum_parts(sg, sc, sp);
+                        sum_parts<UT>(sg, sp);
 #pragma unroll
                         for (int e = 0; e < 3; e++) ss[w][8 * e + lane / 8] = sp[e];
                     }
                 }
-                const float xo[4] = {x4[0], x4[2], x4[1], x4[3]};
-                half4 h, o;
-                hi_lo<TY != G_Q6K>(xo, sc, h, o);
                 if constexpr (TY == G_Q6K) {
                     *(half8*)&xs[w][8 * lane] = __builtin_shufflevector(h, o, 0, 1, 2, 3, 4, 5, 6, 7);
                 } else {
@@ -1152,7 +1164,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_row(const MMParams p) {
                 if constexpr (UT) sum *= (double)m.dl;
                 if constexpr (SUM) {
                     half8 mv;
-                    if constexpr (UT) mv = mins_f16(m.mnA, m.mnB);
+                    if constexpr (UT) mv = mins_f16(m.mnA, m.mnB, mk);
                     else mv = __builtin_bit_cast(half8, u32x4{dd[0], dd[1], dd[2], dd[3]});
                     sum = __builtin_fma((double)m.bl, (double)mfma16(*(const half8*)&ss[w][8 * c], mv, z4)[0], sum);
                 }
@@ -1200,9 +1212,9 @@ constexpr int tl_order() {
 }
 
 // Prepared x of one unit of one input row, a wave: per step 256 bytes, hi of its 64 columns
-// then lo (order 2: 16-byte pieces of four columns' hi and lo); the inverse scale; (SUM) the
-// A operand of the b sum x terms. Rows past n and columns past cols are zeros.
-template <int ORDER, bool SUM>
+// then lo (order 2: 16-byte pieces of four columns' hi and lo); the inverse scale; (SUM: 1, or 2
+// for the K-quants) the A operand of the b sum x terms. Rows past n and columns past cols are zeros.
+template <int ORDER, int SUM>
 __global__ __launch_bounds__(256) void k_mm_prep(const float* __restrict__ x, f16* __restrict__ xp,
                                                  float* __restrict__ ip, f16* __restrict__ sp, uint32_t n,
                                                  uint32_t cols, uint32_t npad, uint32_t steps) {
@@ -1215,18 +1227,18 @@ __global__ __launch_bounds__(256) void k_mm_prep(const float* __restrict__ x, f1
     unit_scale(x4, sc, inv);
     const size_t at = (size_t)u * npad + row;
     if (lane == 0) ip[at] = inv;
-    if constexpr (SUM) {
-        const float sg = group_sum(x4);
+    const float xo[4] = {v.x, ORDER ? v.z : v.y, ORDER ? v.y : v.z, v.w};
+    half4 h, l;
+    hi_lo<ORDER != 2>(xo, sc, h, l);
+    if constexpr (SUM != 0) {
+        const float sg = group_sum(h, l);
         if ((lane & 7u) == 0) {
             f16 p[3];
-            sum_parts(sg, sc, p);
+            sum_parts<SUM == 2>(sg, p);
 #pragma unroll
             for (int e = 0; e < 4; e++) sp[at * 32 + 8 * e + lane / 8] = e < 3 ? p[e] : (f16)0.0f;
         }
     }
-    const float xo[4] = {v.x, ORDER ? v.z : v.y, ORDER ? v.y : v.z, v.w};
-    half4 h, l;
-    hi_lo<ORDER != 2>(xo, sc, h, l);
     const uint32_t step = 4 * u + lane / 16, q = lane % 16;
     if (step >= steps) return;
     f16* dst = xp + ((size_t)step * npad + row) * 128;
@@ -1335,7 +1347,8 @@ __device__ __forceinline__ void tl_stash(const uint32_t (&d)[TLP<TY>], const uin
             const uint32_t dd[MWD<TY>] = {h[0], h[1], h[2], h[3]};
             m = mm_unit<TY>(dd);
             if (qd == 0) *(float2*)(uf + 2 * r) = float2{m.dl, m.bl};
-            if (qd == 1) *(half8*)(um + 8 * r) = mins_f16(m.mnA, m.mnB);
+            // (the m's over the sums' first part, then over the other two)
+            if (qd & 1) *(half8*)(um + 8 * (r + (qd & 2u ? NT : 0))) = mins_f16(m.mnA, m.mnB, mins_scale(qd & 2u));
         }
 #pragma unroll
         for (uint32_t hi = 0; hi < 2; hi++) {
@@ -1470,18 +1483,18 @@ __global__ __launch_bounds__(64 * W) void k_matmul_units(const TLParams p, const
                 float sc, inv;
                 unit_scale(x4, sc, inv);
                 if (lane == 0) isc[u - u0][i] = inv;
+                const float xo[4] = {x4[0], UT ? x4[1] : x4[2], UT ? x4[2] : x4[1], x4[3]};
+                half4 h, o;
+                hi_lo<true>(xo, sc, h, o);
                 if constexpr (SUM) {
-                    const float sg = group_sum(x4);
+                    const float sg = group_sum(h, o);
                     if ((lane & 7) == 0) {
                         f16 sp[3];
-                        sum_parts(sg, sc, sp);
+                        sum_parts<false>(sg, sp);
 #pragma unroll
                         for (int e = 0; e < 3; e++) ss[w][i * 32 + 8 * e + lane / 8] = sp[e];
                     }
                 }
-                const float xo[4] = {x4[0], UT ? x4[1] : x4[2], UT ? x4[2] : x4[1], x4[3]};
-                half4 h, o;
-                hi_lo<true>(xo, sc, h, o);
                 *(half4*)&xs[w][i * XS + 4 * lane] = h;
                 *(half4*)&xs[w][(8 + i) * XS + 4 * lane] = o;
             }
@@ -1573,7 +1586,7 @@ __global__ __launch_bounds__(TL_THREADS, 2) void k_matmul_tile(const TLParams p)
     __shared__ __attribute__((aligned(16))) float is[2][MT];
     __shared__ float sa[2][UT ? 1 : (TY == G_Q6K ? 4 : 2) * TL_NT];
     __shared__ __attribute__((aligned(16))) float uf[2][KQ ? 2 * TL_NT : 1];
-    __shared__ __attribute__((aligned(16))) f16 um[2][SUM ? 8 * TL_NT : 1];
+    __shared__ __attribute__((aligned(16))) f16 um[2][SUM ? 8 * (KQ ? 2 : 1) * TL_NT : 1];
     __shared__ __attribute__((aligned(16))) f16 us[2][SUM ? 32 * MT : 1];
     __shared__ uint32_t last;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1730,7 +1743,7 @@ __global__ __launch_bounds__(TL_THREADS, 2) void k_matmul_tile(const TLParams p)
                             dl[j] = f.x;
                             bl[j] = f.y;
                         }
-                        if constexpr (SUM) mv[j] = *(const half8*)(um[ub] + 8 * r);
+                        if constexpr (SUM) mv[j] = *(const half8*)(um[ub] + 8 * (KQ && c != 0 ? r + TL_NT : r));
                     }
 #pragma unroll
                     for (int i = 0; i < TM; i++) {
@@ -1984,7 +1997,7 @@ static hipError_t matmul_tile_go(const MatmulParams& mp, void* scratch, uint32_t
     float* part = (float*)((char*)sp + t.sp_bytes);
     for (uint32_t n0 = 0; n0 < mp.n; n0 += t.slab) {
         const uint32_t m = min(mp.n - n0, t.slab), nyt = (m + t.mt - 1) / t.mt, npad = nyt * t.mt;
-        hipLaunchKernelGGL((k_mm_prep<tl_order<TY>(), mm_sum<TY>()>), dim3(t.units, npad / 4), dim3(256), 0, s,
+        hipLaunchKernelGGL((k_mm_prep<tl_order<TY>(), tl_kq<TY>() ? 2 : mm_sum<TY>() ? 1 : 0>), dim3(t.units, npad / 4), dim3(256), 0, s,
                            mp.x + (size_t)n0 * mp.cols, xp, ip, sp, m, mp.cols, npad, (t.groups + 1) / 2);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
