@@ -411,6 +411,12 @@ constexpr bool mm_type() {
     return TY == G_F16 || TY == G_Q8_0 || TY == G_Q4_0 || TY == G_Q4_1 || TY == G_Q5_0 || TY == G_Q5_1 ||
            TY == G_Q4K || TY == G_Q5K || TY == G_Q6K;
 }
+// x's order: 0 as it is (F16), 1 in pairs (0, 2, 1, 3 of each four), 2 the same
+// with hi and lo of each four columns together (Q6K).
+template <uint32_t TY>
+constexpr int tl_order() {
+    return TY == G_F16 ? 0 : TY == G_Q6K ? 2 : 1;
+}
 // Formats with b sum x terms.
 template <uint32_t TY>
 constexpr bool mm_sum() {
@@ -629,28 +635,31 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
     return max(r32[0], r32[1]);
 }
 // The power of two that puts the largest |x| of a unit (four columns a lane) in [2^14, 2^15),
-// and its inverse; 1 where that is no finite number (an infinity or NaN in x stays one).
-// Units below 2^-112 take 2^126 (a zero stays zero). Bits of |x| compare as |x| does.
+// and its inverse; an infinity or NaN in x stays one, and its unit takes the scale of the largest
+// finite numbers. Units below 2^-112 take 2^126 (a zero stays zero). Bits of |x| compare as |x| does.
 __device__ __forceinline__ void unit_scale(const float (&x)[4], float& s, float& inv) {
     uint32_t m = 0;
 #pragma unroll
     for (int e = 0; e < 4; e++) m = max(m, __float_as_uint(x[e]) & 0x7fffffffu);
-    const uint32_t e = max(__builtin_amdgcn_readfirstlane(wave_max_u32(m)) >> 23, 15u);
-    s = e == 255u ? 1.0f : __uint_as_float((268u - e) << 23);
-    inv = e == 255u ? 1.0f : __uint_as_float((e - 14u) << 23);
+    const uint32_t e = min(max(__builtin_amdgcn_readfirstlane(wave_max_u32(m)) >> 23, 15u), 254u);
+    s = __uint_as_float((268u - e) << 23);
+    inv = __uint_as_float((e - 14u) << 23);
 }
 // Four columns' hi and lo parts, scaled, in the order of e (x s is exact, so lo's FMA gives
-// x s - hi, at most 8).
+// x s - hi, at most 8). ORDER: tl_order. F16 weights: lo of an infinite x is finite, not
+// inf - inf, so the products are IEEE's, as over one row; the block formats' are NaN.
 constexpr float MM_LO = 4096.0f, MM_LO_INV = 1.0f / 4096.0f;
-template <bool SCALED>
+template <int ORDER>
 __device__ __forceinline__ void hi_lo(const float (&x)[4], float s, half4& h, half4& l) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int e = 0; e < 4; e += 2) {
         const half2 hv = __builtin_convertvector((f32x2{x[e] * s, x[e + 1] * s}), half2);
-        const float k = SCALED ? MM_LO : 1.0f;
-        const half2 lv = __builtin_convertvector((f32x2{k * __builtin_fmaf(x[e], s, -(float)hv[0]),
-                                                        k * __builtin_fmaf(x[e + 1], s, -(float)hv[1])}), half2);
+        const float k = ORDER == 2 ? 1.0f : MM_LO;
+        float r[2] = {k * __builtin_fmaf(x[e], s, -(float)hv[0]), k * __builtin_fmaf(x[e + 1], s, -(float)hv[1])};
+        if constexpr (ORDER == 0)  // (of NaN, med3 gives a bound)
+            for (float& v : r) v = __builtin_amdgcn_fmed3f(v, -8.0f * MM_LO, 8.0f * MM_LO);
+        const half2 lv = __builtin_convertvector((f32x2{r[0], r[1]}), half2);
         h[e] = hv[0]; h[e + 1] = hv[1];
         l[e] = lv[0]; l[e + 1] = lv[1];
     }
@@ -882,7 +891,7 @@ __global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_
                     if (lane == 0) isc[lu * NI + i] = inv;
                     const float xs4[4] = {x4[0], KP ? x4[2] : x4[1], KP ? x4[1] : x4[2], x4[3]};
                     half4 h, l;
-                    hi_lo<TY != G_Q6K>(xs4, sc, h, l);
+                    hi_lo<tl_order<TY>()>(xs4, sc, h, l);
                     if constexpr (SUM) {
                         const float sg = group_sum(h, l);
                         if ((lane & 7) == 0) {
@@ -1110,7 +1119,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_row(const MMParams p) {
                 if (lane == 0) isc[u] = inv;
                 const float xo[4] = {x4[0], x4[2], x4[1], x4[3]};
                 half4 h, o;
-                hi_lo<TY != G_Q6K>(xo, sc, h, o);
+                hi_lo<tl_order<TY>()>(xo, sc, h, o);
                 if constexpr (SUM) {
                     const float sg = group_sum(h, o);
                     if ((lane & 7) == 0) {
@@ -1204,12 +1213,6 @@ template <uint32_t TY>
 constexpr bool tl_kq() {
     return TY == G_Q4K || TY == G_Q5K;
 }
-// x's order: 0 as it is (F16), 1 k_matmul_mm's pairs (0, 2, 1, 3 of each four), 2 the same
-// with hi and lo of each four columns together (Q6K).
-template <uint32_t TY>
-constexpr int tl_order() {
-    return TY == G_F16 ? 0 : TY == G_Q6K ? 2 : 1;
-}
 
 // Prepared x of one unit of one input row, a wave: per step 256 bytes, hi of its 64 columns
 // then lo (order 2: 16-byte pieces of four columns' hi and lo); the inverse scale; (SUM: 1, or 2
@@ -1229,7 +1232,7 @@ __global__ __launch_bounds__(256) void k_mm_prep(const float* __restrict__ x, f1
     if (lane == 0) ip[at] = inv;
     const float xo[4] = {v.x, ORDER ? v.z : v.y, ORDER ? v.y : v.z, v.w};
     half4 h, l;
-    hi_lo<ORDER != 2>(xo, sc, h, l);
+    hi_lo<ORDER>(xo, sc, h, l);
     if constexpr (SUM != 0) {
         const float sg = group_sum(h, l);
         if ((lane & 7u) == 0) {
@@ -1485,7 +1488,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_units(const TLParams p, const
                 if (lane == 0) isc[u - u0][i] = inv;
                 const float xo[4] = {x4[0], UT ? x4[1] : x4[2], UT ? x4[2] : x4[1], x4[3]};
                 half4 h, o;
-                hi_lo<true>(xo, sc, h, o);
+                hi_lo<tl_order<TY>()>(xo, sc, h, o);
                 if constexpr (SUM) {
                     const float sg = group_sum(h, o);
                     if ((lane & 7) == 0) {
