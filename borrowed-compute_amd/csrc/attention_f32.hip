@@ -472,8 +472,9 @@ __global__ __launch_bounds__(F32_THREADS, HD <= 128 ? 2 : 1) void attn_f32_line(
     for (int k = 0; k < NH * VC; k++) o[k] = R[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     auto block = [&](F32Stage<HD>& st, F32Stage<HD>& next, uint32_t key0) {
-        // This stage's loads are in for everyone, and everyone is done with the other's.
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        // This stage's loads are in for everyone, and everyone's reads of the other are done (lgkmcnt:
+        // nothing else keeps their last use before the barrier, behind which the loads below go out).
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         const bool mine = key0 < wlen;
         f32x4 a0;
         if (mine) a0 = st.k[n][g ^ (n & 7u)];  // before the loads below: it would wait for them
