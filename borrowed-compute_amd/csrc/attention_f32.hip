@@ -31,6 +31,8 @@
 #include <hip/hip_ext.h>
 #include <math.h>
 
+#include <type_traits>
+
 namespace bchip {
 
 constexpr int F32_BLK = 32;      // list entries per block
@@ -397,11 +399,13 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
 }
 
 // A block of K or V in LDS, 16-byte units: K's unit u of entry e at u ^ (e % 8), so that the eight
-// entries LDS serves together are in eight groups of banks; V's in order.
+// entries LDS serves together are in eight groups of banks; V's in order. The last V row is zeros:
+// what a wave reads for the entries past its tile's lists (another tile's, whose V may be
+// infinite or NaN, which a P of 0 would not silence).
 template <int HD>
 struct F32Stage {
     f32x4 k[F32_BLK][HD / 4];
-    f32x4 v[F32_BLK][HD / 4];
+    f32x4 v[F32_BLK + 1][HD / 4];
 };
 
 // Bound: the matrix cores (777 rows at 300, llama-8B heads: 8.8 GFLOP in 127 us, 361 with VALU
@@ -459,6 +463,7 @@ __global__ __launch_bounds__(F32_THREADS, HD <= 128 ? 2 : 1) void attn_f32_line(
         }
     };
     load(st0, 0);
+    if (tid < (uint32_t)UN) st0.v[F32_BLK][tid] = st1.v[F32_BLK][tid] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     f32x4 qx[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
@@ -495,16 +500,26 @@ __global__ __launch_bounds__(F32_THREADS, HD <= 128 ? 2 : 1) void attn_f32_line(
         }
         const float cr = softmax_block(s, m, l);
         f32x4 acc[NH * VC] = {};
+        const uint32_t left = wlen - key0;
+        auto pv = [&](auto whole) {
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t e = 16 * t + 4 * g + i, row = whole || e < left ? e : (uint32_t)F32_BLK;
 #pragma unroll
-                for (int h = 0; h < NH; h++) {
-                    const vvec v = *((const vvec*)&st.v[16 * t + 4 * g + i][0] + 16 * h + n);
+                    for (int h = 0; h < NH; h++) {
+                        const vvec v = *((const vvec*)&st.v[row][0] + 16 * h + n);
 #pragma unroll
-                    for (int k = 0; k < VC; k++) acc[VC * h + k] = mfma4(vec_at(v, k), s[t][i], acc[VC * h + k]);
+                        for (int k = 0; k < VC; k++) acc[VC * h + k] = mfma4(vec_at(v, k), s[t][i], acc[VC * h + k]);
+                    }
                 }
+        };
+        // (two copies: the select in every block cost 2%)
+        if (left >= (uint32_t)F32_BLK)
+            pv(std::true_type{});
+        else
+            pv(std::false_type{});
 #pragma unroll
         for (int k = 0; k < NH * VC; k++)
 #pragma unroll

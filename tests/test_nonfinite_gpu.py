@@ -89,3 +89,24 @@ def test_a_non_finite_input_reaches_only_its_own_outputs(ctx, rows, pos, nh, nkv
     np.testing.assert_array_equal(planted[keep].view(np.uint32), clean[keep].view(np.uint32),
                                   err_msg=f"{what}: an output that does not read the planted value moved")
     assert may.any()
+
+
+# Over f32 caches the two forms (below and at 512 tiles of 16 query slots) let an unseen V element
+# reach the rows of its own tile only: a tile's list ends with its last row. (rows, nh, nkv, hd)
+@pytest.mark.parametrize("rows,nh,nkv,hd", [(200, 32, 8, 128), (300, 32, 8, 128), (1040, 8, 8, 64), (600, 16, 1, 32),
+                                            (400, 28, 4, 80), (1030, 8, 8, 256)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_an_unseen_f32_v_element_stays_in_its_tile(ctx, rows, nh, nkv, hd, bad):
+    pos, G = 37, nh // nkv
+    rng = np.random.default_rng(rows)
+    q = rng.standard_normal((rows, nh * hd)).astype(np.float32)
+    kc, vc = rng.standard_normal((2, pos + rows, nkv * hd)).astype(np.float32)
+    clean = _run(ctx, q, kc, vc, rows, pos, nh, nkv, hd, bchip.F32)
+    rb = max(1, 16 // G)
+    for row in (rows - 1, rows // 2, 77):  # its slot; it and later rows see it
+        planted = vc.copy()
+        planted[pos + row, (nkv - 1) * hd + 5] = bad
+        out = _run(ctx, q, kc, planted, rows, pos, nh, nkv, hd, bchip.F32)
+        first = row // rb * rb
+        np.testing.assert_array_equal(out[:first].view(np.uint32), clean[:first].view(np.uint32), err_msg=f"row {row}")
+        assert not np.isfinite(out[row:, (nkv - 1) * G:, 5]).any()
