@@ -1951,11 +1951,17 @@ static hipError_t matmul_mm_go(const MatmulParams& mp, void* scratch, uint32_t* 
     const bool par = scratch && counters && mm_par(TY, mp.rows, mp.cols, mp.n);  // (else in turn: the same bits)
     const MMParams q{mp.w, mp.x, mp.out, (float*)scratch, counters, mp.rows, mp.cols, mp.n, (mp.n + 15) / 16 * 16,
                      mp.row_bytes, mp.cols / 256, ks, par ? 1u : 0u};
-    // Sixteen inputs a workgroup for one such block over a matrix large enough to fill the GPU with
-    // half the workgroups (Q6K 4096 x 14336 at 16 rows: 29 us against 31; Q8_0 896 x 4864 at 17:
-    // 16 against 12). F16's x of 16 inputs would take most of the LDS.
-    if constexpr (TY != G_F16) {
-        if (mp.n > 8 && mp.n <= 16 && (uint64_t)mp.rows * mp.cols >= (1u << 23)) {
+    // Sixteen inputs a workgroup (9 to 16 rows) halve the unpacking but leave one workgroup a CU, so
+    // they pay where a split holds several units, the sooner the dearer the unpacking; us at 9 / 16
+    // rows with eight and with sixteen: 14336 x 4096 (four units) Q6K 32.1 / 33.3 and 26.6 / 28.3, Q8_0
+    // 28.4 / 29.1 and 25.6 / 26.8, Q5K 25.4 / 26.5 and 22.9 / 24.8; 4096 x 4096 (one) 15.7 / 15.9 and
+    // 15.8 / 16.4, 15.0 / 15.2 and 15.7 / 16.4, 14.1 / 14.8 and 14.8 / 15.8. Q4K only where the
+    // workgroups also go around the CUs four times: 28672 x 8192 71 / 75 and 65 / 71, 4096 x 14336 21.4 /
+    // 21.9 and 21.4 / 23.2. Q4_0, Q4_1 and Q5_1 lost or gained nothing. (F16's x of 16 inputs would
+    // take most of the LDS.)
+    constexpr uint32_t MIN_UNITS = TY == G_Q6K ? 2 : TY == G_Q8_0 || TY == G_Q5_0 || TY == G_Q4K || TY == G_Q5K ? 3 : 0;
+    if constexpr (MIN_UNITS > 0) {
+        if (mp.n > 8 && mp.n <= 16 && q.units >= MIN_UNITS * ks && (TY != G_Q4K || rt * ks >= 1024)) {
             const dim3 grid(rt, (mp.n + 15) / 16, par ? ks : 1);
             hipLaunchKernelGGL((k_matmul_mm<TY, 16>), grid, dim3(64 * MM_W<TY>), 0, s, q);
             return hipGetLastError();

@@ -104,3 +104,20 @@ def test_slabs_give_the_small_batches_bits(ctx, ty, rows, cols, n, slab):
         xs.free()
     for b in (wb, xb, ob, part):
         b.free()
+
+
+# k_matmul_mm with sixteen inputs a workgroup (splits of two units or more for Q6K, of three for Q8_0,
+# Q5_0, Q5K and Q4K, the last from 1024 workgroups) and with eight on the other side of its rule.
+@pytest.mark.parametrize("ty,rows,cols", [(O.Q6K, 16300, 2048), (O.Q6K, 16300, 1792), (O.Q8_0, 16300, 3072),
+                                          (O.Q8_0, 16300, 2816), (O.Q5_0, 16300, 3072), (O.Q5K, 16300, 3072),
+                                          (O.Q4K, 32700, 4096), (O.Q4K, 32600, 4096), (O.Q4_0, 16300, 3072)], ids=str)
+def test_batches_of_9_to_16_give_the_bits_of_8(ctx, ty, rows, cols):
+    some = 133
+    data = np.resize(np.asarray(O.random_tensor(ty, some, cols, rows), np.uint8).reshape(some, -1),
+                     (rows, O.row_bytes(ty, cols))).reshape(-1)
+    x = np.random.default_rng(rows).standard_normal((16, cols)).astype(np.float32)
+    first, last, *more = products(ctx, ty, data, rows, cols, [x[:8], x[8:], x, x[:9], x[4:15]])
+    want = np.concatenate((first, last))
+    assert np.isfinite(want).all()
+    for got, (a, b) in zip(more, ((0, 16), (0, 9), (4, 15))):
+        np.testing.assert_array_equal(got, want[a:b], err_msg=f"rows {a}..{b}")
