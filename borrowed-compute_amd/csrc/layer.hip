@@ -1889,13 +1889,6 @@ static bool matmul_uses_mm(uint32_t type, uint32_t cols, uint32_t n) {
     return mm_types(type) && n >= MM_MIN && cols % 256 == 0;
 }
 
-// Which kernel takes a batch of the matrix-core formats; all give an input row the same bits.
-// Batches of 17 rows and 2^29.5 multiply-adds take the tile kernel over k_matmul_mm (Q8_0 896 x
-// 4864 at 67 rows, 0.29 G: 20 us there, 38 here; Q4K 14336 x 4096 at 17, 1.0 G: 31 us there, 26
-// here); with cols no multiple of 256 over k_matmul_units, from 2^27 (Q8_0 4864 x 896 at 16
-// rows, 0.07 G: 9.2 us there, 15.8 here; at 67, 0.29 G: about 35 there, 20 here).
-constexpr uint32_t TL_MIN = 17;
-constexpr uint64_t TL_MACS = 760000000, TL_MACS_RAGGED = 134000000;
 // Bytes of prepared x a launch takes at most, and its input rows (k_mm_prep's grid.y is a quarter of
 // them, of 65535); longer batches go in slabs of input rows.
 constexpr size_t TL_SLAB_BYTES = (size_t)256 << 20, TL_SLAB_ROWS = 4 * 65535;
@@ -1903,13 +1896,6 @@ constexpr size_t TL_SLAB_BYTES = (size_t)256 << 20, TL_SLAB_ROWS = 4 * 65535;
 static bool matmul_uses_units(uint32_t type, uint32_t cols, uint32_t n) {
     return mm_types(type) && cols % 256 != 0 && n >= MM_MIN;
 }
-bool matmul_uses_tile(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n) {
-    const uint64_t macs = (uint64_t)rows * cols * n;
-    if (!mm_types(type)) return false;
-    if (cols % 256 == 0) return n >= TL_MIN && macs >= TL_MACS;
-    return n >= MM_MIN && ((cols + 255) / 256 > WV_UNITS || (n >= TL_MIN && macs >= TL_MACS_RAGGED));
-}
-
 struct TilePlan {
     uint32_t mt, slab, npad, units, groups, ks, nxt, nyt, par;  // npad, nyt, par: of a whole slab
     size_t xp_bytes, ip_bytes, sp_bytes, part_bytes;
@@ -1927,13 +1913,46 @@ static TilePlan tile_plan(uint32_t type, uint32_t rows, uint32_t cols, uint32_t 
     t.npad = (m + t.mt - 1) / t.mt * t.mt;
     t.nyt = t.npad / t.mt;
     t.ks = mm_ks(type, rows, cols);
-    // K splits in parallel where the tiles alone would leave half the CUs without work.
-    t.par = t.ks > 1 && (uint64_t)t.nxt * t.nyt <= 128;
+    // K splits in parallel where the tiles alone would leave half the CUs without work, or, 32 inputs
+    // a workgroup, some of them (18944 x 3584, 148 tiles, at 17 rows: Q4K 39 -> 31 us, Q8_0 59 -> 45).
+    t.par = t.ks > 1 && (uint64_t)t.nxt * t.nyt <= (t.mt == 32 ? 255 : 128);
     t.xp_bytes = (size_t)t.npad * row_bytes;
     t.ip_bytes = ((size_t)t.units * t.npad * sizeof(float) + 255) / 256 * 256;
     t.sp_bytes = (size_t)t.units * t.npad * 64;
     t.part_bytes = t.par ? (size_t)t.ks * t.npad * rows * sizeof(float) : 0;
     return t;
+}
+
+// Which kernel takes a batch of the matrix-core formats; all give an input row the same bits. The
+// tile kernel's work goes by its padded input rows, k_matmul_mm's and k_matmul_units' by eights, so
+// over them it takes batches of 17 rows with enough multiply-adds, by what the unpacking it saves costs,
+// that fill its tiles enough (us there / here):
+//   F16 1024 x 4096 at 33 rows (0.14 G) 28 / 24;
+//   Q8_0, Q6K 4096 x 4096 at 48 rows (0.8 G) 36 / 33 and 38 / 34, at 40 30 / 33 and 33 / 34;
+//   the others 3584 x 3584 at 80 rows (1.0 G) Q4K 41 / 42, at 96 48 / 42; 33 rows in a tile of 64
+//   4096 x 14336 Q4K 44 / 48, 8192 x 8192 45 / 42, but not for a few tiles more than CUs (18944 x 3584 at
+//   65 rows, 296 of them, 89 / 97);
+//   Q4_0, Q5_0 (cheap to unpack) 4096 x 14336 at 64 rows Q4_0 60 / 54, at 80 76 / 90, at 112 105 / 90;
+//   off a multiple of 256 4864 x 896 at 40 rows (0.17 G) Q8_0 15 / 19, at 48 18 / 19, at 56 21 / 19.
+constexpr uint32_t TL_MIN = 17;
+constexpr uint64_t TL_MACS_F16 = 100000000, TL_MACS_8 = 760000000, TL_MACS = 900000000, TL_MACS_4 = 1200000000,
+                   TL_MACS_4_ANY = 5000000000, TL_MACS_RAGGED = 200000000;
+
+bool matmul_uses_tile(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n) {
+    const uint64_t macs = (uint64_t)rows * cols * n;
+    if (!mm_types(type)) return false;
+    if (cols % 256 != 0) return n >= MM_MIN && ((cols + 255) / 256 > WV_UNITS || (n >= TL_MIN && macs >= TL_MACS_RAGGED));
+    if (n < TL_MIN) return false;
+    const TilePlan t = tile_plan(type, rows, cols, n);
+    const uint64_t eights = 100ull * ((min(n, t.slab) + 7) / 8 * 8);  // of npad, in percent
+    const uint32_t tiles = t.nxt * t.nyt;
+    switch (type) {
+        case G_F16: return macs >= TL_MACS_F16;
+        case G_Q4_0: case G_Q5_0: return macs >= TL_MACS_4 && (eights >= 80ull * t.npad || macs >= TL_MACS_4_ANY);
+        default:
+            return macs >= (type == G_Q8_0 || type == G_Q6K ? TL_MACS_8 : TL_MACS) &&
+                   (eights >= 65ull * t.npad || (rows >= 8192 && (tiles <= 256 || tiles > 384)));
+    }
 }
 
 size_t matmul_scratch_bytes(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n, bool tile) {

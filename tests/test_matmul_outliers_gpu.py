@@ -40,9 +40,9 @@ def weights(ty, rows, cols):
 # One row (k_matmul_row), 8 and 16 inputs a workgroup (k_matmul_mm), the tile kernel, and off a
 # multiple of 256 (k_matmul_units, k_matmul_tile; the 32-weight formats and F16).
 BLOCK32 = [O.Q8_0, O.Q4_0, O.Q5_0, O.F16]
-CASES = [(ty, *shape) for shape in ((512, 4096, 1), (512, 256, 1), (512, 4096, 4), (2048, 4096, 12), (2700, 4096, 70))
+CASES = [(ty, *shape) for shape in ((512, 4096, 1), (512, 256, 1), (512, 4096, 4), (2048, 4096, 12), (3100, 4096, 120))
          for ty in BLOCK32 + [O.Q4K, O.Q5K]]
-CASES += [(ty, *shape) for shape in ((512, 896, 4), (2200, 896, 70)) for ty in BLOCK32]
+CASES += [(ty, *shape) for shape in ((512, 896, 4), (2200, 896, 120)) for ty in BLOCK32]
 
 
 @pytest.mark.parametrize("ty,rows,cols,n", CASES, ids=[f"{O.TYPE_NAMES[c[0]]}-{c[1]}-{c[2]}-{c[3]}" for c in CASES])

@@ -34,8 +34,8 @@ def captured(ctx, call):
 # Batches whose K splits would run in parallel (8 and 16 inputs a workgroup), and batches of the
 # tile kernel with 32, 64 and 128 inputs a workgroup.
 @pytest.mark.parametrize("ty", [O.F16, O.Q8_0, O.Q4K, O.Q6K], ids=lambda t: O.TYPE_NAMES[t])
-@pytest.mark.parametrize("rows,cols,n", [(1000, 4096, 3), (4100, 4096, 12), (11650, 4096, 17), (301, 1280, 2000),
-                                         (8300, 1536, 65)])
+@pytest.mark.parametrize("rows,cols,n", [(1000, 4096, 3), (4100, 4096, 12), (13500, 4096, 17), (301, 2048, 2000),
+                                         (8300, 2304, 65), (33000, 512, 200)])
 def test_a_captured_call_without_scratch(ty, rows, cols, n):
     run(ty, rows, cols, n)
 
@@ -43,7 +43,7 @@ def test_a_captured_call_without_scratch(ty, rows, cols, n):
 # Cols off a multiple of 256, on both sides of the 56 units whose sums k_matmul_units holds at
 # once, with one K split, a few and many.
 @pytest.mark.parametrize("ty", [O.F16, O.Q8_0, O.Q4_0, O.Q4_1, O.Q5_0, O.Q5_1], ids=lambda t: O.TYPE_NAMES[t])
-@pytest.mark.parametrize("rows,cols,n", [(4864, 896, 70), (333, 14304, 40), (333, 14368, 40), (65, 29568, 9),
+@pytest.mark.parametrize("rows,cols,n", [(4864, 896, 70), (333, 14304, 60), (333, 14368, 40), (65, 29568, 9),
                                          (20000, 14368, 2), (17, 43040, 33)])
 def test_a_captured_call_off_a_multiple_of_256(ty, rows, cols, n):
     run(ty, rows, cols, n)

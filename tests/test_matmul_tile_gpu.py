@@ -39,11 +39,14 @@ def products(ctx, ty, data, rows, cols, batches):
     return got
 
 
-# rows x cols x n of at least 0.76 G (the tile kernel's threshold): 32 and 64 and 128 input rows a
-# workgroup; K splits in parallel and in turn; one unit, a few, remainders of every size.
+# rows x cols x n above the tile kernel's thresholds (0.1 to 1.2 G by format; the first five reach it
+# for some, the others for all): 32 and 64 and 128 input rows a workgroup; K splits in parallel (up to
+# 128 tiles, 255 of 32 input rows) and in turn; one unit, a few, remainders of every size.
 @pytest.mark.parametrize("ty", TILE_TYPES, ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("rows,cols,n", [(11650, 4096, 17), (5801, 4096, 32), (301, 1280, 2000), (8300, 1536, 65),
-                                         (33000, 256, 100), (32900, 768, 129)])
+                                         (33000, 256, 100), (32900, 768, 129), (9200, 4096, 32), (301, 2048, 2000),
+                                         (8300, 2304, 120), (47000, 256, 100), (32900, 768, 220), (16600, 2560, 31),
+                                         (33000, 1280, 32)])
 def test_tile_gives_the_small_batches_bits(ctx, ty, rows, cols, n):
     # (a block of random rows repeated: random_tensor draws slowly)
     some = 257
@@ -61,8 +64,7 @@ def test_tile_gives_the_small_batches_bits(ctx, ty, rows, cols, n):
 @pytest.mark.parametrize("ty", BLOCK32, ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("rows,cols", [(3, 32), (130, 96), (65, 896), (128, 864), (31, 2080), (17, 4384)])
 def test_cols_off_a_multiple_of_256(ctx, ty, rows, cols):
-    """One launch up to 16 input rows, the tile kernel beyond: a row's bits do not depend on
-    its batch, and its error against the f64 product stays below what its roundings can add
+    """k_matmul_units: a row's bits do not depend on its batch, and its error against the f64 product stays below what its roundings can add
     up to: x in two f16 parts (2^-22 of a term), f32 sums of a group's 32 products in some
     order (32 x 2^-24 of their sizes), two roundings a group and unit after that."""
     n = 70
@@ -82,6 +84,21 @@ def test_cols_off_a_multiple_of_256(ctx, ty, rows, cols):
     err = np.abs(whole - O.matmul_f64(ty, data, rows, cols, x, n))
     print(f"{O.TYPE_NAMES[ty]} {rows}x{cols}: at most {np.max(err / bound):.3g} of the bound", flush=True)
     assert (err <= bound).all()
+
+
+# From 0.2 G multiply-adds off a multiple of 256 the tile kernel: short last units of one and of several
+# steps, odd groups, more units than a split.
+@pytest.mark.parametrize("ty", BLOCK32, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,n", [(4900, 896, 70), (40000, 96, 65), (3100, 2080, 33), (700, 4832, 100)])
+def test_tiles_off_a_multiple_of_256(ctx, ty, rows, cols, n):
+    some = 131
+    data = np.resize(np.asarray(O.random_tensor(ty, some, cols, rows + n), np.uint8).reshape(some, -1),
+                     (rows, O.row_bytes(ty, cols))).reshape(-1)
+    x = np.random.default_rng(cols + n).standard_normal((n, cols)).astype(np.float32)
+    whole, *parts = products(ctx, ty, data, rows, cols, [x, x[:16], x[n - 9:]])
+    np.testing.assert_array_equal(parts[0], whole[:16])
+    np.testing.assert_array_equal(parts[1], whole[n - 9:])
+    assert np.isfinite(whole).all()
 
 
 # Batches of more than one slab of input rows: 256 MiB of prepared x (4608 rows of 14336 columns),
