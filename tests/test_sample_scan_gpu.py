@@ -39,14 +39,15 @@ def masses(scores, temperature):
     return np.add.accumulate(q, dtype=np.float32)
 
 
-@pytest.mark.parametrize("vocab", [2, 1023, 1024, 4096, 4097, 8192, 8193, 16385, 40000])
+@pytest.mark.parametrize("vocab", [1, 2, 511, 513, 1023, 1024, 4096, 4097, 8192, 8193, 16385, 40000])
 @pytest.mark.parametrize("spread", [0.3, 2.0])
 def test_the_nucleus_ends_at_the_token(ctx, vocab, spread):
     rng = np.random.default_rng(vocab)
     row = (rng.standard_normal(vocab) * spread).astype(np.float32)
     mass = masses(row, 0.8)
     scores = np.repeat(row[None], 24, axis=0)
-    for k in {0, min(5, vocab - 1), vocab // 3, vocab // 2}:
+    # (511 and 512: the last candidate whose sums one lane takes, and the first beyond)
+    for k in {0, min(5, vocab - 1), min(511, vocab - 1), min(512, vocab - 1), vocab // 3, vocab // 2}:
         for top_p in (mass[k], np.nextafter(mass[k], np.float32(2))):
             got = ids_of(ctx, scores, 0.8, float(top_p), 99, 7)
             want = [O.sample(row, 0.8, float(top_p), 99, 7 + r) for r in range(24)]
