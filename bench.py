@@ -619,10 +619,10 @@ def main():
             log(json.dumps(extra["verify_loop_70b_256_fused"]))
         if "f32" in want:
             # The drop-in default: an unmodified binding passes the reference's f32 cache
-            # (bchip_rope_append_attention with BCHIP_F32: attn_f32 with the rotation and the append).
+            # (bchip_rope_append_attention with BCHIP_F32: attn_f32_step with the rotation and the append).
             log(f"f32-cache decode (the reference's cache type): configs[1] at {args.ctx} slots, configs[0]")
             r = bench_decode(ctx, hip, args.ctx, 10, 2, kv_type=bchip.F32)
-            r["note"] = "f32 cache, f32 arithmetic (attn_f32): the path an unmodified binding runs"
+            r["note"] = "f32 cache, f32 arithmetic (attn_f32_step): the path an unmodified binding runs"
             extra[f"decode_f32_{args.ctx}"] = r
             log(json.dumps(r))
             r = bench_decode(ctx, hip, 512, args.steps, args.warmup, n_layer=24, nh=14, nkv=2, hd=64, theta=1e6,

@@ -706,7 +706,7 @@ int bchip_rope_append_attention_rows(bchip_ctx* c, float* q, const float* k, con
     CHECK(check_span(c, positions, (uint64_t)rows * 4, "positions"));
     CHECK(check_span(c, inv_freq, (uint64_t)(rope_dim / 2) * 4, "inv_freq"));
     if (kv_type == BCHIP_F32 && rows <= 8) {
-        // f32 caches: attn_f32 rotates q and appends the new rows itself (the two calls' bits).
+        // f32 caches: attn_f32_step rotates q and appends the new rows itself (the two calls' bits).
         const uint64_t limit = std::min(bytes_left(c, kc), bytes_left(c, vc)) / (kvd * esize(kv_type));
         AttnCall a{q, kc, vc, kv_type, out, nullptr, 0u, rows, nh, nkv, hd, pos, scale, limit};
         const RopeArgs r{q, k, v, inv_freq, positions, rope_dim, neox};
@@ -771,7 +771,7 @@ static int fused_step(bchip_ctx* c, Workspace& ws, float* q, const float* k, con
     AttnCall a{q, kc, vc, kv_type, out, nullptr, 0u, 1u, nh, nkv, hd, pos, scale, limit};
     c->take_marks(a);
     if (kv_type == BCHIP_F32) {
-        // f32 caches: attn_f32 rotates q and appends the new row itself (the two calls' bits).
+        // f32 caches: attn_f32_step rotates q and appends the new row itself (the two calls' bits).
         const RopeArgs r{q, k, v, inv_freq, positions, rope_dim, neox};
         HIP_TRY(f32_attention(a, 0, ws, c->stream, &r), "rope_append_attention");
         return BCHIP_OK;

@@ -146,7 +146,8 @@ constexpr uint32_t MATMUL_MAX_N = 8u * 65535u;
 // arrival counters (zero when no product runs).
 constexpr uint32_t MATMUL_COUNTERS = 1024;
 // Larger batches take the tile kernel (tile: matmul_uses_tile), which needs scratch for the
-// prepared input rows. scratch null: the call runs without (tile false, K splits in turn).
+// prepared input rows. scratch null: the call runs without (tile false, K splits in turn), to the
+// same bits.
 bool matmul_uses_tile(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n);
 size_t matmul_scratch_bytes(uint32_t type, uint32_t rows, uint32_t cols, uint32_t n, bool tile);
 hipError_t matmul_launch(const void* w, uint32_t type, const float* x, float* out, uint32_t rows, uint32_t cols,

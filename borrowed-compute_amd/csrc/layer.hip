@@ -2,13 +2,17 @@
 // (crates/bc-infer/src/gpu/kernels.h:51-214, entry cuda.cu:77-79), RMSNorm (kernels.h:216-225,
 // cuda.cu:80) and the elementwise ops (kernels.h:327-330, cuda.cu:86-88).
 //
-// Product layout: weights stay in their ggml blocks, rows of whole blocks (row_bytes =
-// cols / block_weights * block_bytes); every format is read a "group" of 32 weights at a
-// time. A wave owns R weight rows and its 64 lanes take the row's groups, one each per
+// Five kernels share the product: k_matmul_row (one input row of the block formats), k_matmul_mm
+// (batches), k_matmul_units (small batches off a multiple of 256 columns) and k_matmul_tile (large
+// batches) on the matrix cores, the last three in one arithmetic; k_matmul (plain types, and one row
+// that k_matmul_row does not take) on the vector unit. Weights stay in their ggml blocks, rows of
+// whole blocks (row_bytes = cols / block_weights * block_bytes).
+//
+// k_matmul: every format is read a "group" of 32 weights at a time. A wave owns R weight rows and its 64 lanes take the row's groups, one each per
 // column tile: per group the lane loads its rows' packed bytes and its input values (up to
 // NB input rows), unpacks each row's 32 quants and sums in a fixed order. The 64 lane sums meet in a
-// fixed butterfly. So an input row's result depends on that row alone, never on how many
-// rows share the batch, and reruns give the same bits (the reference kernel's properties,
+// fixed butterfly. In each kernel an input row's result depends on that row alone, never on how
+// many rows share the batch, and reruns give the same bits (the reference kernel's properties,
 // kernels.h:9-11).
 #include "common.hpp"
 #include "internal.hpp"
@@ -1078,11 +1082,12 @@ __global__ __launch_bounds__(64 * MM_W<TY>, NI == 16 ? 2 : MM_W<TY> / 2) void k_
 // The vector-unit pass (k_matmul) held 1.75 waves a SIMD on this work, each waiting for a column
 // tile and then converting and multiplying it; here the products go to the matrix cores and the
 // waves are seven a SIMD, which leaves the unpacking (Q6K) and the loads (the others).
-// One row, us a call with the weights from HBM, k_matmul -> here: Q4K 14336 x 4096 14.1 -> 11.3,
-// 4096 x 14336 18.0 -> 11.0; Q6K 22.0 -> 18.0, 26.5 -> 16.4; Q8_0 21.6 -> 15.2, 24.3 -> 15.5;
-// Q4K 1024 x 4096 5.9 -> 3.9. 32 rows a workgroup (x staged once for both) were 6% faster at Q4K
-// 28672 x 8192 and 9-18% slower for Q8_0 and Q4_0. Error against 64 bits at 14336 columns:
-// Q4_0 2.4e-7 -> 0.8e-7, Q8_0 1.2 -> 0.9, Q4K 1.8 -> 1.7, Q5K 1.8 -> 1.6, Q6K 2.4 -> 1.0.
+// One row, us a call, k_matmul -> here, over 470 to 900 MB of matrices in turn (weights from HBM): Q4K
+// 14336 x 4096 15.3 -> 12.6, 4096 x 14336 19.8 -> 12.3, 1024 x 4096 7.0 -> 4.4; Q6K 22.9 -> 18.5, 27.1 ->
+// 17.0, 9.1 -> 5.5; Q8_0 21.6 -> 15.3, 24.3 -> 15.6, 8.1 -> 4.8; over six matrices, which the 256 MB
+// cache holds for Q4K, 14.1 -> 11.3, 18.0 -> 11.0, 5.9 -> 3.9. 32 rows a workgroup (x staged once for
+// both) were 6% faster at Q4K 28672 x 8192 and 9-18% slower for Q8_0 and Q4_0. Error against 64 bits
+// at 4096 columns: Q4_0 2.6e-7 -> 0.8e-7, Q8_0 1.1 -> 0.8, Q4K 1.7 -> 1.4, Q5K 1.7 -> 1.5, Q6K 2.3 -> 1.0.
 constexpr uint32_t ROW_UNITS = 256;  // units whose sums fit the workgroup's LDS
 
 template <uint32_t TY, int W, bool ONE>
@@ -1209,7 +1214,7 @@ __global__ __launch_bounds__(64 * W) void k_matmul_row(const MMParams p) {
 // so a batch of n unpacks every weight n / 8 times and is bound by that VALU work (512 rows
 // of 14336 x 4096 Q4K: 480 us). Here a workgroup of eight waves takes MT input rows x 128
 // weight rows and walks its K range in steps of 64 columns (two groups): the step's packed
-// weights are loaded by four threads a row (one step ahead), unpacked once into f16 in LDS
+// weights are loaded by four threads a row (two steps ahead), unpacked once into f16 in LDS
 // and read back as the B operands of every input tile; x comes from k_mm_prep as scaled hi
 // and lo parts in the operands' order (the conversion once a call instead of once a
 // workgroup). Each wave owns TM x TN 16 x 16 output tiles.

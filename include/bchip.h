@@ -130,9 +130,9 @@ int bchip_rope_append(bchip_ctx* ctx, float* q, const float* k, const float* v, 
  *    every slot the masks name (the caller's Shape guarantees it; in a bchip_alloc buffer a
  *    slot past its end reads as zeros, never out of bounds). rows <= 64, pos + 64 <= 2^32.
  * Requires hd % 8 == 0, hd <= 256, nh % nkv == 0, nh/nkv <= 16.
- * f32 caches (the reference's): f32 arithmetic throughout, the scores by quant::dot's
- * eight-lane sum (quant.rs:617-631), one arithmetic for every row of every call: a row's
- * bits depend only on its q and its visible slot list, whatever the batch, the row's index,
+ * f32 caches (the reference's): f32 arithmetic throughout, every product and sum in one fixed
+ * order on the f32 matrix cores (not quant::dot's order, quant.rs:617-631: within f32 rounding
+ * of it), one arithmetic for every row of every call: a row's bits depend only on its q and its visible slot list, whatever the batch, the row's index,
  * tree or line, one row or many (model.rs:531, 578, 592-594, 641-646).
  * f16 caches: q, K, V and the softmax weights are f16 MFMA operands, f32 accumulation.
  * Every row of a multi-row call (rows >= 2) is computed by the same fixed-order
@@ -153,7 +153,7 @@ int bchip_attention(bchip_ctx* ctx, const float* q, const void* kc, const void* 
  * five commands k_rope(q), k_rope(k), k_copy(k), k_copy(v), k_attention that
  * Layers::forward queues per layer for a one-token pass (gpu/mod.rs:464-482): the rotation
  * and the append run inside the attention kernel, which takes the new row from registers
- * (f16 caches) or LDS (f32 caches: attn_f32 rotates q as it stages it and the fold leaves q
+ * (f16 caches) or LDS (f32 caches: attn_f32_step rotates q as it stages it and the fold leaves q
  * rotated). f16 shapes the fused kernel does not take (hd % 32 != 0, neox pairs with
  * rope_dim/2 not a multiple of 32, or more than 8 query heads per KV head) run as the two
  * calls. positions: device u32 [1]. */
@@ -172,7 +172,7 @@ int bchip_rope_append_attention(bchip_ctx* ctx, float* q, const float* k, const 
  * f16 caches at head_dim 128, at most 16 rows with rows x (nh / nkv) <= 64, a line longer
  * than one 192-slot chunk whose split launch fits the device's CUs at once, neox pairs
  * only at rope_dim 64 or 128, and k and v 16-byte aligned; and for f32 caches of at most 8
- * rows at any shape (attn_f32, then its fold when split). Other calls run as the two calls.
+ * rows at any shape (attn_f32_step, then its fold when split). Other calls run as the two calls.
  * positions: device u32 [rows]. */
 int bchip_rope_append_attention_rows(bchip_ctx* ctx, float* q, const float* k, const float* v, void* kc, void* vc,
                                      uint32_t kv_type, const float* inv_freq, const uint32_t* positions,
@@ -251,10 +251,20 @@ int bchip_rope_append_attention_ragged(bchip_ctx* ctx, float* q, const float* k,
  * cols / block_weights * block_bytes: matmul_rows passes its first `rows` rows only);
  * x [n][cols] and out [n][rows] f32. cols must be a multiple of 32 (256 for the K-quants);
  * w and x 16-byte aligned; n at most 524280 (8 x 65535) a call. Batches of 2 or more rows
- * of the block formats and F16 with cols a multiple of 256 run on the matrix cores, as the
- * reference's do from MM_FROM = 2 rows (gpu/mod.rs:33-41). An input row's result does not
- * depend on n or on its place among the batch's rows; a batch row agrees with the same row
- * passed alone within f32 rounding (as the reference's). Reruns give the same bits. */
+ * of the block formats and F16 run on the matrix cores, as the reference's do from MM_FROM =
+ * 2 rows (gpu/mod.rs:33-41), and so does one row of the block formats with cols a multiple of
+ * 256 up to 65536. There x is held in two f16 parts under one power of two for each 256 columns
+ * of a row: 22 bits of every x within 2^-29 of the largest |x| of the 256 (Q6K: within 2^-17; the
+ * sums of x that Q4_1, Q5_1 and the K-quants' mins multiply: to 2^-40 of it, Q4K and Q5K 2^-52),
+ * less of smaller ones; products are exact, sums f32 or wider. Else x, weights and sums are f32.
+ * An infinite or NaN x gives its row of outputs what IEEE products and sums give over the plain
+ * types (F32, F16, BF16), and NaN over the block formats.
+ * An input row's result does not depend on n >= 2 or on its place among the batch's rows; a batch
+ * row agrees with the same row passed alone within f32 rounding (as the reference's). Reruns
+ * give the same bits, also where scratch cannot be had (memory full, a call under graph
+ * capture): the call then runs without. The context keeps the scratch of its largest call (prepared
+ * x, at most 256 MiB plus its sums and partial sums) until it is destroyed; a larger call replaces
+ * it, so a graph captured over calls that use it is replayed only before that. */
 int bchip_matmul(bchip_ctx* ctx, const void* w, uint32_t type, const float* x, float* out,
                  uint32_t rows, uint32_t cols, uint32_t n);
 
@@ -277,8 +287,8 @@ int bchip_add(bchip_ctx* ctx, float* x, const float* y, uint64_t n);
  * (device f32 [rows][vocab]) at step step0 + r. temperature <= 0: the first index of the
  * highest score. Otherwise p = exp((score - max) / temperature) (exp correctly rounded: the
  * reference takes its C library's expf, equal but for arguments within 0.002 ulp of a rounding
- * midpoint), the smallest prefix of the stable descending order whose mass reaches top_p, and
- * the seeded draw of sample.rs:61-67 with uniform(seed ^ step * 0x9e3779b97f4a7c15). Every sum
+ * midpoint), the smallest prefix of the stable descending order, of at least one token, whose mass
+ * reaches top_p, and the seeded draw of sample.rs:61-67 with uniform(seed ^ step * 0x9e3779b97f4a7c15). Every sum
  * runs in the reference's order, so the ids are the reference's. rows <= 65535. */
 int bchip_sample(bchip_ctx* ctx, const float* scores, uint32_t rows, uint32_t vocab, float temperature,
                  float top_p, uint64_t seed, uint64_t step0, uint32_t* ids);

@@ -14,7 +14,8 @@ non-finite input likewise reaches only the outputs that read it.)
 One difference from that kernel is checked as it stands: the multi-row kernels multiply a
 whole block of V by P (64 entries over f16 caches, 32 over f32), and an entry a row does not
 see has P = 0 there, so a V element that is NaN or infinite (0 x inf is NaN) also reaches,
-in its own dimension, the rows of its KV group that stream its block without seeing it;
+in its own dimension, the rows of its KV group that stream its block without seeing it (over
+f32 caches those of the tile of 16 query slots whose longest list holds it; the last test);
 the reference's loop, bounded by each row's length, does not touch such an entry. A K
 element does not: masked scores are replaced, not multiplied."""
 import math
@@ -79,7 +80,7 @@ def test_a_non_finite_input_reaches_only_its_own_outputs(ctx, rows, pos, nh, nkv
         else:
             vc = cache
         # A row sees s, or (V) streams the block that holds it: 64 entries (f16 caches, MFMA
-        # tiles), 32 (f32 caches, attn_f32's blocks).
+        # tiles), 32 (f32 caches, the blocks of both forms).
         blk = 64 if kv_type == bchip.F16 else 32
         first = s if what == "k_inf" else s - s % blk
         seen = pos + np.arange(rows) + 1 > first
