@@ -58,7 +58,7 @@ struct F32Params {
     uint32_t split;   // attn_f32_step: more than one chunk, the states go to attn_combine
     const float* zero;  // ZERO_BYTES of zeros: the loads of rows past a list
     // A line call fused with RoPE and the K/V append of its rows at slots pos .. pos + rows - 1
-    // (attn_f32_step<HD, NR>, NR > 0: at most NR rows): q is unrotated on entry and rotated as it
+    // (attn_f32_step's NR > 0: at most NR rows): q is unrotated on entry and rotated as it
     // is staged; the new K rows (knew, rotated here) and V rows (vnew) go to the caches and
     // stand in for those slots' cache entries. q is left rotated: by the workgroup itself when
     // unsplit, else by the fold.
@@ -147,7 +147,10 @@ __device__ __forceinline__ float vec_at(V v, int i) {
 // 255 us, so 237). Steps and verify rows run best two workgroups a CU with these registers;
 // trees and short prompts, whose rows read one prefix from cache, three (33 rows at 3001: 265
 // us, 236).
-template <int HD, int NR>
+// SHORT: lists of at most F32_SHORT entries skip the loads of blocks past them, which take their time
+// although they fetch nothing (one row at 0 slots, llama-8B heads, 6.8 -> 4.9 us, at 50 7.8 -> 5.7,
+// a tree of 4 rows at 0 8.6 -> 4.9); in longer lists the branches cost 2-10% (6000 slots 19.1 -> 20.4).
+template <int HD, int NR, bool SHORT>
 __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void attn_f32_step(const F32Params p) {
     constexpr bool FUSE = NR > 0;
     constexpr int NJ = HD / 16;                      // 16-byte reads of a K row a lane
@@ -204,9 +207,11 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
         if (p.tree && kk >= p.pos) s = tail[min(kk - p.pos, (uint32_t)MAX_ITEMS - 1u)] - kb0;
         return kk < kb1 ? s * kvd * 4u : NONE;
     };
+    const uint32_t nblk = kb0 < kb1 ? (kb1 - kb0 + F32_BLK - 1) / F32_BLK : 0u;
     f32x4 kx[TPW][NJ];
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
+        if (SHORT && (wave + F32_WAVES * t) / 2 >= nblk) break;
         const uint32_t ro = row_at(16u * (wave + F32_WAVES * t) + n) + 16u * g;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
@@ -315,7 +320,6 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
 #pragma unroll
     for (int j = 0; j < NJ; j++) qx[j] = *(const f32x4*)&qs[n][16 * j + 4 * g];
 
-    const uint32_t nblk = kb0 < kb1 ? (kb1 - kb0 + F32_BLK - 1) / F32_BLK : 0u;
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
         const uint32_t tile = wave + F32_WAVES * t, e = kb0 + 16 * tile + n;
@@ -335,7 +339,8 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
             ss[tile][lane] = score_tile(a, p.sc, kb0 + 16 * tile + 4 * g, len);
         }
 #pragma unroll
-        for (int v = 0; v < NT / TPW; v++) load_v(NT / TPW * t + v);
+        for (int v = 0; v < NT / TPW; v++)
+            if (!SHORT || (NT / TPW * t + v) / 2u < nblk) load_v(NT / TPW * t + v);
     }
     lds_barrier();
 
@@ -563,19 +568,31 @@ __global__ __launch_bounds__(F32_THREADS, HD <= 128 ? 2 : 1) void attn_f32_line(
 
 static uint32_t ceil_div32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
+constexpr uint64_t F32_SHORT = 128;  // entries (of the farthest list) up to which a call's lists are short
+
+template <int HD, bool SHORT>
+static void launch_step(const F32Params& fp, const dim3& grid, const AttnCall& a, hipStream_t s, bool fuse) {
+    const dim3 wg(F32_THREADS);
+    if (fuse && fp.rows == 1)
+        hipExtLaunchKernelGGL((attn_f32_step<HD, 1, SHORT>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+    else if (fuse)
+        hipExtLaunchKernelGGL((attn_f32_step<HD, (int)F32_FUSE_ROWS, SHORT>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+    else
+        hipExtLaunchKernelGGL((attn_f32_step<HD, 0, SHORT>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+}
+
 template <int HD>
-static hipError_t launch_f32(const F32Params& fp, uint32_t blocks, const AttnCall& a, hipStream_t s, bool fuse, bool line) {
+static hipError_t launch_f32(const F32Params& fp, uint32_t blocks, const AttnCall& a, hipStream_t s, bool fuse, bool line,
+                             bool is_short) {
     const dim3 grid(blocks), wg(F32_THREADS);
     if (line && fp.tree)
         hipExtLaunchKernelGGL((attn_f32_line<HD, true>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
     else if (line)
         hipExtLaunchKernelGGL((attn_f32_line<HD, false>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
-    else if (fuse && fp.rows == 1)
-        hipExtLaunchKernelGGL((attn_f32_step<HD, 1>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
-    else if (fuse)
-        hipExtLaunchKernelGGL((attn_f32_step<HD, (int)F32_FUSE_ROWS>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+    else if (is_short)
+        launch_step<HD, true>(fp, grid, a, s, fuse);
     else
-        hipExtLaunchKernelGGL((attn_f32_step<HD, 0>), grid, wg, 0, s, a.ev_before, a.ev_after, 0, fp);
+        launch_step<HD, false>(fp, grid, a, s, fuse);
     return hipGetLastError();
 }
 
@@ -669,10 +686,10 @@ hipError_t f32_attention(const AttnCall& a, uint64_t kvoff, Workspace& ws, hipSt
         rope = nullptr;
     }
     switch (hdp) {
-        case 32: e = launch_f32<32>(fp, (uint32_t)blocks, a, s, rope != nullptr, line); break;
-        case 64: e = launch_f32<64>(fp, (uint32_t)blocks, a, s, rope != nullptr, line); break;
-        case 128: e = launch_f32<128>(fp, (uint32_t)blocks, a, s, rope != nullptr, line); break;
-        default: e = launch_f32<256>(fp, (uint32_t)blocks, a, s, rope != nullptr, line); break;
+        case 32: e = launch_f32<32>(fp, (uint32_t)blocks, a, s, rope != nullptr, line, far <= F32_SHORT); break;
+        case 64: e = launch_f32<64>(fp, (uint32_t)blocks, a, s, rope != nullptr, line, far <= F32_SHORT); break;
+        case 128: e = launch_f32<128>(fp, (uint32_t)blocks, a, s, rope != nullptr, line, far <= F32_SHORT); break;
+        default: e = launch_f32<256>(fp, (uint32_t)blocks, a, s, rope != nullptr, line, far <= F32_SHORT); break;
     }
     if (e != hipSuccess || !fp.split) return e;
     CombineParams cp{};

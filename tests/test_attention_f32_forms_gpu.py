@@ -54,7 +54,9 @@ def _check64(out, q, kc, vc, rows, nh, nkv, hd, pos):
 # (nh, nkv, hd, rows, pos): tiles below and at 512, lists within a block, a chunk and past both,
 # the last workgroup's tiles cut, head dims below their padded size.
 LINES = [(8, 8, 128, 1024, 3), (32, 8, 128, 253, 189), (32, 8, 128, 256, 189), (14, 2, 64, 515, 31), (16, 16, 40, 520, 160),
-         (8, 8, 256, 1030, 65), (16, 1, 32, 513, 0), (28, 4, 80, 517, 383)]
+         (8, 8, 256, 1030, 65), (16, 1, 32, 513, 0), (28, 4, 80, 517, 383),
+         # lists of at most 128 entries and one more (own calls: at most)
+         (32, 8, 128, 120, 9), (14, 2, 64, 100, 28), (16, 8, 256, 110, 30), (8, 2, 32, 97, 31)]
 
 
 @pytest.mark.parametrize("nh,nkv,hd,rows,pos", LINES)
@@ -71,7 +73,7 @@ def test_a_row_has_the_bits_of_its_own_call(ctx, nh, nkv, hd, rows, pos):
 
 
 # The last: slots of more elements than the split form's offsets reach.
-TREES = [(8, 8, 128, 64, 300), (64, 8, 128, 63, 190), (16, 16, 64, 33, 500), (4100, 4100, 256, 5, 2)]
+TREES = [(32, 8, 128, 40, 0), (14, 2, 64, 33, 64), (14, 2, 64, 33, 65), (8, 8, 128, 64, 300), (64, 8, 128, 63, 190), (16, 16, 64, 33, 500), (4100, 4100, 256, 5, 2)]
 
 
 @pytest.mark.parametrize("nh,nkv,hd,rows,pos", TREES)
