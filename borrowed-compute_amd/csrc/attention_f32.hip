@@ -54,6 +54,9 @@ struct F32Params {
     uint64_t slot_limit;  // slots the caches hold (tree slots past it read as zeros)
     float sc;         // scale * log2(e)
     uint32_t rb, nrb; // rows a tile (1 for trees), tiles of a KV head
+    // A split tree's chunks wholly below pos, which hold the same slots for every row: chunks,
+    // rows a tile, tiles of a KV head (npc 0: none such).
+    uint32_t npc, prb, npt;
     uint32_t nchunk;  // chunks of the farthest list
     uint32_t split;   // attn_f32_step: more than one chunk, the states go to attn_combine
     const float* zero;  // ZERO_BYTES of zeros: the loads of rows past a list
@@ -171,25 +174,27 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
     const uint32_t n = lane & 15u, g = lane >> 4;    // n: an entry, a slot or a dim's place
     // The tiles of a chunk of a KV head side by side in launch order, so that they find its K and V
     // in cache.
-    const uint32_t kvh = blockIdx.x % p.nkv, b0 = blockIdx.x / p.nkv;
-    const uint32_t rbi = b0 % p.nrb, c = b0 / p.nrb;
-    const uint32_t grp = kvh * p.nrb + rbi;          // canonical group of the chunk states
-    const uint32_t r0 = rbi * p.rb, hd = p.hd, kvd = p.nkv * hd;
+    const uint32_t kvh = blockIdx.x % p.nkv, b0 = blockIdx.x / p.nkv, np = p.npc * p.npt;
+    const bool prefix = !FUSE && b0 < np;  // a tree's rows together
+    const uint32_t rb = prefix ? p.prb : p.rb;
+    const uint32_t rbi = prefix ? b0 % p.npt : (b0 - np) % p.nrb, c = prefix ? b0 / p.npt : p.npc + (b0 - np) / p.nrb;
+    const uint32_t r0 = rbi * rb, hd = p.hd, kvd = p.nkv * hd;
+    const bool tree = p.tree && !prefix;
 
-    // A tree's tile is one row: its list is the slots below pos, then pos + j for each set bit j
+    // Else a tree's tile is one row: its list is the slots below pos, then pos + j for each set bit j
     // of its mask, in order (kernels.h:266-278).
     uint32_t ntail = 0;
-    if (p.tree) {
+    if (tree) {
         const uint32_t lo = p.masks[2 * r0], hi = p.masks[2 * r0 + 1];
         ntail = __popc(lo) + __popc(hi);
         if (tid < ntail) tail[tid] = p.pos + nth_set_bit(lo, hi, tid);
         __syncthreads();
     }
     // Slot n: head kvh * G + n / rb of row r0 + n % rb.
-    auto slot_valid = [&](uint32_t k) { return k / p.rb < p.G && r0 + k % p.rb < p.rows; };
-    const uint32_t rlast = min(r0 + p.rb, p.rows) - 1u;
+    auto slot_valid = [&](uint32_t k) { return k / rb < p.G && r0 + k % rb < p.rows; };
+    const uint32_t rlast = min(r0 + rb, p.rows) - 1u;
     const uint32_t maxlen = p.tree ? p.pos + ntail : p.pos + rlast + 1u;
-    const uint32_t len = !slot_valid(n) ? 0u : p.tree ? maxlen : p.pos + r0 + n % p.rb + 1u;
+    const uint32_t len = !slot_valid(n) ? 0u : p.tree ? maxlen : p.pos + r0 + n % rb + 1u;
     const uint32_t kb0 = c * CHUNK_MULTI, kb1 = min(kb0 + CHUNK_MULTI, maxlen);
 
     // K and V through buffer descriptors from the chunk's first slot on: entries past the list and
@@ -204,7 +209,7 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
     auto row_at = [&](uint32_t e) -> uint32_t {  // bytes from the chunk's first slot to entry e
         const uint32_t kk = kb0 + e;
         uint32_t s = e;
-        if (p.tree && kk >= p.pos) s = tail[min(kk - p.pos, (uint32_t)MAX_ITEMS - 1u)] - kb0;
+        if (tree && kk >= p.pos) s = tail[min(kk - p.pos, (uint32_t)MAX_ITEMS - 1u)] - kb0;
         return kk < kb1 ? s * kvd * 4u : NONE;
     };
     const uint32_t nblk = kb0 < kb1 ? (kb1 - kb0 + F32_BLK - 1) / F32_BLK : 0u;
@@ -275,7 +280,7 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
             const bool rot = rope_pair(pp, p.rope_dim, p.neox, a, b);
             float y0 = 0.0f, y1 = 0.0f;
             if (pp < hd / 2 && slot_valid(k)) {
-                const uint32_t r = r0 + k % p.rb, h = kvh * p.G + k / p.rb;
+                const uint32_t r = r0 + k % rb, h = kvh * p.G + k / rb;
                 const float* qh = p.q + ((size_t)r * p.nh + h) * hd;
                 y0 = qh[a];
                 y1 = qh[b];
@@ -289,7 +294,7 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
             const uint32_t k = e / (HD / 4), d = 4 * (e % (HD / 4));
             f32x4 v = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             if (d < hd && slot_valid(k)) {
-                const uint32_t r = r0 + k % p.rb, h = kvh * p.G + k / p.rb;
+                const uint32_t r = r0 + k % rb, h = kvh * p.G + k / rb;
                 v = *(const f32x4*)&p.q[((size_t)r * p.nh + h) * hd + d];
             }
             *(f32x4*)&qs[k][d] = v;
@@ -310,7 +315,7 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
             for (uint32_t e = tid; e < F32_SLOTS * HD; e += F32_THREADS) {
                 const uint32_t k = e / HD, d = e % HD;
                 if (d < hd && slot_valid(k)) {
-                    const uint32_t r = r0 + k % p.rb, h = kvh * p.G + k / p.rb;
+                    const uint32_t r = r0 + k % rb, h = kvh * p.G + k / rb;
                     p.qw[((size_t)r * p.nh + h) * hd + d] = qs[k][d];
                 }
             }
@@ -376,10 +381,12 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
     // Lane (n, g): dims vb .. vb + 4 VC - 1 of slot n, dim vb + VC i + k in o[k][i].
     const uint32_t vb = VW * wave + 4 * VC * g;
     if (p.split) {
-        const size_t u = (size_t)grp * p.nchunk + c;
-        if (n >= min((uint32_t)F32_SLOTS, p.G * p.rb)) return;  // attn_combine reads no slot past them
+        // A tree's states are its rows' (head n / rb of row r0 + n % rb), a line's its tiles'.
+        const size_t u = ((size_t)kvh * p.nrb + (p.tree ? r0 + n % rb : rbi)) * p.nchunk + c;
+        const uint32_t at = p.tree ? n / rb : n;
+        if (n >= min((uint32_t)F32_SLOTS, p.G * rb) || (prefix && !slot_valid(n))) return;  // attn_combine reads no slot past them
         if (vb < (uint32_t)HD) {
-            float* dst = p.part_o + (u * F32_SLOTS + n) * HD + vb;
+            float* dst = p.part_o + (u * F32_SLOTS + at) * HD + vb;
 #pragma unroll
             for (int q4 = 0; q4 < VC; q4++) {
                 f32x4 v;
@@ -388,11 +395,11 @@ __global__ __launch_bounds__(F32_THREADS, HD > 128 ? 1 : NR == 0 ? 3 : 2) void a
                 *(f32x4*)(dst + 4 * q4) = v;
             }
         }
-        if (wave == 0 && g == 0) *(float2*)(p.part_ml + (u * F32_SLOTS + n) * 2) = float2{m, l};
+        if (wave == 0 && g == 0) *(float2*)(p.part_ml + (u * F32_SLOTS + at) * 2) = float2{m, l};
         return;
     }
     if (!slot_valid(n)) return;
-    float* dst = p.out + ((size_t)(r0 + n % p.rb) * p.nh + kvh * p.G + n / p.rb) * hd + vb;
+    float* dst = p.out + ((size_t)(r0 + n % rb) * p.nh + kvh * p.G + n / rb) * hd + vb;
 #pragma unroll
     for (int q4 = 0; q4 < VC; q4++)
         if (vb + 4 * q4 < hd) {
@@ -676,7 +683,14 @@ hipError_t f32_attention(const AttnCall& a, uint64_t kvoff, Workspace& ws, hipSt
             return e;
         }
     }
-    const uint64_t blocks = line ? (uint64_t)a.nkv * ceil_div32(fp.nrb, a.tree ? 1 : F32_WAVES) : groups * fp.nchunk;
+    if (fp.split && a.tree && fp.G <= F32_SLOTS / 2) {
+        // Rows share the tiles of the chunks below pos: else each row's tile of G slots fetches and
+        // multiplies its own (33 rows at 500 slots, one head a KV head: 61 us, 45 on the vector unit).
+        fp.npc = a.pos / CHUNK_MULTI;
+        fp.prb = std::min<uint32_t>((uint32_t)F32_SLOTS / fp.G, a.rows);
+        fp.npt = ceil_div32(a.rows, fp.prb);
+    }
+    const uint64_t blocks = line ? (uint64_t)a.nkv * ceil_div32(fp.nrb, a.tree ? 1 : F32_WAVES) : groups * (fp.nchunk - fp.npc) + (uint64_t)a.nkv * fp.npc * fp.npt;
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
     hipError_t e;
     if (line && rope) {  // the line form is not fused

@@ -72,8 +72,11 @@ def test_a_row_has_the_bits_of_its_own_call(ctx, nh, nkv, hd, rows, pos):
     _check64(out, q, kc, vc, rows, nh, nkv, hd, pos)
 
 
-# The last: slots of more elements than the split form's offsets reach.
-TREES = [(32, 8, 128, 40, 0), (14, 2, 64, 33, 64), (14, 2, 64, 33, 65), (8, 8, 128, 64, 300), (64, 8, 128, 63, 190), (16, 16, 64, 33, 500), (4100, 4100, 256, 5, 2)]
+# Chunks below pos, whose tiles hold several rows: none, one, several, pos at a chunk's end, one to
+# sixteen heads a KV head, rows that don't fill a tile. The last: slots of more elements than the
+# split form's offsets reach.
+TREES = [(32, 8, 128, 40, 0), (14, 2, 64, 33, 64), (14, 2, 64, 33, 65), (8, 8, 128, 64, 300), (64, 8, 128, 63, 190), (16, 16, 64, 33, 500), (32, 8, 128, 33, 777), (28, 4, 64, 17, 1153),
+         (16, 1, 32, 30, 400), (8, 2, 128, 3, 576), (40, 8, 256, 21, 575), (4100, 4100, 256, 5, 2)]
 
 
 @pytest.mark.parametrize("nh,nkv,hd,rows,pos", TREES)
